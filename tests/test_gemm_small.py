@@ -1,0 +1,105 @@
+"""GEMMs of few outputs (below 256 tiles of 128 x 128): the K-split tiles and
+the small DMA tiles, at the edges of tiles, of the K chunks and of the tile
+rule, against the oracle (atol 2e-2 / rtol 1e-2, the tolerance of every
+16-bit output here)."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+import torch
+
+import oracle
+from tests.conftest import close
+from tests.test_asm_waits import CSRC, ROOT, scan
+
+ACTS = {"none": 0, "gelu": 1, "silu": 2, "relu": 3}
+
+
+def _mk(m, n, k, dtype, seed=0, wstd=0.05):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(m, k, generator=g).to(dtype)
+    w = (wstd * torch.randn(n, k, generator=g)).to(dtype)
+    return x, w, (wstd * torch.randn(n, generator=g)).to(dtype)
+
+
+# (m, n, k): one output and one chunk; a wave without a chunk (k < 256); every
+# remainder of the last chunk's 8-wide units; the 32x32, 64x32, 64x64 (4 and 2
+# waves), 128x64 and 128x128 tiles with ragged edges, N no multiple of 8
+SHAPES = [(17, 1, 8), (17, 33, 64), (31, 64, 72), (32, 96, 200), (33, 100, 248), (77, 1024, 3072),
+          (65, 1003, 1000), (230, 1024, 2048), (300, 2048, 1000), (510, 1024, 1024),
+          (230, 4096, 1024), (600, 1028, 520), (2000, 1024, 1024), (1990, 1030, 320),
+          (1000, 3072, 1024), (1000, 4100, 64), (1024, 4095, 128), (513, 4000, 192)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act,bias", [("none", False), ("gelu", True), ("silu", False)])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_linear_few_outputs(dev, m, n, k, act, bias):
+    from torchplusplus_amd._native import ext
+    dtype = torch.float16 if m % 2 else torch.bfloat16
+    x, w, b = _mk(m, n, k, dtype, seed=m + k)
+    b = b if bias else None
+    y = ext().linear(x.to(dev), w.to(dev), None if b is None else b.to(dev), ACTS[act])
+    close(y, oracle.linear_act(x, w, b, act), what=f"linear {act} {m}x{n}x{k}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,i,k", [(17, 32, 64), (40, 96, 1000), (230, 3072, 1024), (512, 3072, 1024),
+                                   (129, 2048, 768), (1000, 1024, 136)])
+def test_swiglu_few_outputs(dev, m, i, k):
+    from torchplusplus_amd._native import ext
+    from torchplusplus_amd.dlops.linear import interleave_gate_up
+    x, wg, _ = _mk(m, i, k, torch.bfloat16, seed=3)
+    _, wu, _ = _mk(m, i, k, torch.bfloat16, seed=4)
+    y = ext().linear_swiglu(x.to(dev), interleave_gate_up(wg, wu).to(dev))
+    g = oracle.linear_act(x, wg, None, "silu").float()
+    u = oracle.linear_act(x, wu, None, "none").float()
+    close(y, (g * u).to(x.dtype), what=f"swiglu {m}x{i}x{k}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(40, 96, 1000), (230, 1024, 264), (2000, 1024, 192)])
+def test_linear_reads_nothing_past_a_row(dev, m, n, k):
+    """Rows with a pitch: NaNs between them must not reach an output, and the
+    output's own gap stays untouched."""
+    from torchplusplus_amd._native import lib
+    x, w, _ = _mk(m, n, k, torch.bfloat16, seed=5)
+    xp = torch.full((m, k + 8), float("nan"), dtype=x.dtype, device=dev)
+    xp[:, :k] = x.to(dev)
+    out = torch.zeros(m, n + 8, dtype=x.dtype, device=dev)
+    wd, i64, ptr = w.to(dev), ctypes.c_int64, ctypes.c_void_p
+    rc = lib().tpp_linear_act(ptr(xp.data_ptr()), ptr(wd.data_ptr()), None, ptr(out.data_ptr()),
+                              i64(m), i64(n), i64(k), i64(k + 8), i64(n + 8), ctypes.c_int(0),
+                              ctypes.c_int(1), ptr(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    close(out[:, :n], oracle.linear_act(x, w, None, "none"), what="pitched rows")
+    assert torch.count_nonzero(out[:, n:]) == 0
+
+
+@pytest.mark.gpu
+def test_linear_few_outputs_keeps_infinities(dev):
+    """An infinity in the last K unit of a K that is no multiple of 64 reaches
+    its row and no other (the units past K are zeros, not copies of it)."""
+    from torchplusplus_amd._native import ext
+    x, w, _ = _mk(40, 64, 1000, torch.bfloat16, seed=6)
+    x[7, 999] = float("inf")
+    y = ext().linear(x.to(dev), w.to(dev), None, 0).cpu()
+    want = oracle.linear_act(x, w, None, "none")
+    assert torch.equal(torch.isinf(y), torch.isinf(want)) and not torch.isnan(y).any()
+    rows = [i for i in range(40) if i != 7]
+    close(y[rows], want[rows], what="rows without the infinity")
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not installed")
+def test_gemm_fragment_reads_waited_for(tmp_path):
+    """The K-split kernel's asm fragment reads: no compiler-made instruction
+    touches their registers before the wait."""
+    out = str(tmp_path / "gemm.s")
+    subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature",
+                    "-Xclang", "-packed-fp32-ops", "-ffp-contract=fast", f"-I{os.path.join(ROOT, 'include')}",
+                    "--cuda-device-only", "-S", os.path.join(CSRC, "gemm.hip"), "-o", out],
+                   check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL, timeout=600)
+    loads, bad = scan(open(out).read())
+    assert loads > 0 and not bad, "\n".join(bad[:10])

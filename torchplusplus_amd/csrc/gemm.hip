@@ -49,8 +49,8 @@ constexpr int kBigBK = TPP_BIG_BK, kBigNST = TPP_BIG_NST;
 // (one block per CU): 5 for 128x128, 4 for 128x192, 3 for 128x256 (at the
 // Linear+act shape 3 stages were 6% faster than 2, and 4 another 3%)
 constexpr int kSmallBK = 64;
-// below this many outputs the register-staged kernel's smaller LDS footprint
-// (several blocks per CU) wins over the deeper DMA ring
+// below this many outputs 128-row tiles leave CUs idle: smaller tiles, chosen
+// by pick_small_tile
 constexpr int64_t kDmaMinMN = 256 * 128 * 128;
 // the DMA kernel addresses a tile's rows by 32-bit byte offsets from its
 // first row: 256 rows * ld * 2 bytes stays below 2^32 up to this pitch
@@ -768,6 +768,196 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small outputs (short prompts, batches of decode tokens): 32FM x 32FN tiles,
+// the K dimension split over the block's NW waves. Wave w takes the 64-deep K
+// chunks w, w + NW, ... through its own two-slot LDS ring (LDS-DMA, no barrier
+// in the K loop), then the waves' partial tiles are summed in LDS in wave
+// order (deterministic) and the epilogue runs on the sums.
+// What bounds it: with few outputs a 128-row tile leaves most CUs idle and
+// its K steps form a serial chain of memory round trips ([230 x 3072] .
+// [1024 x 3072]^T: 16 blocks, 48 steps of ~0.9 us). Small tiles fill the chip
+// but read more operand bytes per CU (~60 B/clk through L1), and the NW waves'
+// independent rings keep 64-128 KB of them in flight per CU, so the launch
+// costs its bytes over that rate plus ~3 us of launch, first round trip and
+// sum. Measured (bf16, weights cold, us; the register-staged 128x128 kernel
+// first): 230x1024x3072 45.0 -> 6.8, 230x4096x1024 19.1 -> 6.8, 77x1024x3072
+// + bias + GeLU 52.1 -> 7.4, 600x1024x1024 18.7 -> 6.6, 230x6144x1024 SwiGLU
+// 18.7 -> 9.2. Splitting K over blocks instead would need a cross-block sum
+// (~2 us); rings of 3 and 4 slots, 8 waves per 32x32 tile and 4 waves of two
+// K halves per 64x64 tile were no faster.
+template <typename T, int EPI, int ACT, int FM, int FN, int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_ksplit_kernel(
+    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
+    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
+  typedef typename VecT<T>::v8 V8;
+  constexpr int NST = 2; // ring slots per wave
+  constexpr int BM = 32 * FM, BN = 32 * FN, ROWS = BM + BN;
+  constexpr int NQ = ROWS / 8;        // DMA instructions per chunk (8 rows of 128 bytes each)
+  constexpr int STG = ROWS * 8;       // 16-byte units per ring slot
+  constexpr int LDR = BN + 4;         // fp32 pitch of a partial tile (odd in 16-byte units)
+  constexpr int WREG = NST * STG > BM * LDR / 4 ? NST * STG : BM * LDR / 4; // LDS units per wave
+  static_assert(NQ * (NST - 1) < 64, "vmcnt range");
+  static_assert(EPI != kGSwiGLU || FN % 2 == 0, "whole [gate | up] pairs per tile");
+  __shared__ V8 smem[NW * WREG];
+
+  const int ntm = (M + BM - 1) / BM, ntn = (N + BN - 1) / BN;
+  int tm, tn;
+  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // DMA instruction q: slot rows 8q .. 8q + 7 (A rows, then B rows), lane l
+  // row 8q + l / 8, fetching the chunk that its slot position holds under the
+  // XOR swizzle. Rows past M / N read the last row (outputs never stored).
+  const char *src[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int r = 8 * q + (lane >> 3);
+    src[q] = 8 * q < BM
+                 ? reinterpret_cast<const char *>(A + (int64_t)min(m0 + r, M - 1) * lda)
+                 : reinterpret_cast<const char *>(B + (int64_t)min(n0 + r - BM, N - 1) * ldb);
+  }
+  // k of the lane's unit in chunk 0, for even and odd q
+  const int k_even = ((lane & 7) ^ (lane >> 4)) * 8, k_odd = ((lane & 7) ^ (4 + (lane >> 4))) * 8;
+  V8 *const ring = smem + w * WREG;
+  // units past K (the last chunk of a K that is no multiple of 64) read the
+  // row's last one; the fragments zero them
+  auto issue = [&](int c, int slot) {
+    const int ke = min(c * 64 + k_even, K - 8) * (int)sizeof(T);
+    const int ko = min(c * 64 + k_odd, K - 8) * (int)sizeof(T);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      __builtin_amdgcn_global_load_lds(
+          (const void *)(src[q] + (uint32_t)((q & 1) ? ko : ke)),
+          (__attribute__((address_space(3))) void *)(ring + slot * STG + q * 64), 16, 0, 0);
+  };
+
+  const int nch = (K + 63) / 64;
+  const int n = w < nch ? (nch - w + NW - 1) / NW : 0; // this wave's chunks
+#pragma unroll
+  for (int i = 0; i < NST; ++i)
+    if (i < n) issue(w + i * NW, i);
+
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  const int l32 = lane & 31, half = lane >> 5, sw = swz(l32);
+  const unsigned lbase = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char *)ring + l32 * 128;
+  int slot = 0;
+  for (int i = 0; i < n; ++i) {
+    wait_tiles<NQ, NST - 1>(n - 1 - i); // chunk i landed
+    const unsigned sb = lbase + slot * (STG * 16);
+    V8 f[4][FM + FN];
+    static_for<4>([&](auto kk) {
+      constexpr int ks = decltype(kk)::value;
+      const unsigned a = sb + (((ks * 2 + half) ^ sw) << 4);
+      static_for<FM + FN>([&](auto ii) {
+        constexpr int r = decltype(ii)::value;
+        f[ks][r] = lds_read_b128<r * 32 * 128, V8>(a);
+      });
+    });
+    const int c = w + i * NW;
+    const bool tail = c * 64 + 64 > K;
+    static_for<4>([&](auto kk) {
+      constexpr int ks = decltype(kk)::value;
+      lds_wait_tied<(3 - ks) * (FM + FN)>(f[ks]);
+      if constexpr (ks == 3) {
+        // every fragment is in registers: refill the slot
+        if (i + NST < n) issue(c + NST * NW, slot);
+      }
+      if (tail) {
+        const bool past = c * 64 + (ks * 2 + half) * 8 >= K;
+#pragma unroll
+        for (int r = 0; r < FM + FN; ++r)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[ks][r][e] = past ? (T)0.0f : f[ks][r][e];
+      }
+#pragma unroll
+      for (int ii = 0; ii < FM; ++ii)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[ii][j] = mfma32<T>(f[ks][FM + j], f[ks][ii], acc[ii][j]);
+    });
+    slot = slot + 1 == NST ? 0 : slot + 1;
+  }
+
+  // Partial tiles in LDS (each wave over its own ring, drained above), W rows
+  // first in the MFMA: a lane holds output row lane & 31 and four consecutive
+  // columns per register group.
+  float *const part = reinterpret_cast<float *>(ring);
+#pragma unroll
+  for (int ii = 0; ii < FM; ++ii)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[ii][j][4 * q + e];
+        *reinterpret_cast<f32x4 *>(part + (ii * 32 + l32) * LDR + j * 32 + q * 8 + half * 4) = v;
+      }
+  __syncthreads();
+
+  constexpr int OW = (EPI == kGSwiGLU) ? BN / 2 : BN, CPR = OW / 8; // output columns, 8-column groups
+  const int NO = (EPI == kGSwiGLU) ? N / 2 : N, oc0 = (EPI == kGSwiGLU) ? n0 / 2 : n0;
+  const bool vec_ok = (ldc % 8 == 0) && ((reinterpret_cast<uintptr_t>(C) & 15) == 0);
+  auto total = [&](int row, int col, float (&v)[8]) {
+    const float *p = reinterpret_cast<const float *>(smem) + row * LDR + col;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) {
+      const f32x4 a = *reinterpret_cast<const f32x4 *>(p + ww * WREG * 4);
+      const f32x4 b = *reinterpret_cast<const f32x4 *>(p + ww * WREG * 4 + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += a[e], v[e + 4] += b[e];
+    }
+  };
+  for (int idx = tid; idx < BM * CPR; idx += 64 * NW) {
+    const int rl = idx / CPR, cl = (idx % CPR) * 8;
+    const int row = m0 + rl, col = oc0 + cl;
+    if (row >= M || col >= NO) continue;
+    float v[8];
+    if constexpr (EPI == kGSwiGLU) {
+      // gate columns 64p .. + 31, up columns the next 32, of pair p
+      const int wc = (cl / 32) * 64 + cl % 32;
+      float u[8];
+      total(rl, wc, v);
+      total(rl, wc + 32, u);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float s = to_f32(from_f32<T>(act_silu(to_f32(from_f32<T>(v[e])))));
+        v[e] = s * to_f32(from_f32<T>(u[e]));
+      }
+    } else {
+      total(rl, cl, v);
+      if constexpr (EPI == kGBiasAct) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (bias) v[e] += to_f32(bias[col + e < N ? col + e : N - 1]);
+          v[e] = apply_act<ACT>(to_f32(from_f32<T>(v[e])));
+        }
+      }
+    }
+    V8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = from_f32<T>(v[e]);
+    T *dst = C + (int64_t)row * ldc + col;
+    if (vec_ok && col + 8 <= NO) {
+      *reinterpret_cast<V8 *>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (col + e < NO) dst[e] = o[e];
+    }
+  }
+}
+
 // Tile shape for the DMA kernel: minimise (tiles per CU, rounded up) x tile
 // area / relative efficiency (one block per CU for every candidate). SwiGLU
 // needs whole [gate|up] 64-column pairs per wave (FN even).
@@ -792,6 +982,34 @@ static int pick_dma_tile(int64_t M, int64_t N, bool swiglu, int cus) {
   return best;
 }
 
+// Tile of an output below kDmaMinMN elements: the cheapest candidate by its
+// measured time per round of resident tiles (1 or 2 per CU), in us per 1024 of
+// K beyond the ~3 us every launch costs; one tile per CU at most is cheaper
+// than a full round for the two-per-CU shapes. Measured at M 32 - 2048, N
+// 1024 - 6144, K 1024 - 3072 (bf16): it picks the fastest or within 10% of it,
+// e.g. 512x1024x3072: 32x32 11.0, 64x32 8.8, 64x64 11.0, 128x64 18.7 us;
+// 2000x1024x1024: 16.1, 15.3, 9.7, 9.2, 128x128 11.2 us; 1000x3072x1024 +
+// bias: 28.5, 27.4, 21.1, 15.6, 13.5 us.
+enum SmallTile { kKs32x32, kKs64x32, kKs64x64w4, kKs64x64w2, kDma128x64, kDma128x128 };
+static SmallTile pick_small_tile(int64_t M, int64_t N, bool swiglu, bool dma_ok, int cus) {
+  struct Cand { SmallTile id; int bm, bn, per_cu; double one, full; };
+  const Cand cands[] = {{kKs32x32, 32, 32, 2, 1.25, 2.6},   {kKs64x32, 64, 32, 1, 1.95, 2.6},
+                        {kKs64x64w4, 64, 64, 1, 3.6, 4.2},  {kKs64x64w2, 64, 64, 2, 4.5, 6.2},
+                        {kDma128x64, 128, 64, 2, 6.2, 10.3}, {kDma128x128, 128, 128, 1, 9.4, 9.4}};
+  SmallTile best = kKs64x64w4;
+  double best_t = -1.0;
+  for (const Cand &c : cands) {
+    // SwiGLU needs whole [gate | up] 64-column pairs per wave
+    if (swiglu && (c.bn < 64 || c.id == kDma128x64)) continue;
+    if (!dma_ok && (c.id == kDma128x64 || c.id == kDma128x128)) continue;
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const int64_t round = (int64_t)cus * c.per_cu;
+    const double t = tiles <= cus ? c.one : (double)((tiles + round - 1) / round) * c.full;
+    if (best_t < 0 || t < best_t) best = c.id, best_t = t;
+  }
+  return best;
+}
+
 static int device_cus() {
   const int n = device_cu_count();
   return n > 0 ? n : 256;
@@ -804,6 +1022,16 @@ static void launch_dma(const void *A, int64_t lda, const void *B, int64_t ldb, v
   constexpr int BM = 32 * WM * FM, BN = 32 * WN * FN;
   const int64_t nb = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   gemm_dma_kernel<T, EPI, ACT, FM, FN, NST, WM, WN, BK><<<dim3((unsigned)nb), dim3(64 * WM * WN), 0, st>>>(
+      (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N, (int)K);
+}
+
+template <typename T, int EPI, int ACT, int FM, int FN, int NW>
+static void launch_ksplit(const void *A, int64_t lda, const void *B, int64_t ldb, void *C,
+                          int64_t ldc, const void *bias, int64_t M, int64_t N, int64_t K,
+                          hipStream_t st) {
+  constexpr int BM = 32 * FM, BN = 32 * FN;
+  const int64_t nb = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  gemm_ksplit_kernel<T, EPI, ACT, FM, FN, NW><<<dim3((unsigned)nb), dim3(64 * NW), 0, st>>>(
       (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N, (int)K);
 }
 
@@ -875,6 +1103,22 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
       if (!done) launch_dma<T, EPI, ACT, 2, 4, 4, 2, kBigBK, kBigNST>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
       break;
     }
+    }
+  } else if (vec && M * N < (int64_t)kDmaMinMN) {
+    const bool dma_ok = K % 64 == 0 && lda <= kDmaMaxLd && ldb <= kDmaMaxLd;
+    switch (pick_small_tile(M, N, EPI == kGSwiGLU, dma_ok, device_cus())) {
+    case kKs32x32:
+      if constexpr (EPI != kGSwiGLU) launch_ksplit<T, EPI, ACT, 1, 1, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
+      break;
+    case kKs64x32:
+      if constexpr (EPI != kGSwiGLU) launch_ksplit<T, EPI, ACT, 2, 1, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
+      break;
+    case kKs64x64w4: launch_ksplit<T, EPI, ACT, 2, 2, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
+    case kKs64x64w2: launch_ksplit<T, EPI, ACT, 2, 2, 2>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
+    case kDma128x64:
+      if constexpr (EPI != kGSwiGLU) launch_dma<T, EPI, ACT, 1, 1, 4, 2, kSmallBK, 3>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
+      break;
+    case kDma128x128: launch_dma<T, EPI, ACT, 1, 2, 4, 2, kSmallBK, 5>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
     }
   } else if (vec) {
     const int64_t nb = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
