@@ -279,6 +279,20 @@ int tpp_attn_prefill(const void *q, const void *k, const void *v, void *o,
                      int window_left, int window_right, int dtype,
                      void *stream);
 
+/* tpp_attn_prefill with a workspace (16-byte aligned, no initialisation
+ * required, at least tpp_attn_prefill_workspace_size bytes; NULL = none): with
+ * few query rows against many keys the keys of a row are then split over
+ * workgroups too, and the fp32 partials combined by a second launch. The size
+ * is 0 for shapes that need none. */
+size_t tpp_attn_prefill_workspace_size(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv,
+                                       int64_t D, int causal, int window_left, int window_right);
+int tpp_attn_prefill_ws(const void *q, const void *k, const void *v, void *o,
+                        const int64_t *q_strides, const int64_t *k_strides,
+                        const int64_t *v_strides, const int64_t *o_strides, int64_t B, int64_t Sq,
+                        int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D, float softmax_scale,
+                        int causal, int window_left, int window_right, int dtype,
+                        void *workspace, size_t ws_bytes, void *stream);
+
 /* Bytes of workspace tpp_attn_decode needs. The workspace must be 128-byte
  * aligned and its first 64 KiB zero-filled before the first use: they hold
  * per-(batch, KV head) arrival counters that every call leaves at zero

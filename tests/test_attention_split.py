@@ -1,0 +1,86 @@
+"""Prefill attention with few work items: the key-split kernel, one chunk and
+several (partials merged by a second launch), against the CPU oracle (atol
+2e-2 / rtol 1e-2, the tolerance of every 16-bit output here)."""
+import pytest
+import torch
+
+import oracle
+from tests.conftest import close
+
+pytestmark = pytest.mark.gpu
+
+
+def _qkv(b, sq, sk, hq, hkv, d, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(b, s, h, d, generator=g).to(dtype) for s, h in ((sq, hq), (sk, hkv), (sk, hkv))]
+
+
+def _workspace(b, sq, sk, hq, hkv, d, causal, window):
+    import ctypes
+    from torchplusplus_amd._native import lib
+    f = lib().tpp_attn_prefill_workspace_size
+    f.restype = ctypes.c_size_t
+    i64 = ctypes.c_int64
+    return f(i64(b), i64(sq), i64(sk), i64(hq), i64(hkv), i64(d), int(causal), window[0], window[1])
+
+
+# one key; tile and query-tile edges (32 / 64 keys, 32 / 64 queries, one past);
+# groups of 1, 2, 3, 4 and 8 heads per KV head; Sq > Sk (rows without a key);
+# windows that begin inside a tile; pair counts that split over the XCDs or not
+ONE_CHUNK = [(1, 1, 1, 2, 1, 128, True, (-1, -1)), (1, 17, 33, 4, 2, 128, True, (-1, -1)),
+             (2, 32, 32, 8, 8, 128, True, (-1, -1)), (1, 33, 64, 16, 8, 128, False, (-1, -1)),
+             (1, 65, 129, 3, 3, 64, True, (-1, -1)), (1, 64, 65, 6, 2, 64, False, (-1, -1)),
+             (1, 100, 40, 8, 2, 128, True, (-1, -1)), (1, 230, 230, 16, 8, 128, True, (-1, -1)),
+             (2, 200, 300, 16, 2, 64, True, (70, 0)), (1, 300, 300, 8, 4, 128, True, (33, 0)),
+             (1, 90, 200, 4, 4, 128, False, (20, 50)), (1, 600, 700, 16, 8, 128, True, (-1, -1))]
+CHUNKS = [(1, 1, 3000, 8, 8, 64, False, (-1, -1)), (1, 33, 4001, 16, 8, 128, True, (-1, -1)),
+          (1, 200, 3001, 16, 8, 128, True, (-1, -1)), (2, 40, 2500, 4, 1, 64, True, (-1, -1)),
+          (1, 70, 2050, 3, 1, 128, True, (2000, 0)), (1, 17, 5000, 12, 4, 64, False, (-1, -1))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,sq,sk,hq,hkv,d,causal,window", ONE_CHUNK + CHUNKS)
+def test_split_prefill(dev, dtype, b, sq, sk, hq, hkv, d, causal, window):
+    from torchplusplus_amd.attention import flash_attn_func
+    shape = (b, sq, sk, hq, hkv, d, causal, window)
+    assert (_workspace(*shape) > 0) == (shape in CHUNKS)
+    q, k, v = _qkv(b, sq, sk, hq, hkv, d, dtype, seed=sq + sk)
+    # k and v as views of a cache [B, H, L, D] with rows past Sk that must not be read
+    cache = torch.full((2, b, hkv, sk + 3, d), float("nan"), dtype=dtype, device=dev)
+    cache[0, :, :, :sk], cache[1, :, :, :sk] = k.transpose(1, 2).to(dev), v.transpose(1, 2).to(dev)
+    kd, vd = (c[:, :, :sk].transpose(1, 2) for c in cache)
+    o = flash_attn_func(q.to(dev), kd, vd, causal=causal, window_size=window)
+    close(o, oracle.attention(q, k, v, causal=causal, window=window), what=f"split prefill {shape}")
+    again = flash_attn_func(q.to(dev), kd, vd, causal=causal, window_size=window)
+    assert torch.equal(o, again)
+
+
+def test_split_prefill_captured(dev):
+    """Several chunks inside a graph: every replay equals the eager result."""
+    from torchplusplus_amd.attention import flash_attn_func
+    q, k, v = (t.to(dev) for t in _qkv(1, 33, 4001, 16, 8, 128, torch.bfloat16, seed=9))
+    want = flash_attn_func(q, k, v, causal=True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        o = flash_attn_func(q, k, v, causal=True)
+    for _ in range(3):
+        o.zero_()
+        graph.replay()
+        assert torch.equal(o, want)
+        assert torch.equal(flash_attn_func(q, k, v, causal=True), want)
+
+
+def test_split_prefill_nan_stays_in_its_row(dev):
+    """A NaN query makes its own rows NaN in both forms, and no other."""
+    from torchplusplus_amd.attention import flash_attn_func
+    for sq, sk in ((100, 100), (33, 4001)):
+        q, k, v = _qkv(1, sq, sk, 4, 2, 128, torch.bfloat16, seed=4)
+        q[0, 20, 3] = float("nan")
+        o = flash_attn_func(q.to(dev), k.to(dev), v.to(dev), causal=True).cpu()
+        assert torch.isnan(o[0, 20, 3]).all()
+        o[0, 20, 3] = 0
+        q[0, 20, 3] = 0
+        want = oracle.attention(q, k, v, causal=True)
+        want[0, 20, 3] = 0
+        close(o, want, what="rows without the NaN")

@@ -105,6 +105,27 @@ template <int D> __device__ __forceinline__ int vswz(int r) {
   else return 4 * ((r >> 1) & 1);
 }
 
+// Tiles [t_begin, t_end) of `kt` keys that queries q0 .. q_last see (causal
+// and window bounds are aligned bottom-right: query i sits at key i + Sk - Sq).
+struct KeyBand {
+  int t_begin, t_end;
+};
+__host__ __device__ inline KeyBand key_band(int q0, int q_last, int Sq, int Sk, int left, int right,
+                                            int kt) {
+  const int off = Sk - Sq;
+  int hi = Sk, lo = 0;
+  if (right >= 0) {
+    const int64_t lim = (int64_t)q_last + off + right + 1;
+    hi = lim < hi ? (int)lim : hi;
+  }
+  if (left >= 0) {
+    const int64_t lim = (int64_t)q0 + off - left;
+    lo = lim > 0 ? (int)lim : 0;
+  }
+  const int tb = lo / kt;
+  return {tb, hi > lo ? (hi + kt - 1) / kt : tb};
+}
+
 // K / V ring slots of the prefill kernel: tile t in slot (t - t_begin) % 3
 constexpr int kPrefillSlots = 3;
 template <typename T, int D> struct PrefillSmem {
@@ -581,6 +602,349 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(AttnArgs p, int h
     }
     if (!more) break;
   }
+}
+
+// ---------------------------------------------------------------------------
+// Prefill with few work items (a short prompt, a follow-up turn against a
+// long cache): the keys are split inside the block, and over blocks where
+// that still leaves CUs idle. A block is 32 queries of two heads of a KV head
+// (64 queries of one head when the group size is odd), its 8 waves four key
+// groups of two waves; group g takes the KT-key tiles g, g + 4, ... of the
+// block's chunk of `ct` tiles, staged in its own two-slot LDS ring (the
+// group's first wave fetches K, the second V). The groups' running (m, l, O)
+// are merged through LDS at the end; with more than one chunk the merged fp32
+// partial goes to the workspace, slot = row * nsmax + chunk, and
+// attn_prefill_merge_kernel combines the chunks.
+// What bounds it: attn_prefill_kernel gives a 128-query item all its keys, so
+// 200 queries against 3001 cached keys ran 47 serial tiles on 16 of 256 CUs.
+// Here a round of four 32-key tiles takes 1.1-1.45 us (LDS reads and a barrier
+// per round; the DMA of the next round in flight beside it) and a block's
+// start, merge and stores ~4 us. Splitting the keys in the block first keeps
+// the partials small (fp32 rows are 520 bytes per chunk, written and read
+// back): the same split over blocks alone would write four times as many. Two
+// accumulators per score block (shorter MFMA chains) were no faster.
+template <int D> constexpr int kSplitTile = D == 128 ? 32 : 64; // keys per tile (8 KB of K)
+constexpr int kSplitGroups = 4;
+
+template <typename T, int D>
+__global__ __launch_bounds__(512) void attn_prefill_split_kernel(AttnArgs p, int hpb, int ct, int nsmax,
+                                                                 float *__restrict__ ws_o,
+                                                                 float *__restrict__ ws_ml) {
+  typedef typename VecT<T>::v8 V8;
+  constexpr int KT = kSplitTile<D>, NB = KT / 32; // 32-key blocks per tile
+  constexpr int CPR = D / 8, NT = D / 32, NG = kSplitGroups;
+  constexpr int TU = KT * CPR;                    // 16-byte units per K or V tile
+  constexpr int KPI = 64 / CPR, NDMA = KT / KPI;  // keys per DMA instruction, instructions per tile
+  constexpr int LDO = D + 4;                      // fp32 pitch of a merged row (odd in 16-byte units)
+  constexpr int RING = 2 * NG * 2 * TU, MRG = 8 * 32 * LDO / 4;
+  __shared__ V8 smem[RING > MRG ? RING : MRG];
+  __shared__ float s_m[8][32], s_l[8][32];
+
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = w >> 1, wu = w & 1, h = lane >> 5, ql = lane & 31;
+  const int G = p.Hq / p.Hkv, QL = hpb == 2 ? 32 : 64;
+  const int nqt = (p.Sq + QL - 1) / QL, nhg = p.Hq / hpb, npair = p.B * nhg, ipp = nqt * nsmax;
+  // all items of a (batch, head group) pair on one XCD (XCD = blockIdx % 8)
+  // when the pairs split evenly: their K / V rows stay in its L2
+  int pair, r;
+  if (npair % 8 == 0) {
+    const int j = blockIdx.x / 8;
+    pair = (j / ipp) * 8 + blockIdx.x % 8;
+    r = j % ipp;
+  } else {
+    pair = blockIdx.x / ipp;
+    r = blockIdx.x % ipp;
+  }
+  const int qt = nqt - 1 - r / nsmax, split = r % nsmax; // late (causal: heavy) query tiles first
+  const int b = pair / nhg, hg = pair % nhg;
+  const int hq = hg * hpb + (hpb == 2 ? wu : 0), hk = (hg * hpb) / G;
+  const int q0 = qt * QL, q_last = (q0 + QL < p.Sq ? q0 + QL : p.Sq) - 1;
+  const int qw = q0 + (hpb == 2 ? 0 : wu * 32);
+  const int off = p.Sk - p.Sq;
+  const KeyBand kb = key_band(q0, q_last, p.Sq, p.Sk, p.left, p.right, KT);
+  const int t0 = kb.t_begin + split * ct, t1 = min(kb.t_end, t0 + ct);
+  if (t0 >= t1 && (split > 0 || nsmax > 1)) return; // (no key at all and one chunk: rows of zeros)
+  const int niter = t0 < t1 ? (t1 - t0 + NG - 1) / NG : 0;
+
+  // this wave's DMA: K tiles (first wave of the group) or V tiles (second)
+  const bool kwave = wu == 0;
+  const int64_t ss = kwave ? p.k_ss : p.v_ss;
+  const char *src = kwave ? (const char *)((const T *)p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh)
+                          : (const char *)((const T *)p.v + (int64_t)b * p.v_sb + (int64_t)hk * p.v_sh);
+  const int dkey = lane / CPR, dslot = lane % CPR;
+  V8 *const gring = smem + g * (4 * TU); // [slot][K | V][TU]
+  auto issue = [&](int i) {
+    const int t = t0 + i * NG + g;
+    if (t >= t1) return; // wave-uniform
+    const char *tb = src + (int64_t)t * KT * ss * (int64_t)sizeof(T);
+    const int kmax = p.Sk - 1 - t * KT; // keys past Sk read the last one (masked)
+    V8 *dst = gring + (i & 1) * (2 * TU) + (kwave ? 0 : TU);
+#pragma unroll
+    for (int j = 0; j < NDMA; ++j) {
+      const int key = j * KPI + dkey;
+      const int ch = kwave ? dslot ^ (key & (CPR - 1)) : dslot ^ vswz<D>(key);
+      const unsigned o = (unsigned)((min(key, kmax) * ss + ch * 8) * (int64_t)sizeof(T));
+      __builtin_amdgcn_global_load_lds((const void *)(tb + o),
+                                       (__attribute__((address_space(3))) void *)&dst[j * 64], 16, 0, 0);
+    }
+  };
+  issue(0);
+
+  // q rows, past Sq the last one (never stored); one round trip with the
+  // first tiles, waited for here so that no wait for them sits in the loop
+  const T *qp = (const T *)p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh +
+                (int64_t)min(qw + ql, p.Sq - 1) * p.q_ss;
+  V8 qf[D / 16];
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) qf[ks] = *reinterpret_cast<const V8 *>(qp + ks * 16 + h * 8);
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) asm volatile("" ::"v"(qf[ks]));
+
+  f32x16 o[NT];
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[tt][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  const float c2 = p.scale_log2;
+
+  const unsigned gbase = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char *)gring;
+  // V operand addresses within a tile (attn_prefill_kernel explains the layout)
+  const int grp = lane >> 4, a4 = lane & 3, c4 = (lane >> 2) & 3, kl = 4 * (grp >> 1) + c4;
+  unsigned vo[NT];
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    const int d0 = tt * 32 + 16 * (grp & 1) + 4 * a4;
+    vo[tt] = TU * 16 + kl * D * 2 + (((d0 >> 3) ^ vswz<D>(kl)) << 4) + ((d0 & 7) << 1);
+  }
+
+  auto tile = [&](int t, int slot) {
+    const unsigned base = gbase + slot * (2 * TU * 16);
+    // S^T = K Q^T, fragments two steps ahead
+    constexpr int KS = D / 16;
+    f32x16 s[NB];
+#pragma unroll
+    for (int st = 0; st < NB; ++st)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[st][i] = 0.f;
+    // step i reads two fragments: the two 32-key blocks of K step i, or K
+    // steps 2i and 2i + 1 of a one-block tile
+    constexpr int NS = KS * NB / 2;
+    V8 kr[3][2];
+    auto kfrag = [&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      static_for<2>([&](auto jj) {
+        constexpr int j = decltype(jj)::value, ks = NB == 2 ? i : 2 * i + j;
+        const unsigned a = base + (unsigned)((ql * CPR + ((ks * 2 + h) ^ (ql & (CPR - 1)))) * 16);
+        kr[i % 3][j] = lds_read_b128<(NB == 2 ? j : 0) * 32 * D * 2, V8>(a);
+      });
+    };
+    kfrag(std::integral_constant<int, 0>{});
+    kfrag(std::integral_constant<int, 1>{});
+    static_for<NS>([&](auto ii) {
+      constexpr int i = decltype(ii)::value;
+      if constexpr (i + 2 < NS) kfrag(std::integral_constant<int, i + 2>{});
+      lds_wait_tied<(i + 2 < NS ? 2 : NS - 1 - i) * 2>(kr[i % 3]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        s[j % NB] = mfma32x32<T>(kr[i % 3][j], qf[NB == 2 ? i : 2 * i + j], s[j % NB]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    // online softmax, as attn_prefill_kernel: raw running max moved only by
+    // more than 2^8, masking on band edges
+    const int k0 = t * KT;
+    if ((p.right >= 0 && k0 + KT - 1 > q0 + off + p.right) ||
+        (p.left >= 0 && k0 < q_last + off - p.left) || k0 + KT > p.Sk) {
+      const int qpos = qw + ql + off;
+      int hi = p.Sk - 1;
+      if (p.right >= 0) hi = min(hi, qpos + p.right);
+      const int lo = p.left >= 0 ? max(qpos - p.left, 0) : 0;
+      const int jb = k0 + h * 4;
+      const int ca = max(lo - jb, 0), cb = min(hi - jb, KT - 1);
+      const unsigned ninf = __float_as_uint(-INFINITY);
+#pragma unroll
+      for (int st = 0; st < NB; ++st) {
+        const int l0 = max(ca - 32 * st, 0), h0 = min(cb - 32 * st, 31);
+        const unsigned keep = l0 <= h0 ? ((2u << h0) - 1u) & ~((1u << l0) - 1u) : 0u;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const unsigned bm = (unsigned)__builtin_amdgcn_sbfe((int)keep, (i >> 2) * 8 + (i & 3), 1);
+          s[st][i] = __uint_as_float((__float_as_uint(s[st][i]) & bm) | (ninf & ~bm));
+        }
+      }
+    }
+    float mx[4] = {s[0][0], s[0][1], s[0][2], s[0][3]};
+#pragma unroll
+    for (int st = 0; st < NB; ++st)
+#pragma unroll
+      for (int i = st == 0 ? 4 : 0; i < 16; ++i) mx[i & 3] = fmaxf(mx[i & 3], s[st][i]);
+    float mt = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+    mt = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    const bool move = (mt - m_run) * c2 > 8.f;
+    const float m_new = move ? mt : m_run;
+    const float mc = m_new == -INFINITY ? 0.f : m_new * c2;
+    const float alpha = move ? __builtin_amdgcn_exp2f(m_run * c2 - mc) : 1.f;
+    float ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < NB; ++st)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[st][i], c2, -mc));
+        s[st][i] = e;
+        ps[i & 3] += e;
+      }
+    l_run = l_run * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+    m_run = m_new;
+    if (__any(move)) {
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[tt][i] *= alpha;
+    }
+    V8 pb[2 * NB];
+#pragma unroll
+    for (int c = 0; c < 2 * NB; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) pb[c][j] = from_f32<T>(s[c >> 1][(c & 1) * 8 + j]);
+    // O^T += V^T P^T, one 16-key step ahead
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    constexpr int R = 2 * NT;
+    s16x4 vr[2][R];
+    auto vfrag = [&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        vr[c % 2][2 * tt] = lds_read_tr16<c * 32 * D>(base + vo[tt]);
+        vr[c % 2][2 * tt + 1] = lds_read_tr16<c * 32 * D + 16 * D>(base + vo[tt]);
+      }
+    };
+    vfrag(std::integral_constant<int, 0>{});
+    static_for<2 * NB>([&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+      if constexpr (c + 1 < 2 * NB) vfrag(std::integral_constant<int, c + 1>{});
+      lds_wait_tied<(c + 1 < 2 * NB ? R : 0)>(vr[c % 2]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        const s16x8 r12 = __builtin_shufflevector(vr[c % 2][2 * tt], vr[c % 2][2 * tt + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+        o[tt] = mfma32x32<T>(__builtin_bit_cast(V8, r12), pb[c], o[tt]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  // One barrier per iteration: past it every wave's share of this iteration's
+  // tiles has landed and every wave is done with the other slot, which is
+  // refilled while this iteration computes.
+  for (int i = 0; i < niter; ++i) {
+    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(i + 1);
+    if (t0 + i * NG + g < t1) tile(t0 + i * NG + g, i & 1);
+  }
+  __syncthreads(); // the ring is free
+
+  // merge of the key groups
+  float *const mo = reinterpret_cast<float *>(smem) + (w * 32 + ql) * LDO;
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = o[tt][rg * 4 + e];
+      *reinterpret_cast<f32x4 *>(mo + tt * 32 + rg * 8 + h * 4) = v;
+    }
+  const float l = l_run + __shfl_xor(l_run, 32, kWave);
+  if (h == 0) s_m[w][ql] = m_run, s_l[w][ql] = l;
+  __syncthreads();
+  for (int idx = tid; idx < 64 * CPR; idx += 512) {
+    const int row = idx / CPR, c = idx % CPR, u = row >> 5, rl = row & 31; // u: wave of the groups
+    const int qi = q0 + (hpb == 2 ? 0 : u * 32) + rl, hr = hg * hpb + (hpb == 2 ? u : 0);
+    if (qi >= p.Sq) continue;
+    float mg[NG], mx = -INFINITY;
+#pragma unroll
+    for (int gg = 0; gg < NG; ++gg) mg[gg] = s_m[gg * 2 + u][rl], mx = fmaxf(mx, mg[gg]);
+    const float ms = mx == -INFINITY ? 0.f : mx;
+    float ls = 0.f, v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.f;
+#pragma unroll
+    for (int gg = 0; gg < NG; ++gg) {
+      const float a = __builtin_amdgcn_exp2f((mg[gg] - ms) * c2);
+      ls += a * s_l[gg * 2 + u][rl];
+      const float *q = reinterpret_cast<const float *>(smem) + ((gg * 2 + u) * 32 + rl) * LDO + c * 8;
+      const f32x4 x = *reinterpret_cast<const f32x4 *>(q), y = *reinterpret_cast<const f32x4 *>(q + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += a * x[e], v[e + 4] += a * y[e];
+    }
+    if (nsmax == 1) {
+      const float inv = ls > 0.f ? 1.f / ls : 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= inv;
+      store8((T *)p.o + (int64_t)b * p.o_sb + (int64_t)qi * p.o_ss + (int64_t)hr * p.o_sh + c * 8, v);
+    } else {
+      const int64_t sl = (((int64_t)b * p.Hq + hr) * p.Sq + qi) * nsmax + split;
+      f32x4 x, y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = v[e], y[e] = v[e + 4];
+      *reinterpret_cast<f32x4 *>(ws_o + sl * D + c * 8) = x;
+      *reinterpret_cast<f32x4 *>(ws_o + sl * D + c * 8 + 4) = y;
+      if (c == 0) ws_ml[sl * 2] = mx, ws_ml[sl * 2 + 1] = ls;
+    }
+  }
+}
+
+// Combine the key chunks of every (batch, head, query) row: D / 4 lanes per
+// row, the chunks' (m, l) and outputs read eight at a time.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnArgs p, int QL, int ct, int nsmax,
+                                                                 const float *__restrict__ ws_o,
+                                                                 const float *__restrict__ ws_ml) {
+  constexpr int LPR = D / 4, MG = 8;
+  const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  const int d4 = threadIdx.x % LPR;
+  if (row >= (int64_t)p.B * p.Hq * p.Sq) return;
+  const int qi = (int)(row % p.Sq), hq = (int)(row / p.Sq % p.Hq), b = (int)(row / p.Sq / p.Hq);
+  const int q0 = qi / QL * QL, q_last = (q0 + QL < p.Sq ? q0 + QL : p.Sq) - 1;
+  const KeyBand kb = key_band(q0, q_last, p.Sq, p.Sk, p.left, p.right, kSplitTile<D>);
+  const int ns = (kb.t_end - kb.t_begin + ct - 1) / ct; // chunks written for this query tile
+  float mu = -INFINITY, ls = 0.f, os[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < ns; s0 += MG) {
+    float2 ml[MG];
+    f32x4 ov[MG];
+#pragma unroll
+    for (int j = 0; j < MG; ++j) {
+      const int64_t sl = row * nsmax + (s0 + j < ns ? s0 + j : ns - 1);
+      ml[j] = *reinterpret_cast<const float2 *>(ws_ml + sl * 2);
+      ov[j] = *reinterpret_cast<const f32x4 *>(ws_o + sl * D + d4 * 4);
+    }
+    float mx = mu;
+#pragma unroll
+    for (int j = 0; j < MG; ++j) mx = fmaxf(mx, ml[j].x);
+    const float mn = mx == -INFINITY ? 0.f : mx;
+    const float a = __builtin_amdgcn_exp2f((mu - mn) * p.scale_log2);
+    ls *= a;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) os[e] *= a;
+#pragma unroll
+    for (int j = 0; j < MG; ++j) {
+      const float wgt = s0 + j < ns ? __builtin_amdgcn_exp2f((ml[j].x - mn) * p.scale_log2) : 0.f;
+      ls += wgt * ml[j].y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) os[e] += wgt * ov[j][e];
+    }
+    mu = mx;
+  }
+  const float inv = ls > 0.f ? 1.f / ls : 0.f;
+  typename VecT<T>::v4 pk;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) pk[e] = from_f32<T>(os[e] * inv);
+  *reinterpret_cast<typename VecT<T>::v4 *>((T *)p.o + (int64_t)b * p.o_sb + (int64_t)qi * p.o_ss +
+                                            (int64_t)hq * p.o_sh + d4 * 4) = pk;
 }
 
 // Generic prefill (any D <= 256, any alignment): one wave per (b, query,
@@ -1377,14 +1741,111 @@ static bool strides16(const AttnArgs &a) {
          al(a.v_ss) && al(a.v_sh) && al(a.o_sb) && al(a.o_ss) && al(a.o_sh);
 }
 
+// Prefill plan: the whole-chip kernel (one workgroup per CU looping over 8-wave
+// work items), or the key-split kernel with `nsmax` chunks of `ct` tiles.
+struct PrefillPlan {
+  bool split;
+  int hpb, ct, nsmax;
+  int64_t blocks;
+  size_t ws_bytes;
+};
+
+// Estimated times in us, from measurements of both kernels (bf16, B 1 - 4, Sq
+// 17 - 4096, Sk 64 - 8000): the whole-chip kernel takes 6.5 us plus 1.55 (D =
+// 128; 2.0 with every CU busy) or 1.2 (D = 64) per 64-key tile of its longest
+// CU; a key-split block 4.2 us plus 1.1 (1.45 with most CUs busy) or 1.3 per
+// round of four tiles, and several chunks a merge launch of 2.5 us + 0.55 us
+// per MB of partials. The split kernel is taken where it is expected to be
+// 10% faster at least (the margin covers the estimate's error), e.g. 230
+// causal tokens of 16 heads 12.6 -> 9.0 us, 1000 tokens 32.6 -> 17.0 us, 200
+// tokens against 3001 cached keys 80.4 -> 20.1 us (4 chunks), 33 against 8000
+// 203 -> 17.2 us (16 chunks); left alone: 4 x 512 tokens (20.5 against 21.5
+// us), 4096 tokens in a window of 512 (32 against 50 us).
+static PrefillPlan plan_prefill(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
+                                int left, int right, bool workspace) {
+  PrefillPlan pl{};
+  pl.nsmax = 1;
+  const int64_t G = Hq / Hkv;
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  pl.hpb = G % 2 == 0 ? 2 : 1;
+  const int64_t ql = 64 / pl.hpb, nqt = (Sq + ql - 1) / ql, npair = B * (Hq / pl.hpb);
+  if (npair * nqt > 8 * (int64_t)cus || Sk > (1 << 30)) return pl;
+  // tiles of `kt` keys per query tile of `len` queries: largest and average
+  // (first, middle and last tile)
+  auto tiles = [&](int64_t len, int kt, double &most, double &mean) {
+    const int64_t n = (Sq + len - 1) / len;
+    auto at = [&](int64_t t) {
+      const int64_t q0 = t * len, last = (q0 + len < Sq ? q0 + len : Sq) - 1;
+      const KeyBand kb = key_band((int)q0, (int)last, (int)Sq, (int)Sk, left, right, kt);
+      return (double)(kb.t_end - kb.t_begin);
+    };
+    const double f = at(0), m = at(n / 2), l = at(n - 1);
+    most = f > m ? (f > l ? f : l) : (m > l ? m : l);
+    mean = (f + 2 * m + l) / 4;
+  };
+  double most, mean;
+  const int hpb8 = (G % 4 == 0) ? 4 : (G % 2 == 0) ? 2 : 1;
+  const int64_t len8 = (8 / hpb8) * 32;
+  tiles(len8, kKvTile, most, mean);
+  const double items8 = (double)(B * (Hq / hpb8) * ((Sq + len8 - 1) / len8));
+  const double per8 = D == 128 ? (items8 >= cus ? 2.0 : 1.55) : 1.2;
+  const double whole = items8 * (4.5 + mean * per8) / cus > 4.5 + most * per8
+                           ? 2.0 + items8 * (4.5 + mean * per8) / cus
+                           : 6.5 + most * per8;
+  tiles(ql, D == 128 ? kSplitTile<128> : kSplitTile<64>, most, mean);
+  double best = 0.9 * whole;
+  for (const int n : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+    int ct = ((int)(most + n - 1) / n + kSplitGroups - 1) / kSplitGroups * kSplitGroups;
+    if (ct < kSplitGroups) ct = kSplitGroups;
+    const int ns = most > ct ? (int)((most + ct - 1) / ct) : 1;
+    const double parts = mean / ct > 1 ? mean / ct + (ns > 1 ? 0.5 : 0) : 1; // chunks per query tile
+    const double blocks = (double)(npair * nqt) * (parts < ns ? parts : ns), load = blocks / cus;
+    const double c = D == 128 ? (load >= 0.75 ? 1.45 : 1.1) : 1.3;
+    const double longest = 4.2 + (most < ct ? (int)(most + kSplitGroups - 1) / kSplitGroups : ct / kSplitGroups) * c;
+    const double each = 4.2 + (mean / (parts < ns ? parts : ns) / kSplitGroups + 0.4) * c;
+    const double rounds = load <= 1 ? 1 : (load + 0.5 < ceil(load) ? load + 0.5 : ceil(load));
+    const size_t ws = ns > 1 ? (size_t)(B * Hq * Sq * ns) * (size_t)(D + 2) * sizeof(float) : 0;
+    const double t = 2.0 + (rounds * each > longest ? rounds * each : longest) +
+                     (ns > 1 ? 2.5 + 0.55e-6 * (double)ws : 0.0);
+    if (t < best && (ns == 1 || workspace)) {
+      best = t;
+      pl.split = true;
+      pl.ct = ct, pl.nsmax = ns, pl.ws_bytes = ws;
+      pl.blocks = npair * nqt * ns;
+    }
+    if (ct == kSplitGroups) break;
+  }
+  return pl;
+}
+
 template <typename T>
-static int launch_prefill(const AttnArgs &a, int64_t D, hipStream_t st, const char *name) {
+static int launch_prefill(const AttnArgs &a, int64_t D, void *ws, size_t ws_bytes, hipStream_t st,
+                          const char *name) {
   if (a.B == 0 || a.Sq == 0) return TPP_OK;
   const int G = a.Hq / a.Hkv;
-  // the tiled kernel addresses a 64-row K / V tile with 32-bit byte offsets
+  // the tiled kernels address a 64-row K / V tile with 32-bit byte offsets
   const bool rows_fit = a.k_ss >= 0 && a.v_ss >= 0 && (int64_t)kKvTile * a.k_ss * 2 < (1LL << 31) &&
                         (int64_t)kKvTile * a.v_ss * 2 < (1LL << 31);
   if ((D == 64 || D == 128) && strides16(a) && rows_fit) {
+    const PrefillPlan pl = plan_prefill(a.B, a.Sq, a.Sk, a.Hq, a.Hkv, D, a.left, a.right, ws != nullptr);
+    if (pl.split) {
+      if (pl.ws_bytes > ws_bytes)
+        return set_error(TPP_E_WORKSPACE, "%s: workspace of %zu bytes required", name, pl.ws_bytes);
+      const int64_t rows = (int64_t)a.B * a.Hq * a.Sq;
+      float *wo = (float *)ws, *wml = wo + (pl.nsmax > 1 ? rows * pl.nsmax * D : 0);
+      auto go = [&](auto dd) {
+        constexpr int DD = decltype(dd)::value;
+        attn_prefill_split_kernel<T, DD><<<dim3((unsigned)pl.blocks), dim3(512), 0, st>>>(
+            a, pl.hpb, pl.ct, pl.nsmax, wo, wml);
+        constexpr int rpb = 256 / (DD / 4); // rows per merge block
+        if (pl.nsmax > 1)
+          attn_prefill_merge_kernel<T, DD><<<dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(256), 0, st>>>(
+              a, 64 / pl.hpb, pl.ct, pl.nsmax, wo, wml);
+      };
+      if (D == 128) go(std::integral_constant<int, 128>{});
+      else go(std::integral_constant<int, 64>{});
+      return check_launch(name);
+    }
     const int hpb = (G % 4 == 0) ? 4 : (G % 2 == 0) ? 2 : 1;
     constexpr int QG = kPrefillQG;
     constexpr int NW = kPrefillWaves;
@@ -1537,24 +1998,48 @@ static AttnArgs make_args(const void *q, const void *k, const void *v, void *o,
   return a;
 }
 
-extern "C" int tpp_attn_prefill(const void *q, const void *k, const void *v, void *o,
-                                const int64_t *q_strides, const int64_t *k_strides,
-                                const int64_t *v_strides, const int64_t *o_strides, int64_t B,
-                                int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
-                                float softmax_scale, int causal, int window_left,
-                                int window_right, int dtype, void *stream) {
+extern "C" size_t tpp_attn_prefill_workspace_size(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq,
+                                                  int64_t Hkv, int64_t D, int causal,
+                                                  int window_left, int window_right) {
+  if (B < 1 || Sq < 1 || Sk < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || (D != 64 && D != 128) ||
+      B > 0x7fffffff || Sq > 0x7fffffff || Sk > 0x7fffffff)
+    return 0;
+  const int right = causal ? 0 : (window_right < 0 ? -1 : window_right);
+  return plan_prefill(B, Sq, Sk, Hq, Hkv, D, window_left < 0 ? -1 : window_left, right, true).ws_bytes;
+}
+
+extern "C" int tpp_attn_prefill_ws(const void *q, const void *k, const void *v, void *o,
+                                   const int64_t *q_strides, const int64_t *k_strides,
+                                   const int64_t *v_strides, const int64_t *o_strides, int64_t B,
+                                   int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
+                                   float softmax_scale, int causal, int window_left,
+                                   int window_right, int dtype, void *workspace, size_t ws_bytes,
+                                   void *stream) {
   const char *name = "tpp_attn_prefill";
   if (!q_strides || !k_strides || !v_strides || !o_strides)
     return set_error(TPP_E_INVALID, "%s: null stride array", name);
   if (B > 0x7fffffff || Sq > 0x7fffffff || Sk > 0x7fffffff)
     return set_error(TPP_E_UNSUPPORTED, "%s: dimension too large", name);
+  if (workspace && !aligned16(workspace))
+    return set_error(TPP_E_WORKSPACE, "%s: the workspace must be 16-byte aligned", name);
   const int right = causal ? 0 : (window_right < 0 ? -1 : window_right);
   const int left = window_left < 0 ? -1 : window_left;
   AttnArgs a = make_args(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Sq, Sk, Hq,
                          Hkv, D, softmax_scale, left, right);
   if (int e = check_attn(name, a, D)) return e;
   hipStream_t st = as_stream(stream);
-  return TPP_DISPATCH_HALF(dtype, [&] { return launch_prefill<T>(a, D, st, name); });
+  return TPP_DISPATCH_HALF(dtype, [&] { return launch_prefill<T>(a, D, workspace, ws_bytes, st, name); });
+}
+
+extern "C" int tpp_attn_prefill(const void *q, const void *k, const void *v, void *o,
+                                const int64_t *q_strides, const int64_t *k_strides,
+                                const int64_t *v_strides, const int64_t *o_strides, int64_t B,
+                                int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
+                                float softmax_scale, int causal, int window_left,
+                                int window_right, int dtype, void *stream) {
+  return tpp_attn_prefill_ws(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Sq, Sk, Hq,
+                             Hkv, D, softmax_scale, causal, window_left, window_right, dtype, nullptr,
+                             0, stream);
 }
 
 extern "C" size_t tpp_attn_decode_workspace_size(int64_t B, int64_t Hq, int64_t Hkv, int64_t D,

@@ -621,9 +621,16 @@ at::Tensor attn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, bool causal, int64
   const int64_t ks[3] = {k.stride(0), k.stride(1), k.stride(2)};
   const int64_t vs[3] = {v.stride(0), v.stride(1), v.stride(2)};
   const int64_t os[3] = {o.stride(0), o.stride(1), o.stride(2)};
-  check_rc(tpp_attn_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), qs, ks, vs,
-                            os, B, Sq, Sk, Hq, Hkv, D, (float)softmax_scale, causal ? 1 : 0,
-                            (int)window_left, (int)window_right, dtype_code(q), cur_stream(q)),
+  // partials of a key split over workgroups (none for most shapes): from the
+  // caching allocator, so the bytes belong to this call on its stream
+  const size_t wsb = tpp_attn_prefill_workspace_size(B, Sq, Sk, Hq, Hkv, D, causal ? 1 : 0,
+                                                     (int)window_left, (int)window_right);
+  at::Tensor ws;
+  if (wsb) ws = torch::empty({(int64_t)wsb}, q.options().dtype(at::kByte));
+  check_rc(tpp_attn_prefill_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), qs, ks, vs,
+                               os, B, Sq, Sk, Hq, Hkv, D, (float)softmax_scale, causal ? 1 : 0,
+                               (int)window_left, (int)window_right, dtype_code(q),
+                               wsb ? ws.data_ptr() : nullptr, wsb, cur_stream(q)),
            "flash_attn_func");
   return o;
 }
