@@ -141,6 +141,18 @@ int tpp_qkv_rope_cache(const void *qkv, void *q_out, void *k_cache,
                        int64_t Lmax, float eps, int dtype, int cs_dtype,
                        void *stream);
 
+/* Per-head RMSNorm over D (q_norm_w / k_norm_w [D], NULL = none) and RoPE of
+ * q [B, S, Hq, D] and k [B, S, Hk, D] in place, in one launch: token t's heads
+ * are contiguous at q + t * q_stride and k + t * k_stride; cos/sin [S, D] row s
+ * for sequence index s. Rounded to T after the norm and after the rotation.
+ * D in {64, 128, 256}; 16-byte aligned pointers and strides. Replaces q_norm,
+ * k_norm and rope_apply at torchpp/attention/mha.py:71-80 (swa.py, mqa.py the
+ * same). */
+int tpp_qk_norm_rope(void *q, int64_t q_stride, void *k, int64_t k_stride,
+                     const void *q_norm_w, const void *k_norm_w, const void *cos,
+                     const void *sin, int64_t B, int64_t S, int64_t Hq, int64_t Hk, int64_t D,
+                     float eps_q, float eps_k, int dtype, int cs_dtype, void *stream);
+
 /* ---- linear layers ------------------------------------------------------- */
 
 /* y[M, N] = act(T(x[M, K] . w[N, K]^T + bias)) on MFMA; w is the nn.Linear

@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from torchplusplus_amd.attention._common import head_rmsnorm, rope_bshd
+from torchplusplus_amd.attention._common import norm_rope_qk
 from torchplusplus_amd.attention.flash import flash_attn_func
 from torchplusplus_amd.dlops.linear import linear
 
@@ -38,9 +38,9 @@ class MultiHeadAttention(nn.Module):
 
     def forward(self, x: torch.Tensor, cos, sin):
         bsz, seq, _ = x.shape
-        q = head_rmsnorm(self._heads(linear(x, self.Wq.weight), bsz, seq), self.q_norm)
-        k = head_rmsnorm(self._heads(linear(x, self.Wk.weight), bsz, seq), self.k_norm)
+        q = self._heads(linear(x, self.Wq.weight), bsz, seq)
+        k = self._heads(linear(x, self.Wk.weight), bsz, seq)
         v = self._heads(linear(x, self.Wv.weight), bsz, seq)
-        q, k = rope_bshd(q, cos, sin), rope_bshd(k, cos, sin)
+        q, k = norm_rope_qk(q, k, self.q_norm, self.k_norm, cos, sin)
         o = flash_attn_func(q, k, v, causal=True).reshape(bsz, seq, self.embed_dim)
         return linear(o, self.out_projection.weight, self.out_projection.bias)

@@ -7,7 +7,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from torchplusplus_amd.attention._common import head_rmsnorm, rope_bshd
+from torchplusplus_amd.attention._common import norm_rope_qk
 from torchplusplus_amd.attention.flash import flash_attn_func
 from torchplusplus_amd.dlops.linear import linear
 
@@ -33,8 +33,7 @@ class MultiQueryAttention(nn.Module):
         q = linear(x, self.Wq.weight).view(bsz, seq, self.num_q_head, self.head_dim)
         k = linear(x, self.Wk.weight).view(bsz, seq, 1, self.head_dim)
         v = linear(x, self.Wv.weight).view(bsz, seq, 1, self.head_dim)
-        if self.qk_norm:
-            q, k = head_rmsnorm(q, self.q_norm), head_rmsnorm(k, self.k_norm)
-        q, k = rope_bshd(q, cos, sin), rope_bshd(k, cos, sin)
+        norms = (self.q_norm, self.k_norm) if self.qk_norm else (None, None)
+        q, k = norm_rope_qk(q, k, *norms, cos, sin)
         o = flash_attn_func(q, k, v, causal=True)
         return linear(o.reshape(bsz, seq, self.embed_dim), self.out_projection.weight)

@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import torch
 
-from torchplusplus_amd.attention._common import head_rmsnorm, rope_bshd
+from torchplusplus_amd.attention._common import norm_rope_qk
 from torchplusplus_amd.attention.flash import flash_attn_func
 from torchplusplus_amd.attention.mha import MultiHeadAttention
 from torchplusplus_amd.dlops.linear import linear
@@ -20,10 +20,10 @@ class SlidingWindowAttention(MultiHeadAttention):
 
     def forward(self, x: torch.Tensor, cos, sin):
         bsz, seq, _ = x.shape
-        q = head_rmsnorm(self._heads(linear(x, self.Wq.weight), bsz, seq), self.q_norm)
-        k = head_rmsnorm(self._heads(linear(x, self.Wk.weight), bsz, seq), self.k_norm)
+        q = self._heads(linear(x, self.Wq.weight), bsz, seq)
+        k = self._heads(linear(x, self.Wk.weight), bsz, seq)
         v = self._heads(linear(x, self.Wv.weight), bsz, seq)
-        q, k = rope_bshd(q, cos, sin), rope_bshd(k, cos, sin)
+        q, k = norm_rope_qk(q, k, self.q_norm, self.k_norm, cos, sin)
         o = flash_attn_func(q, k, v, causal=True, window_size=(self.window_size - 1, 0))
         return linear(o.reshape(bsz, seq, self.embed_dim), self.out_projection.weight,
                       self.out_projection.bias)

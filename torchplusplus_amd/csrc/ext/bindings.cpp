@@ -278,6 +278,47 @@ void qkv_rope_cache(at::Tensor qkv, at::Tensor q_out, at::Tensor k_cache, at::Te
            "qkv_rope_cache");
 }
 
+// per-head RMSNorm (optional) + RoPE, in place on q [B, S, Hq, D] and k
+// [B, S, Hk, D]; false (nothing done) for layouts, head sizes and alignments
+// that the one-launch kernel does not take
+bool qk_norm_rope(at::Tensor q, at::Tensor k, c10::optional<at::Tensor> q_norm_w,
+                  c10::optional<at::Tensor> k_norm_w, double eps_q, double eps_k,
+                  at::Tensor cos_cache, at::Tensor sin_cache) {
+  TORCH_CHECK(q.is_cuda() && k.is_cuda() && is_half_or_bf16(q) && k.scalar_type() == q.scalar_type(),
+              "q and k must be CUDA half/bfloat16 tensors of one dtype");
+  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && q.size(0) == k.size(0) && q.size(1) == k.size(1) &&
+                  q.size(3) == k.size(3),
+              "q and k must be [B, S, H, D] with the same B, S and D");
+  const int64_t B = q.size(0), S = q.size(1), D = q.size(3);
+  if ((D != 64 && D != 128 && D != 256) || q.numel() == 0 || k.numel() == 0) return false;
+  auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  auto rows_ok = [&](const at::Tensor &t) { // token-major, contiguous heads, 16-byte rows
+    return t.stride(3) == 1 && t.stride(2) == D && t.stride(1) % 8 == 0 && t.stride(1) >= t.size(2) * D &&
+           (B == 1 || t.stride(0) == S * t.stride(1)) && al16(t.data_ptr());
+  };
+  check_rope_tables(q, cos_cache, sin_cache, S, D);
+  auto weight = [&](const c10::optional<at::Tensor> &w) -> at::Tensor {
+    if (!w.has_value() || !w->defined()) return at::Tensor();
+    TORCH_CHECK(w->is_cuda(), "weight must be CUDA");
+    TORCH_CHECK(w->scalar_type() == q.scalar_type(),
+                "weight must have the input's dtype (half or bfloat16)");
+    TORCH_CHECK(w->dim() == 1 && w->size(0) == D, "weight must be 1-D and length == embed_dim");
+    return w->contiguous();
+  };
+  const at::Tensor qw = weight(q_norm_w), kw = weight(k_norm_w);
+  const void *qp = qw.defined() ? qw.data_ptr() : nullptr, *kp = kw.defined() ? kw.data_ptr() : nullptr;
+  if (!rows_ok(q) || !rows_ok(k) || !al16(qp) || !al16(kp) || !al16(cos_cache.data_ptr()) ||
+      !al16(sin_cache.data_ptr()))
+    return false;
+  c10::DeviceGuard g(q.device());
+  check_rc(tpp_qk_norm_rope(q.data_ptr(), q.stride(1), k.data_ptr(), k.stride(1), qp, kp,
+                            cos_cache.data_ptr(), sin_cache.data_ptr(), B, S, q.size(2), k.size(2), D,
+                            (float)eps_q, (float)eps_k, dtype_code(q), dtype_code(cos_cache),
+                            cur_stream(q)),
+           "qk_norm_rope");
+  return true;
+}
+
 // ---- Linear + activation (binding.cu:11-160) --------------------------------
 void check_linear(const at::Tensor &input, const at::Tensor &weight) {
   TORCH_CHECK(input.dim() >= 1, "Input must be at least 1D");
@@ -868,6 +909,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q_out"), py::arg("k_cache"), py::arg("v_cache"), py::arg("q_norm_w"),
         py::arg("k_norm_w"), py::arg("cos"), py::arg("sin"), py::arg("positions"),
         py::arg("eps") = 1e-6);
+  m.def("qk_norm_rope_", &qk_norm_rope,
+        "per-head RMSNorm + RoPE of q and k [B, S, H, D], in place; false if it does not take them",
+        py::arg("q"), py::arg("k"), py::arg("q_norm_w"), py::arg("k_norm_w"), py::arg("eps_q"),
+        py::arg("eps_k"), py::arg("cos_cache"), py::arg("sin_cache"));
   m.def("LinearGelu", &linear_gelu, "Linear + GeLU(tanh) (fp16/bf16, MFMA)", py::arg("input"),
         py::arg("weight"), py::arg("bias") = py::none());
   m.def("LinearSilu", &linear_silu, "Linear + SiLU (fp16/bf16, MFMA)", py::arg("input"),
