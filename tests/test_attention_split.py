@@ -84,3 +84,43 @@ def test_split_prefill_nan_stays_in_its_row(dev):
         want = oracle.attention(q, k, v, causal=True)
         want[0, 20, 3] = 0
         close(o, want, what="rows without the NaN")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,hq,hkv,d,cap,window", [
+    (8, 16, 8, 128, 3000, -1),   # splits merged in the kernel
+    (3, 6, 3, 64, 2500, -1),     # merge kernel, groups of two
+    (2, 8, 2, 128, 5000, -1),    # groups of four
+    (8, 16, 8, 128, 3000, 200),  # a window, from inside a batch
+    (1, 8, 1, 64, 4097, 700), (16, 8, 8, 128, 130, -1)])
+def test_decode_lengths_far_below_the_capacity(dev, dtype, b, hq, hkv, d, cap, window):
+    """Sequences of every length in one batch (none, one key, a batch of keys
+    and one more, all of the capacity, past it): the keys are dealt to the
+    splits by each sequence's length. The workspace starts as NaN past its
+    counters, so a slot that no split wrote must not be read."""
+    import ctypes
+    from torchplusplus_amd._native import lib
+    g = torch.Generator().manual_seed(cap)
+    q = torch.randn(b, 1, hq, d, generator=g).to(dtype)
+    k, v = (torch.randn(b, hkv, cap, d, generator=g).to(dtype) for _ in range(2))
+    pool = [0, 1, 129, cap, cap + 5, 128, 511, 2 * cap // 3, 64, 65, 700, 2, cap - 1, 257, 300, 1000]
+    lens = torch.tensor([min(x, cap + 5) for x in pool[:b]] if b > 1 else [300], dtype=torch.int32)
+    lb, ptr, i64 = lib(), ctypes.c_void_p, ctypes.c_int64
+    lb.tpp_attn_decode_workspace_size.restype = ctypes.c_size_t
+    size = lb.tpp_attn_decode_workspace_size(*map(i64, (b, hq, hkv, d, cap)))
+    ws = torch.full((size // 4 + 64,), float("nan"), dtype=torch.float32, device=dev)
+    ws[:16384] = 0
+    qd, kd, vd, ld = q.to(dev), k.to(dev), v.to(dev), lens.to(dev)
+    o = torch.full_like(qd, float("nan"))
+    s3 = lambda *a: (i64 * 3)(*a)  # noqa: E731
+    for _ in range(2):  # the second call finds the counters at zero again
+        rc = lb.tpp_attn_decode(
+            ptr(qd.data_ptr()), ptr(kd.data_ptr()), ptr(vd.data_ptr()), ptr(o.data_ptr()),
+            s3(hq * d, hq * d, d), s3(hkv * cap * d, d, cap * d), s3(hkv * cap * d, d, cap * d),
+            s3(hq * d, hq * d, d), ptr(ld.data_ptr()), i64(b), i64(hq), i64(hkv), i64(d), i64(cap),
+            ctypes.c_float(0), ctypes.c_int(window), ctypes.c_int(0 if dtype == torch.float16 else 1),
+            ptr(ws.data_ptr()), ctypes.c_size_t(size), ptr(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        want = oracle.decode_attention(q, k, v, lens.clamp(max=cap), window_left=window)
+        close(o, want, what=f"decode lens {lens.tolist()} cap {cap} window {window}")
+        o.fill_(float("nan"))

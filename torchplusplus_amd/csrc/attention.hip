@@ -29,10 +29,10 @@
 //    so a K/V tile in LDS serves up to 4 heads; causal/window tiles outside
 //    the block's band are skipped, masks are evaluated only on band edges,
 //    and the heaviest (latest) query tiles are dispatched first.
-// Decode kernel: a block = (batch, KV head, key chunk); each 16-lane DPP row
+// Decode kernel: a block = (batch, KV head, split); each 16-lane DPP row
 // (D/8 lanes) handles one key, all query heads of the group are scored
 // against it, online softmax per lane, then log-sum-exp merges across rows,
-// waves (LDS) and chunks (a small merge kernel per (batch, KV head)).
+// waves (LDS) and splits (in the last block, or a small merge kernel).
 #include "tpp_common.hpp"
 
 #include <atomic>
@@ -1260,11 +1260,44 @@ __device__ __forceinline__ void attn_decode_oproj_tail(const AttnArgs &p, const 
   resid[(int64_t)b * E + n] = from_f32<T>(to_f32(rres) + to_f32(from_f32<T>(sum)));
 }
 
+// How a sequence's keys are dealt to the splits of its pair: whole batches of
+// `stride` keys (a power of two) from key `lead`, the batch that holds the
+// first visible key `lo`, `batches` of them per split. By the sequence's
+// length: runs cut from the capacity left most splits empty where the cache
+// has room to spare (bf16, 16 / 8 heads, D 128: 8 x 500 keys of 8192 14.9 ->
+// 10.4 us, 1 x 900 13.7 -> 9.2 us, 32 / 8 heads 16 x 2000 of 4096 60.6 -> 41.1
+// us; with the folded projection 8 x 2058 of 2304 22.0 -> 20.6 us). Dealing
+// the batches to the splits in turn instead was 5% slower at 16000 keys.
+struct SplitRun {
+  int lo, lead, nbatch, batches;
+  // splits that have a batch (the first `live`), at least one
+  __host__ __device__ int live() const { return nbatch > 0 ? (nbatch + batches - 1) / batches : 1; }
+};
+// x / n as a multiply by inv = 2^32 / n rounded up (0 for n = 1), exact for
+// x * n < 2^32. A decode block's first loads wait for its split and sequence:
+// two integer divisions there (~60 dependent instructions) cost 0.2 us.
+__host__ __device__ inline unsigned inv_of(int n) {
+  return n > 1 ? (unsigned)((1ULL << 32) / (unsigned)n + 1) : 0u;
+}
+__host__ __device__ inline int div_inv(unsigned x, unsigned inv) {
+  return inv ? (int)(((uint64_t)x * inv) >> 32) : (int)x;
+}
+__host__ __device__ inline SplitRun split_run(int L, int left, int stride, int nsplit, unsigned inv) {
+  SplitRun r;
+  r.lo = left >= 0 && L - 1 - left > 0 ? L - 1 - left : 0;
+  r.lead = r.lo & ~(stride - 1);
+  r.nbatch = L > r.lead ? (int)((unsigned)(L - r.lead + stride - 1) / (unsigned)stride) : 0;
+  const int per = div_inv((unsigned)(r.nbatch + nsplit - 1), inv); // < 2^24 batches, nsplit <= 256
+  r.batches = per > 0 ? per : 1;
+  return r;
+}
+
 template <typename T, int D, int G, int NW, bool OP = false>
 __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const int *__restrict__ seqlens,
                                                               int fixed_len, float *__restrict__ ws_o,
-                                                              float *__restrict__ ws_ml, int chunk,
-                                                              int nsplit, DecodeFuse fz,
+                                                              float *__restrict__ ws_ml, int nsplit,
+                                                              unsigned nsplit_inv, unsigned hkv_inv,
+                                                              DecodeFuse fz,
                                                               int *__restrict__ counters,
                                                               DecodeOproj op) {
   typedef typename VecT<T>::v8 V8;
@@ -1295,10 +1328,10 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     // (XCD = blockIdx % 8): all splits of a (batch, KV head) pair share an
     // XCD, so their partials meet in that XCD's L2
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int pair = (slot / nsplit) * 8 + xcd;
-    split = slot % nsplit;
-    hk = pair % p.Hkv;
-    b = pair / p.Hkv;
+    const int group = div_inv(slot, nsplit_inv), pair = group * 8 + xcd;
+    split = slot - group * nsplit;
+    b = div_inv(pair, hkv_inv);
+    hk = pair - b * p.Hkv;
   }
   const T *kp = (const T *)p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh + dp * 8;
   const T *vp = (const T *)p.v + (int64_t)b * p.v_sb + (int64_t)hk * p.v_sh + dp * 8;
@@ -1318,14 +1351,24 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
       vr[u] = ld_nt(reinterpret_cast<const V8 *>(vp + (int64_t)key * p.v_ss));
     }
   };
-  // The first two batches of the chunk go out before the sequence length is
-  // known (their keys depend on the block alone; clamped to the cache), so
-  // that round trip overlaps the first K/V loads. Three register sets: while
-  // one batch is scored the next two are in flight.
-  const int first = split * chunk + w * KPW;
+  // The split's keys: the sequence's batches in `nsplit` even runs (by its
+  // length, not the cache's: a length far below the capacity still spreads
+  // over all splits), from the window's first batch on. Splits without a batch
+  // leave at once, except that the folded projection needs every workgroup.
+  // The length is one scalar load ahead of the first K/V loads (0.4 us;
+  // loading two batches of the capacity's split before the length was known
+  // cost more wherever the sequence is short: 64 KB per batch and block).
+  const int Lraw = seqlens ? seqlens[b] : fixed_len;
+  const int L = Lraw < p.Sk ? (Lraw > 0 ? Lraw : 0) : p.Sk; // never read past the cache
+  const SplitRun run = split_run(L, p.left, STRIDE, nsplit, nsplit_inv);
+  const int64_t c0 = run.lead + (int64_t)split * run.batches * STRIDE;
+  if (!OP && split > 0 && c0 >= L) return;
+  const int first = (int)(c0 < L ? c0 : L) + w * KPW;
+  const int last0 = L > 0 ? L - 1 : 0;
+  // Three register sets: while one batch is scored the next two are in flight.
   V8 k0[U], v0[U], k1[U], v1[U], k2[U], v2[U];
-  load_batch(first, p.Sk - 1, k0, v0);
-  load_batch(first + STRIDE, p.Sk - 1, k1, v1);
+  load_batch(first, last0, k0, v0);
+  load_batch(first + STRIDE, last0, k1, v1);
   if constexpr (OP) {
     // the projection weight tile W[32 j .. 32 j + 31][x G D .. + G D) by
     // LDS-DMA (1 KB per wave instruction). Issued before the prologue loads,
@@ -1345,15 +1388,10 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     }
   }
 
-  const int Lraw = seqlens ? seqlens[b] : fixed_len;
-  const int L = Lraw < p.Sk ? (Lraw > 0 ? Lraw : 0) : p.Sk; // never read past the cache
-  int lo = 0;
-  if (p.left >= 0) lo = L - 1 - p.left > 0 ? L - 1 - p.left : 0;
-  int k_begin = split * chunk, k_end = k_begin + chunk;
-  k_begin = k_begin > lo ? k_begin : lo;
-  k_end = k_end < L ? k_end : L;
+  const int k_begin = (int)(c0 > run.lo ? (c0 < L ? c0 : L) : run.lo);
+  int k_end = (int)(c0 + (int64_t)run.batches * STRIDE < L ? c0 + (int64_t)run.batches * STRIDE : L);
   // fused prologue: position L-1 is the new token; this block attends to it
-  // from registers (if it falls in its chunk) and the cache loop stops before it
+  // from registers (if it falls in its run) and the cache loop stops before it
   const bool fused = fz.qkv != nullptr;
   const int pnew = L - 1;
   const bool own_new = fused && Lraw <= p.Sk && pnew >= k_begin && pnew < k_end;
@@ -1478,10 +1516,10 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
   // Whole triples of batches in the loop (a single exit: with a break after
   // every batch the compiler merges the exits into one latch, whose state
   // then has a batch in flight, and waits for everything at the loop head),
-  // the last one or two batches after it. Batches past the chunk that a
+  // the last one or two batches after it. Batches past the keys that a
   // triple loads are clamped rows and never scored.
   // this wave's keys: first + i*STRIDE + u*NW*KPW + row, scored iff in
-  // [k_begin, k_end) (a window can start inside the chunk)
+  // [k_begin, k_end) (a window can start inside a batch)
   const int k_last = k_end > 0 ? k_end - 1 : 0;
   int nbat = k_begin < k_end && first < k_end ? (k_end - first + STRIDE - 1) / STRIDE : 0;
   int base = first;
@@ -1567,8 +1605,9 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     }
   }
   __syncthreads();
-  // merge the NW waves: thread -> (gi, d); write this chunk's partial, or the
-  // final output when the whole key range is one chunk
+  const int live = run.live(); // splits with a batch (at least one)
+  // merge the NW waves: thread -> (gi, d); write this split's partial, or the
+  // final output when one split has all the keys
   for (int idx = threadIdx.x; idx < G * D; idx += blockDim.x) {
     const int gi = idx / D, d = idx % D;
     float mx = -INFINITY;
@@ -1583,7 +1622,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
       os += red_o[ww][gi][d] * c;
     }
     const int hq = hk * G + gi;
-    if (nsplit == 1) {
+    if (!OP && live == 1) {
       T *op = (T *)p.o + (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh;
       op[d] = from_f32<T>(ls > 0.f ? os / ls : 0.f);
       continue;
@@ -1606,12 +1645,12 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     else attn_decode_oproj_tail<T, D, G, NW, 8>(p, ws_o, nsplit, op, s_w, s_o, s_red);
     return;
   }
-  if (!counters || nsplit == 1) return;
+  if (!counters || live == 1) return;
   // The last block of the pair to finish merges the splits. Every thread
   // waits for its partial stores to reach L2 (an explicit vmcnt(0): the
   // workgroup-scope fence of __syncthreads does not wait for global stores),
   // then one thread counts the block in with an atomic in L2; the block that
-  // takes the count to nsplit reads the other partials from the same L2.
+  // takes the count to `live` reads the other partials from the same L2.
   // Each partial slot is whole 128-byte lines written by one block only, and
   // a block reads other blocks' slots only here, so this CU's L1 (clean at
   // kernel start) holds no stale copy of them.
@@ -1625,8 +1664,8 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     // atomic is performed in that XCD's L2 either way
     const int old = __hip_atomic_fetch_add(&counters[pair], 1, __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-    s_last = old == nsplit - 1;
-    if (old == nsplit - 1) // leave the counter at 0 for the next launch
+    s_last = old == live - 1;
+    if (old == live - 1) // leave the counter at 0 for the next launch
       __hip_atomic_store(&counters[pair], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
@@ -1640,11 +1679,11 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     // first rescale the running sums (online softmax)
     constexpr int MG = 8;
     float mu = -INFINITY, ls = 0.f, os = 0.f;
-    for (int s0 = 0; s0 < nsplit; s0 += MG) {
+    for (int s0 = 0; s0 < live; s0 += MG) {
       float mv[MG], lv[MG], ov[MG];
 #pragma unroll
       for (int j = 0; j < MG; ++j) {
-        const int sp = s0 + j < nsplit ? s0 + j : nsplit - 1;
+        const int sp = s0 + j < live ? s0 + j : live - 1;
         const float *q = sl + (int64_t)sp * (D + 32);
         mv[j] = q[D];
         lv[j] = q[D + 1];
@@ -1653,14 +1692,14 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
       float mx = mu;
 #pragma unroll
       for (int j = 0; j < MG; ++j)
-        if (s0 + j < nsplit) mx = fmaxf(mx, mv[j]);
+        if (s0 + j < live) mx = fmaxf(mx, mv[j]);
       const float mn = mx == -INFINITY ? 0.f : mx;
       const float a = mu == -INFINITY ? 0.f : exp2f(mu - mn);
       ls *= a;
       os *= a;
 #pragma unroll
       for (int j = 0; j < MG; ++j) {
-        const float wgt = s0 + j < nsplit ? exp2f(mv[j] - mn) : 0.f;
+        const float wgt = s0 + j < live ? exp2f(mv[j] - mn) : 0.f;
         ls += wgt * lv[j];
         os += wgt * ov[j];
       }
@@ -1671,33 +1710,40 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
   }
 }
 
-// Merge the chunk partials of one (batch, KV head): grid (Hkv, B), 256
+// Merge the split partials of one (batch, KV head): grid (Hkv, B), 256
 // threads, G query heads. A separate launch on purpose: publishing partials
 // across blocks inside one kernel needs device-scope release/acquire fences,
 // which on MI355X write back / invalidate the XCD's L2 (the 8 XCD L2s are not
 // coherent) and cost far more than a kernel boundary.
 template <typename T, int D, int G>
-__global__ __launch_bounds__(G * D) void attn_decode_merge_kernel(AttnArgs p,
+__global__ __launch_bounds__(G * D) void attn_decode_merge_kernel(AttnArgs p, const int *__restrict__ seqlens,
+                                                                  int fixed_len, int stride,
                                                                   const float *__restrict__ ws_o,
                                                                   const float *__restrict__ ws_ml,
-                                                                  int nsplit) {
+                                                                  int slots, unsigned slots_inv) {
   constexpr int PRE = 16; // partial outputs prefetched per thread
   __shared__ float s_w[G][kDecMaxSplit], s_l[G][kDecMaxSplit], s_inv[G];
   const int hk = blockIdx.x, b = blockIdx.y, lane = lane_id(), w = wave_id();
   const int gi = threadIdx.x / D, d = threadIdx.x % D;
-  const int64_t s0 = ((int64_t)b * p.Hq + hk * G) * nsplit; // slot of (gi = 0, split 0)
-  // this thread's partial outputs do not depend on the weights: load first
-  const float *po = ws_o + (s0 + (int64_t)gi * nsplit) * D + d;
+  const int64_t s0 = ((int64_t)b * p.Hq + hk * G) * slots; // slot of (gi = 0, split 0)
+  // this thread's partial outputs and the (m, l) pairs do not depend on the
+  // length: load first (slots without keys hold anything and are not used)
+  const float *po = ws_o + (s0 + (int64_t)gi * slots) * D + d;
   float pre[PRE];
 #pragma unroll
-  for (int j = 0; j < PRE; ++j) pre[j] = j < nsplit ? po[(int64_t)j * D] : 0.f;
-  for (int idx = threadIdx.x; idx < G * nsplit; idx += blockDim.x) {
-    const int g2 = idx / nsplit, sp = idx % nsplit;
-    const float *ml = ws_ml + (s0 + (int64_t)g2 * nsplit + sp) * 2;
+  for (int j = 0; j < PRE; ++j) pre[j] = po[(int64_t)(j < slots ? j : 0) * D];
+  for (int idx = threadIdx.x; idx < G * slots; idx += blockDim.x) {
+    const int g2 = idx / slots, sp = idx % slots;
+    const float *ml = ws_ml + (s0 + (int64_t)g2 * slots + sp) * 2;
     s_w[g2][sp] = ml[0];
     s_l[g2][sp] = ml[1];
   }
+  // splits that had keys; with one, that split wrote the output itself
+  const int Lraw = seqlens ? seqlens[b] : fixed_len;
+  const int L = Lraw < p.Sk ? (Lraw > 0 ? Lraw : 0) : p.Sk;
+  const int nsplit = split_run(L, p.left, stride, slots, slots_inv).live();
   __syncthreads();
+  if (nsplit <= 1) return;
   const int nwave = blockDim.x / kWave;
   for (int g2 = w; g2 < G; g2 += nwave) { // one wave per query head
     float mx = -INFINITY;
@@ -1869,7 +1915,7 @@ static int launch_prefill(const AttnArgs &a, int64_t D, void *ws, size_t ws_byte
 }
 
 struct DecodePlan {
-  int chunk, nsplit, nw;
+  int nsplit, nw;
   bool inline_merge; // the last split block merges (no merge kernel)
   size_t o_bytes, ml_bytes, ws_bytes;
 };
@@ -1889,8 +1935,9 @@ static void use_merge_layout(DecodePlan &pl, size_t slots, int64_t D, bool inlin
   }
 }
 
-// Split-KV plan: about one 8-wave block per CU, each (batch, KV head) pair's
-// keys split into whole load batches; one split needs no merge kernel.
+// Split-KV plan: about one 8-wave block per CU; each sequence's load batches
+// are dealt evenly to the splits of its (batch, KV head) pair on the device
+// (split_run). One split needs no merge.
 static DecodePlan plan_decode(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax) {
   DecodePlan pl{};
   const int64_t kpw = kWave / (D / 8);
@@ -1905,7 +1952,6 @@ static DecodePlan plan_decode(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int
   chunk = ((chunk + batch - 1) / batch) * batch;
   if (chunk < batch) chunk = batch;
   while ((Lmax + chunk - 1) / chunk > kDecMaxSplit) chunk += batch;
-  pl.chunk = (int)chunk;
   pl.nsplit = (int)((Lmax + chunk - 1) / chunk);
   if (pl.nsplit < 1) pl.nsplit = 1;
   pl.inline_merge = pl.nsplit > 1 && pairs % 8 == 0 && pairs * (int64_t)sizeof(int) <= kDecOpCtrOffset &&
@@ -1934,19 +1980,20 @@ static void launch_decode_g(const AttnArgs &a, dim3 grid, const int *seqlens, in
   if constexpr (G <= 2) {
     if (pl.nw == kDecBigNW) {
       attn_decode_kernel<T, D, G, kDecBigNW><<<grid, dim3(64 * kDecBigNW), 0, st>>>(
-          a, seqlens, L, ws_o, ws_ml, pl.chunk, pl.nsplit, fz, counters, none);
+          a, seqlens, L, ws_o, ws_ml, pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters, none);
     } else {
       attn_decode_kernel<T, D, G, 4><<<grid, dim3(256), 0, st>>>(a, seqlens, L, ws_o, ws_ml,
-                                                                 pl.chunk, pl.nsplit, fz, counters,
+                                                                 pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters,
                                                                  none);
     }
   } else
     attn_decode_kernel<T, D, G, 4><<<grid, dim3(256), 0, st>>>(a, seqlens, L, ws_o, ws_ml,
-                                                               pl.chunk, pl.nsplit, fz, counters,
+                                                               pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters,
                                                                none);
   if (pl.nsplit > 1 && !counters)
     attn_decode_merge_kernel<T, D, G><<<dim3(a.Hkv, a.B), dim3(G * D), 0, st>>>(
-        a, ws_o, ws_ml, pl.nsplit);
+        a, seqlens, L, pl.nw * (kWave / (D / 8)) * kDecU, ws_o, ws_ml, pl.nsplit,
+        inv_of(pl.nsplit));
 }
 
 template <typename T, int D>
@@ -2207,8 +2254,8 @@ extern "C" int tpp_attn_decode_fused(const void *qkv, const void *q_norm_w, cons
 
 // ---- decode attention + output projection + residual add -------------------
 // The OP kernel's plan: one workgroup per CU (Hkv = 8 KV heads x B sequences
-// x 32 / B splits = 256), splits in whole 128-key load batches (trailing
-// splits may hold no key). Workspace: the counters region (the projection's
+// x 32 / B splits = 256), 128-key load batches dealt evenly to the splits by
+// the sequence's length (some may hold no key). Workspace: the counters region (the projection's
 // counters at kDecOpCtrOffset), the split partial slots, then the fp32
 // per-XCD partial projections [8][B][E].
 static bool oproj_shape(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t E) {
@@ -2217,17 +2264,13 @@ static bool oproj_shape(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t E
 }
 
 struct OprojPlan {
-  int nsplit, chunk;
+  int nsplit;
   size_t part_off, ws_bytes;
 };
 
-static OprojPlan plan_oproj(int64_t B, int64_t Hq, int64_t D, int64_t Lmax, int64_t E) {
+static OprojPlan plan_oproj(int64_t B, int64_t Hq, int64_t D, int64_t E) {
   OprojPlan pl{};
-  constexpr int64_t stride = kDecBigNW * (kWave / 16) * kDecU; // keys per block-wide batch (D 128)
   pl.nsplit = (int)(kOpPerXcd / B);
-  int64_t chunk = (Lmax + pl.nsplit - 1) / pl.nsplit;
-  chunk = (chunk + stride - 1) / stride * stride;
-  pl.chunk = (int)chunk;
   pl.part_off = (size_t)kDecCounterBytes + (size_t)(B * Hq * pl.nsplit) * (size_t)(D + 32) * sizeof(float);
   pl.ws_bytes = pl.part_off + (size_t)kOpXcds * B * E * sizeof(float);
   return pl;
@@ -2237,7 +2280,7 @@ extern "C" size_t tpp_attn_decode_oproj_workspace_size(int64_t B, int64_t Hq, in
                                                        int64_t D, int64_t Lmax, int64_t E) {
   const size_t plain = plan_decode(B, Hq, Hkv, D, Lmax).ws_bytes;
   if (!oproj_shape(B, Hq, Hkv, D, E) || Lmax < 1) return plain;
-  const size_t op = plan_oproj(B, Hq, D, Lmax, E).ws_bytes;
+  const size_t op = plan_oproj(B, Hq, D, E).ws_bytes;
   return op > plain ? op : plain;
 }
 
@@ -2290,7 +2333,7 @@ extern "C" int tpp_attn_decode_oproj(const void *qkv, const void *q_norm_w, cons
                          Hkv, D, softmax_scale, window_left < 0 ? -1 : window_left, 0);
   if (int rc = check_attn(name, a, D)) return rc;
   if (!strides16(a)) return set_error(TPP_E_INVALID, "%s: 16-byte alignment required", name);
-  const OprojPlan pl = plan_oproj(B, Hq, D, Lmax, E);
+  const OprojPlan pl = plan_oproj(B, Hq, D, E);
   DecodeFuse fz{qkv, q_norm_w, k_norm_w, cos, sin, cs_dtype, (int)ctx, eps};
   char *ws = (char *)workspace;
   DecodeOproj op{w_o, residual, (int *)(ws + kDecOpCtrOffset), (float *)(ws + pl.part_off), (int)E};
@@ -2299,10 +2342,10 @@ extern "C" int tpp_attn_decode_oproj(const void *qkv, const void *q_norm_w, cons
   return TPP_DISPATCH_HALF(dtype, [&] {
     if (Hq == 16)
       attn_decode_kernel<T, 128, 2, kDecBigNW, true><<<grid, block, 0, st>>>(
-          a, seqlens, (int)Lmax, ws_o, nullptr, pl.chunk, pl.nsplit, fz, (int *)ws, op);
+          a, seqlens, (int)Lmax, ws_o, nullptr, pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, (int *)ws, op);
     else
       attn_decode_kernel<T, 128, 1, kDecBigNW, true><<<grid, block, 0, st>>>(
-          a, seqlens, (int)Lmax, ws_o, nullptr, pl.chunk, pl.nsplit, fz, (int *)ws, op);
+          a, seqlens, (int)Lmax, ws_o, nullptr, pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, (int *)ws, op);
     return check_launch(name);
   });
 }
