@@ -124,3 +124,42 @@ def test_decode_lengths_far_below_the_capacity(dev, dtype, b, hq, hkv, d, cap, w
         want = oracle.decode_attention(q, k, v, lens.clamp(max=cap), window_left=window)
         close(o, want, what=f"decode lens {lens.tolist()} cap {cap} window {window}")
         o.fill_(float("nan"))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,hq,hkv,d,lens,cap,window", [
+    (1, 3, 1, 128, [1], 40, -1), (2, 4, 1, 128, [31, 33], 64, -1), (2, 10, 2, 64, [64, 65], 300, -1),
+    (3, 8, 1, 128, [0, 129, 500], 512, -1), (8, 32, 8, 128, [5, 700, 128, 1500, 2000, 2, 256, 999], 2000, -1),
+    (4, 24, 4, 64, [3000, 1, 257, 1024], 4000, -1), (8, 8, 1, 128, [900] * 8, 1000, 300),
+    (1, 28, 4, 64, [2100], 2100, 65), (4, 16, 8, 128, [1, 33, 640, 900], 1000, -1),
+    (1, 2, 1, 64, [4000], 4096, 50)])
+def test_decode_groups(dev, dtype, b, hq, hkv, d, lens, cap, window):
+    """Two to eight query heads per KV head (the matrix-core kernel): wave
+    and tile edges, empty sequences, windows, one split and several; rows past
+    each length hold NaN and must not be read."""
+    from torchplusplus_amd.attention import decode_attention
+    g = torch.Generator().manual_seed(hq + cap)
+    q = torch.randn(b, 1, hq, d, generator=g).to(dtype)
+    k, v = (torch.randn(b, hkv, cap, d, generator=g).to(dtype) for _ in range(2))
+    sl = torch.tensor(lens, dtype=torch.int32)
+    kd, vd = k.to(dev), v.to(dev)
+    for i, n in enumerate(lens):
+        if n:
+            kd[i, :, n:], vd[i, :, n:] = float("nan"), float("nan")
+    o = decode_attention(q.to(dev), kd, vd, sl.to(dev), window_left=window)
+    close(o, oracle.decode_attention(q, k, v, sl, window_left=window), what=f"group of {hq // hkv}, lens {lens}")
+
+
+def test_decode_group_keeps_infinities(dev):
+    """An infinite value in V makes its column infinite, not NaN, and no other."""
+    from torchplusplus_amd.attention import decode_attention
+    g = torch.Generator().manual_seed(3)
+    q = torch.randn(1, 1, 4, 128, generator=g).bfloat16()
+    k, v = (torch.randn(1, 1, 300, 128, generator=g).bfloat16() for _ in range(2))
+    v[0, 0, 50, 7], v[0, 0, 131, 100] = float("inf"), float("-inf")
+    sl = torch.tensor([290], dtype=torch.int32)
+    o = decode_attention(q.to(dev), k.to(dev), v.to(dev), sl.to(dev)).cpu()
+    want = oracle.decode_attention(q, k, v, sl)
+    assert torch.equal(torch.isinf(o), torch.isinf(want)) and not torch.isnan(o).any()
+    fin = torch.isfinite(want)
+    close(o[fin], want[fin], what="finite columns")

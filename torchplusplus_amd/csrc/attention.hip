@@ -1292,6 +1292,76 @@ __host__ __device__ inline SplitRun split_run(int L, int left, int stride, int n
   return r;
 }
 
+// In-kernel merge of a pair's splits, after this workgroup wrote its partial
+// slots (`live` of the `nsplit` slots of a head hold keys).
+template <typename T, int D>
+__device__ __forceinline__ void decode_merge_splits(const AttnArgs &p, int b, int hk, int G, int nsplit,
+                                                    int live, const float *__restrict__ ws_o,
+                                                    int *__restrict__ counters) {
+  // The last block of the pair to finish merges the splits. Every thread
+  // waits for its partial stores to reach L2 (an explicit vmcnt(0): the
+  // workgroup-scope fence of __syncthreads does not wait for global stores),
+  // then one thread counts the block in with an atomic in L2; the block that
+  // takes the count to `live` reads the other partials from the same L2.
+  // Each partial slot is whole 128-byte lines written by one block only, and
+  // a block reads other blocks' slots only here, so this CU's L1 (clean at
+  // kernel start) holds no stale copy of them.
+  __shared__ int s_last;
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+  __syncthreads();
+  const int pair = b * p.Hkv + hk;
+  if (threadIdx.x == 0) {
+    // agent scope: the counter is shared by workgroups (of one XCD); the
+    // atomic is performed in that XCD's L2 either way
+    const int old = __hip_atomic_fetch_add(&counters[pair], 1, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+    s_last = old == live - 1;
+    if (old == live - 1) // leave the counter at 0 for the next launch
+      __hip_atomic_store(&counters[pair], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int idx = threadIdx.x; idx < G * D; idx += blockDim.x) {
+    const int gi = idx / D, d = idx % D;
+    const float *sl = ws_o + (((int64_t)b * p.Hq + hk * G + gi) * nsplit) * (D + 32);
+    // the partials in groups of MG splits: a group's loads all go out before
+    // any is used (indices past nsplit read the last split and weigh 0), one
+    // L2 round trip per group instead of two per split; groups after the
+    // first rescale the running sums (online softmax)
+    constexpr int MG = 8;
+    float mu = -INFINITY, ls = 0.f, os = 0.f;
+    for (int s0 = 0; s0 < live; s0 += MG) {
+      float mv[MG], lv[MG], ov[MG];
+#pragma unroll
+      for (int j = 0; j < MG; ++j) {
+        const int sp = s0 + j < live ? s0 + j : live - 1;
+        const float *q = sl + (int64_t)sp * (D + 32);
+        mv[j] = q[D];
+        lv[j] = q[D + 1];
+        ov[j] = q[d];
+      }
+      float mx = mu;
+#pragma unroll
+      for (int j = 0; j < MG; ++j)
+        if (s0 + j < live) mx = fmaxf(mx, mv[j]);
+      const float mn = mx == -INFINITY ? 0.f : mx;
+      const float a = mu == -INFINITY ? 0.f : exp2f(mu - mn);
+      ls *= a;
+      os *= a;
+#pragma unroll
+      for (int j = 0; j < MG; ++j) {
+        const float wgt = s0 + j < live ? exp2f(mv[j] - mn) : 0.f;
+        ls += wgt * lv[j];
+        os += wgt * ov[j];
+      }
+      mu = mx;
+    }
+    T *op = (T *)p.o + (int64_t)b * p.o_sb + (int64_t)(hk * G + gi) * p.o_sh;
+    op[d] = from_f32<T>(ls > 0.f ? os / ls : 0.f);
+  }
+}
+
 template <typename T, int D, int G, int NW, bool OP = false>
 __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const int *__restrict__ seqlens,
                                                               int fixed_len, float *__restrict__ ws_o,
@@ -1646,68 +1716,308 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
     return;
   }
   if (!counters || live == 1) return;
-  // The last block of the pair to finish merges the splits. Every thread
-  // waits for its partial stores to reach L2 (an explicit vmcnt(0): the
-  // workgroup-scope fence of __syncthreads does not wait for global stores),
-  // then one thread counts the block in with an atomic in L2; the block that
-  // takes the count to `live` reads the other partials from the same L2.
-  // Each partial slot is whole 128-byte lines written by one block only, and
-  // a block reads other blocks' slots only here, so this CU's L1 (clean at
-  // kernel start) holds no stale copy of them.
-  __shared__ int s_last;
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
-  __syncthreads();
-  const int pair = b * p.Hkv + hk;
-  if (threadIdx.x == 0) {
-    // agent scope: the counter is shared by workgroups (of one XCD); the
-    // atomic is performed in that XCD's L2 either way
-    const int old = __hip_atomic_fetch_add(&counters[pair], 1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    s_last = old == live - 1;
-    if (old == live - 1) // leave the counter at 0 for the next launch
-      __hip_atomic_store(&counters[pair], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  decode_merge_splits<T, D>(p, b, hk, G, nsplit, live, ws_o, counters);
+}
+
+// ---------------------------------------------------------------------------
+// Decode with two or more query heads per KV head, on the matrix cores. The
+// VALU kernel above scores every head of the group against every key: at four
+// heads it is bound by that work (3.2 TB/s of the cache, at eight 1.2 TB/s).
+// Here the group's heads are the columns of S^T = K Q^T (32x32x16, at most 8
+// of 32 columns used: still several times the rate the cache arrives at) and
+// of O^T = V^T P^T. A block is 4 waves; each wave streams its own tiles of the
+// split's run (K and V by LDS-DMA into a private slot, no barrier in the
+// loop): the next K tile is requested as soon as this one's fragments are
+// read, the next V tile after this one's. The probabilities stay fp32-exact to
+// 2^-17: P = hi + lo in T, two products. Waves, then splits, are merged as in
+// the kernel above. Measured (bf16): 16 sequences of 2000 keys, 32 / 8 heads,
+// D 128, 41.1 -> 26.6 us; 64 sequences of 64-4000 keys, 8 / 1 heads, 57.6 ->
+// 22.2 us; 8 of 300-3000, 32 / 8 heads, D 64, 22.1 -> 12.1 us; two heads: 1
+// sequence of 900 keys, 16 / 8 heads, D 128, 9.1 -> 8.3 us, 32 of 100-4096
+// 55.3 -> 51.8 us, 8 of 2058 16.9 -> 17.0 us.
+// ---------------------------------------------------------------------------
+template <typename T, int D>
+__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const int *__restrict__ seqlens,
+                                                               int fixed_len, float *__restrict__ ws_o,
+                                                               float *__restrict__ ws_ml, int nsplit,
+                                                               unsigned nsplit_inv, unsigned hkv_inv,
+                                                               int *__restrict__ counters) {
+  typedef typename VecT<T>::v8 V8;
+  constexpr int KT = kSplitTile<D>, NB = KT / 32, NW = 4, STRIDE = NW * KT;
+  constexpr int CPR = D / 8, NT = D / 32, TU = KT * CPR;
+  constexpr int KPI = 64 / CPR, NDMA = KT / KPI;
+  constexpr int LDO = D + 4; // fp32 pitch of a wave's partial rows
+  __shared__ V8 smem[NW * 2 * TU];
+  __shared__ float s_m[NW][kDecMaxG], s_l[NW][kDecMaxG];
+  static_assert(kDecMaxG * LDO * 4 <= 2 * TU * 16, "a wave's partial rows fit its tile slot");
+
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, ql = lane & 31, G = p.Hq / p.Hkv;
+  int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  if (counters) { // splits of a pair on one XCD, as above
+    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const int group = div_inv(slot, nsplit_inv), pair = group * 8 + xcd;
+    split = slot - group * nsplit;
+    b = div_inv(pair, hkv_inv);
+    hk = pair - b * p.Hkv;
   }
-  __syncthreads();
-  if (!s_last) return;
-  for (int idx = threadIdx.x; idx < G * D; idx += blockDim.x) {
-    const int gi = idx / D, d = idx % D;
-    const float *sl = ws_o + (((int64_t)b * p.Hq + hk * G + gi) * nsplit) * (D + 32);
-    // the partials in groups of MG splits: a group's loads all go out before
-    // any is used (indices past nsplit read the last split and weigh 0), one
-    // L2 round trip per group instead of two per split; groups after the
-    // first rescale the running sums (online softmax)
-    constexpr int MG = 8;
-    float mu = -INFINITY, ls = 0.f, os = 0.f;
-    for (int s0 = 0; s0 < live; s0 += MG) {
-      float mv[MG], lv[MG], ov[MG];
+  const int Lraw = seqlens ? seqlens[b] : fixed_len;
+  const int L = Lraw < p.Sk ? (Lraw > 0 ? Lraw : 0) : p.Sk; // never read past the cache
+  const SplitRun run = split_run(L, p.left, STRIDE, nsplit, nsplit_inv);
+  const int64_t c0 = run.lead + (int64_t)split * run.batches * STRIDE;
+  if (split > 0 && c0 >= L) return;
+  const int k_begin = (int)(c0 > run.lo ? (c0 < L ? c0 : L) : run.lo);
+  const int k_end = (int)(c0 + (int64_t)run.batches * STRIDE < L ? c0 + (int64_t)run.batches * STRIDE : L);
+
+  // LDS-DMA of this wave's tiles: keys past the run read its last one (finite,
+  // masked)
+  const char *ks = (const char *)((const T *)p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh);
+  const char *vs = (const char *)((const T *)p.v + (int64_t)b * p.v_sb + (int64_t)hk * p.v_sh);
+  const int dkey = lane / CPR, dslot = lane % CPR;
+  V8 *const ring = smem + w * (2 * TU);
+  auto issue = [&](bool kt, int base) {
+    const char *src = kt ? ks : vs;
+    const int64_t ss = kt ? p.k_ss : p.v_ss;
 #pragma unroll
-      for (int j = 0; j < MG; ++j) {
-        const int sp = s0 + j < live ? s0 + j : live - 1;
-        const float *q = sl + (int64_t)sp * (D + 32);
-        mv[j] = q[D];
-        lv[j] = q[D + 1];
-        ov[j] = q[d];
-      }
-      float mx = mu;
-#pragma unroll
-      for (int j = 0; j < MG; ++j)
-        if (s0 + j < live) mx = fmaxf(mx, mv[j]);
-      const float mn = mx == -INFINITY ? 0.f : mx;
-      const float a = mu == -INFINITY ? 0.f : exp2f(mu - mn);
-      ls *= a;
-      os *= a;
-#pragma unroll
-      for (int j = 0; j < MG; ++j) {
-        const float wgt = s0 + j < live ? exp2f(mv[j] - mn) : 0.f;
-        ls += wgt * lv[j];
-        os += wgt * ov[j];
-      }
-      mu = mx;
+    for (int j = 0; j < NDMA; ++j) {
+      const int key = j * KPI + dkey;
+      const int ch = kt ? dslot ^ (key & (CPR - 1)) : dslot ^ vswz<D>(key);
+      __builtin_amdgcn_global_load_lds(
+          (const void *)(src + ((int64_t)min(base + key, k_end - 1) * ss + ch * 8) * (int64_t)sizeof(T)),
+          (__attribute__((address_space(3))) void *)(ring + (kt ? 0 : TU) + j * 64), 16, 0, kCpolNT);
     }
-    T *op = (T *)p.o + (int64_t)b * p.o_sb + (int64_t)(hk * G + gi) * p.o_sh;
-    op[d] = from_f32<T>(ls > 0.f ? os / ls : 0.f);
+  };
+  const int first = (int)(c0 < L ? c0 : L) + w * KT;
+  const int n = first < k_end ? (k_end - first + STRIDE - 1) / STRIDE : 0; // this wave's tiles
+  if (n > 0) {
+    issue(true, first);
+    issue(false, first);
   }
+  // query heads of the group as columns (columns past G repeat the last head)
+  const T *qp = (const T *)p.q + (int64_t)b * p.q_sb + (int64_t)(hk * G + min(ql, G - 1)) * p.q_sh;
+  V8 qf[D / 16];
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) qf[i] = *reinterpret_cast<const V8 *>(qp + i * 16 + h * 8);
+  // waited for here (with the first tiles): no wait for them inside the loop
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) asm volatile("" ::"v"(qf[i]));
+
+  f32x16 o[NT];
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[tt][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  const float c2 = p.scale_log2;
+  const unsigned base0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char *)ring;
+  const int grp = lane >> 4, a4 = lane & 3, c4 = (lane >> 2) & 3, kl = 4 * (grp >> 1) + c4;
+  unsigned vo[NT];
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    const int d0 = tt * 32 + 16 * (grp & 1) + 4 * a4;
+    vo[tt] = base0 + TU * 16 + kl * D * 2 + (((d0 >> 3) ^ vswz<D>(kl)) << 4) + ((d0 & 7) << 1);
+  }
+  for (int i = 0; i < n; ++i) {
+    const int kb = first + i * STRIDE;
+    const bool more = i + 1 < n;
+    vm_wait<NDMA>(); // this tile's K landed (its V may be in flight)
+    constexpr int KS = D / 16, NS = KS * NB / 2;
+    f32x16 s[NB];
+#pragma unroll
+    for (int st = 0; st < NB; ++st)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[st][r] = 0.f;
+    V8 kr[3][2];
+    auto kfrag = [&](auto ii) {
+      constexpr int x = decltype(ii)::value;
+      static_for<2>([&](auto jj) {
+        constexpr int j = decltype(jj)::value, k = NB == 2 ? x : 2 * x + j;
+        const unsigned a = base0 + (unsigned)((ql * CPR + ((k * 2 + h) ^ (ql & (CPR - 1)))) * 16);
+        kr[x % 3][j] = lds_read_b128<(NB == 2 ? j : 0) * 32 * D * 2, V8>(a);
+      });
+    };
+    kfrag(std::integral_constant<int, 0>{});
+    kfrag(std::integral_constant<int, 1>{});
+    static_for<NS>([&](auto ii) {
+      constexpr int x = decltype(ii)::value;
+      if constexpr (x + 2 < NS) kfrag(std::integral_constant<int, x + 2>{});
+      lds_wait_tied<(x + 2 < NS ? 2 : NS - 1 - x) * 2>(kr[x % 3]);
+      // every K fragment is in registers: the next K tile may land
+      if constexpr (x == NS - 1) {
+        asm volatile("" ::: "memory");
+        if (more) issue(true, kb + STRIDE);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        s[j % NB] = mfma32x32<T>(kr[x % 3][j], qf[NB == 2 ? x : 2 * x + j], s[j % NB]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if (kb < k_begin || kb + KT > k_end) {
+      const int jb = kb + h * 4;
+      const int ca = max(k_begin - jb, 0), cb = min(k_end - 1 - jb, KT - 1);
+      const unsigned ninf = __float_as_uint(-INFINITY);
+#pragma unroll
+      for (int st = 0; st < NB; ++st) {
+        const int l0 = max(ca - 32 * st, 0), h0 = min(cb - 32 * st, 31);
+        const unsigned keep = l0 <= h0 ? ((2u << h0) - 1u) & ~((1u << l0) - 1u) : 0u;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const unsigned bm = (unsigned)__builtin_amdgcn_sbfe((int)keep, (r >> 2) * 8 + (r & 3), 1);
+          s[st][r] = __uint_as_float((__float_as_uint(s[st][r]) & bm) | (ninf & ~bm));
+        }
+      }
+    }
+    float mx[4] = {s[0][0], s[0][1], s[0][2], s[0][3]};
+#pragma unroll
+    for (int st = 0; st < NB; ++st)
+#pragma unroll
+      for (int r = st == 0 ? 4 : 0; r < 16; ++r) mx[r & 3] = fmaxf(mx[r & 3], s[st][r]);
+    float mt = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+    mt = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    const bool move = mt > m_run;
+    const float m_new = move ? mt : m_run;
+    const float mc = m_new == -INFINITY ? 0.f : m_new * c2;
+    const float alpha = move ? __builtin_amdgcn_exp2f(m_run * c2 - mc) : 1.f;
+    float ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < NB; ++st)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[st][r], c2, -mc));
+        s[st][r] = e;
+        ps[r & 3] += e;
+      }
+    l_run = l_run * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+    m_run = m_new;
+    if (__any(move)) {
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[tt][r] *= alpha;
+    }
+    V8 ph[2 * NB], pl[2 * NB];
+#pragma unroll
+    for (int c = 0; c < 2 * NB; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float e = s[c >> 1][(c & 1) * 8 + j];
+        ph[c][j] = from_f32<T>(e);
+        pl[c][j] = from_f32<T>(e - to_f32(ph[c][j]));
+      }
+    // this tile's V landed (the next K may be in flight)
+    if (more) vm_wait<NDMA>();
+    else vm_wait<0>();
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    constexpr int R = 2 * NT;
+    s16x4 vr[2][R];
+    auto vfrag = [&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        vr[c % 2][2 * tt] = lds_read_tr16<c * 32 * D>(vo[tt]);
+        vr[c % 2][2 * tt + 1] = lds_read_tr16<c * 32 * D + 16 * D>(vo[tt]);
+      }
+    };
+    vfrag(std::integral_constant<int, 0>{});
+    static_for<2 * NB>([&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+      if constexpr (c + 1 < 2 * NB) vfrag(std::integral_constant<int, c + 1>{});
+      lds_wait_tied<(c + 1 < 2 * NB ? R : 0)>(vr[c % 2]);
+      if constexpr (c + 1 == 2 * NB) {
+        asm volatile("" ::: "memory");
+        if (more) issue(false, kb + STRIDE);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int tt = 0; tt < NT; ++tt) {
+        const s16x8 r12 = __builtin_shufflevector(vr[c % 2][2 * tt], vr[c % 2][2 * tt + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+        const V8 va = __builtin_bit_cast(V8, r12);
+        o[tt] = mfma32x32<T>(va, ph[c], o[tt]);
+        o[tt] = mfma32x32<T>(va, pl[c], o[tt]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+
+  // this wave's rows (its tile slot is drained), then the block's
+  const float l = l_run + __shfl_xor(l_run, 32, kWave);
+  float *const part = reinterpret_cast<float *>(ring);
+  if (ql < G) {
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = o[tt][rg * 4 + e];
+        *reinterpret_cast<f32x4 *>(part + ql * LDO + tt * 32 + rg * 8 + h * 4) = v;
+      }
+    if (h == 0) s_m[w][ql] = m_run == -INFINITY ? m_run : m_run * c2, s_l[w][ql] = l;
+  }
+  // An infinity in V: its products with the two halves of P (which may be zero
+  // or of opposite sign) sum to NaN where P times V is infinite. A wave with a
+  // non-finite sum therefore redoes its sums with one product per key.
+  bool odd = false;
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) odd |= !(fabsf(o[tt][r]) < INFINITY);
+  if (__any(odd)) {
+    for (int gi = 0; gi < G; ++gi) {
+      const T *qr = (const T *)p.q + (int64_t)b * p.q_sb + (int64_t)(hk * G + gi) * p.q_sh;
+      const float mg = __shfl(m_run, gi, kWave), mc = mg == -INFINITY ? 0.f : mg * c2;
+      float acc[D / 64];
+#pragma unroll
+      for (int c = 0; c < D / 64; ++c) acc[c] = 0.f;
+      for (int i = 0; i < n; ++i)
+        for (int key = max(first + i * STRIDE, k_begin); key < min(first + i * STRIDE + KT, k_end); ++key) {
+          const T *kr = (const T *)ks + (int64_t)key * p.k_ss, *vr = (const T *)vs + (int64_t)key * p.v_ss;
+          float sd = 0.f;
+#pragma unroll
+          for (int c = 0; c < D / 64; ++c) sd += to_f32(qr[c * 64 + lane]) * to_f32(kr[c * 64 + lane]);
+          const float e = __builtin_amdgcn_exp2f(fmaf(wave_sum(sd), c2, -mc));
+#pragma unroll
+          for (int c = 0; c < D / 64; ++c) acc[c] += e * to_f32(vr[c * 64 + lane]);
+        }
+#pragma unroll
+      for (int c = 0; c < D / 64; ++c) part[gi * LDO + c * 64 + lane] = acc[c];
+    }
+  }
+  __syncthreads();
+  const int live = run.live();
+  for (int idx = tid; idx < G * D; idx += 64 * NW) {
+    const int gi = idx / D, d = idx % D;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) mx = fmaxf(mx, s_m[ww][gi]);
+    const float mu = mx == -INFINITY ? 0.f : mx;
+    float ls = 0.f, os = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) {
+      const float c = exp2f(s_m[ww][gi] - mu);
+      ls += s_l[ww][gi] * c;
+      os += reinterpret_cast<const float *>(smem + ww * (2 * TU))[gi * LDO + d] * c;
+    }
+    const int hq = hk * G + gi;
+    if (live == 1) {
+      T *op = (T *)p.o + (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh;
+      op[d] = from_f32<T>(ls > 0.f ? os / ls : 0.f);
+      continue;
+    }
+    const int64_t slot = ((int64_t)b * p.Hq + hq) * nsplit + split;
+    if (counters) {
+      float *sl = ws_o + slot * (D + 32);
+      sl[d] = os;
+      if (d == 0) sl[D] = mx, sl[D + 1] = ls;
+    } else {
+      ws_o[slot * D + d] = os;
+      if (d == 0) ws_ml[slot * 2] = mx, ws_ml[slot * 2 + 1] = ls;
+    }
+  }
+  if (!counters || live == 1) return;
+  decode_merge_splits<T, D>(p, b, hk, G, nsplit, live, ws_o, counters);
 }
 
 // Merge the split partials of one (batch, KV head): grid (Hkv, B), 256
@@ -1977,22 +2287,23 @@ static void launch_decode_g(const AttnArgs &a, dim3 grid, const int *seqlens, in
                             float *ws_ml, int *counters, const DecodePlan &pl, const DecodeFuse &fz,
                             hipStream_t st) {
   const DecodeOproj none{};
-  if constexpr (G <= 2) {
-    if (pl.nw == kDecBigNW) {
-      attn_decode_kernel<T, D, G, kDecBigNW><<<grid, dim3(64 * kDecBigNW), 0, st>>>(
-          a, seqlens, L, ws_o, ws_ml, pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters, none);
-    } else {
-      attn_decode_kernel<T, D, G, 4><<<grid, dim3(256), 0, st>>>(a, seqlens, L, ws_o, ws_ml,
-                                                                 pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters,
-                                                                 none);
-    }
-  } else
-    attn_decode_kernel<T, D, G, 4><<<grid, dim3(256), 0, st>>>(a, seqlens, L, ws_o, ws_ml,
-                                                               pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters,
-                                                               none);
+  // The matrix-core kernel from two heads per KV head on; one head leaves its
+  // products too little to do (64 sequences of 64-4000 keys, 8 / 8 heads, 88
+  // us by the VALU kernel, 100 us by it). The fused prologue is the VALU
+  // kernel's only.
+  const bool mfma = G >= 2 && !fz.qkv;
+  if (mfma) {
+    attn_decode_mfma_kernel<T, D><<<grid, dim3(256), 0, st>>>(a, seqlens, L, ws_o, ws_ml, pl.nsplit,
+                                                              inv_of(pl.nsplit), inv_of(a.Hkv), counters);
+  } else {
+    constexpr int NW = G <= 2 ? kDecBigNW : 4; // as plan_decode
+    attn_decode_kernel<T, D, G, NW><<<grid, dim3(64 * NW), 0, st>>>(
+        a, seqlens, L, ws_o, ws_ml, pl.nsplit, inv_of(pl.nsplit), inv_of(a.Hkv), fz, counters, none);
+  }
   if (pl.nsplit > 1 && !counters)
     attn_decode_merge_kernel<T, D, G><<<dim3(a.Hkv, a.B), dim3(G * D), 0, st>>>(
-        a, seqlens, L, pl.nw * (kWave / (D / 8)) * kDecU, ws_o, ws_ml, pl.nsplit,
+        a, seqlens, L, mfma ? 4 * kSplitTile<D> : pl.nw * (kWave / (D / 8)) * kDecU, ws_o,
+        ws_ml, pl.nsplit,
         inv_of(pl.nsplit));
 }
 

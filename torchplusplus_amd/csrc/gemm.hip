@@ -869,6 +869,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_ksplit_kernel(
       lds_wait_tied<(3 - ks) * (FM + FN)>(f[ks]);
       if constexpr (ks == 3) {
         // every fragment is in registers: refill the slot
+        asm volatile("" ::: "memory");
         if (i + NST < n) issue(c + NST * NW, slot);
       }
       if (tail) {
