@@ -141,6 +141,14 @@ int tpp_qkv_rope_cache(const void *qkv, void *q_out, void *k_cache,
                        int64_t Lmax, float eps, int dtype, int cs_dtype,
                        void *stream);
 
+/* tpp_qkv_rope_cache with one first position for every sequence, passed by
+ * value (no positions array to fill). */
+int tpp_qkv_rope_cache_at(const void *qkv, void *q_out, void *k_cache, void *v_cache,
+                          const void *q_norm_w, const void *k_norm_w, const void *cos,
+                          const void *sin, int64_t ctx, int64_t start, int64_t B, int64_t S,
+                          int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax, float eps, int dtype,
+                          int cs_dtype, void *stream);
+
 /* Per-head RMSNorm over D (q_norm_w / k_norm_w [D], NULL = none) and RoPE of
  * q [B, S, Hq, D] and k [B, S, Hk, D] in place, in one launch: token t's heads
  * are contiguous at q + t * q_stride and k + t * k_stride; cos/sin [S, D] row s
@@ -367,6 +375,17 @@ int tpp_attn_decode_fused(const void *qkv, const void *q_norm_w,
                           int64_t Lmax, float softmax_scale, int window_left,
                           int dtype, void *workspace, size_t ws_bytes,
                           void *stream);
+
+/* tpp_attn_decode_fused with every sequence's new token at one position,
+ * passed by value (seqlens[b] = position + 1). */
+int tpp_attn_decode_fused_at(const void *qkv, const void *q_norm_w, const void *k_norm_w,
+                             const void *cos, const void *sin, int64_t ctx, int cs_dtype,
+                             float eps, void *k_cache, void *v_cache, void *o,
+                             const int64_t *k_strides, const int64_t *v_strides,
+                             const int64_t *o_strides, int64_t position, int64_t B, int64_t Hq,
+                             int64_t Hkv, int64_t D, int64_t Lmax, float softmax_scale,
+                             int window_left, int dtype, void *workspace, size_t ws_bytes,
+                             void *stream);
 
 /* Workspace bytes of tpp_attn_decode_oproj (256-byte aligned, zero-filled
  * before first use; counters in it are left at zero by every call; it may be

@@ -19,7 +19,6 @@ import torch
 import torch.nn as nn
 
 from torchplusplus_amd._native import ext as _ext
-from torchplusplus_amd.attention.flash import flash_attn_func
 from torchplusplus_amd.dlops.derived import DerivedWeight, attach
 from torchplusplus_amd.dlops.linear import linear
 from torchplusplus_amd.llmops.kvcache import KVCache
@@ -130,34 +129,21 @@ class GroupedQueryAttention(nn.Module):
                cache_pos: Optional[int] = None) -> torch.Tensor:
         """Steps 2-3: rope/cache the projected qkv and attend; returns the
         attention output [B, S, Hq*D] (before the output projection)."""
+        qn, kn = self.q_norm, self.k_norm
+        eps = qn.eps if qn is not None and qn.eps is not None else 1e-6
+        shape = (self.num_heads, self.n_kv_heads, self.head_dim)
+        norms = (None if qn is None else qn.weight, None if kn is None else kn.weight)
+        if kv_cache is None:
+            return _C.gqa_attend(qkv, *norms, eps, cos, sin, None, None, 0, *shape)
         bs, seq_len = qkv.shape[0], qkv.shape[1]
-        dev = qkv.device
-        if kv_cache is not None:
-            start = kv_cache.cache_len if cache_pos is None else int(cache_pos)
-            kv_cache.ensure(bs, start + seq_len)
-            total = start + seq_len
-            # the cache may hold more sequences than this call (allocated for
-            # an earlier, larger batch): the kernels get this batch's rows
-            kc_b, vc_b = kv_cache.k_cache[:bs], kv_cache.v_cache[:bs]
-            if seq_len == 1:
-                # one new token: QK-norm + RoPE + cache append fused into the
-                # split-KV decode kernel
-                seqlens = _positions(bs, total, dev)
-                kv_cache.cache_len = max(kv_cache.cache_len, total)
-                return self.decode_fused(qkv, cos, sin, kc_b, vc_b,
-                                         seqlens).reshape(bs, seq_len, self.d_out)
-            positions = _positions(bs, start, dev)
-            q = self.rope_cache(qkv, cos, sin, kc_b, vc_b, positions)
-            kv_cache.cache_len = max(kv_cache.cache_len, start + seq_len)
-            o = flash_attn_func(q, kc_b[:, :, :total].transpose(1, 2),
-                                vc_b[:, :, :total].transpose(1, 2), causal=True)
-        else:
-            k = torch.empty(bs, self.n_kv_heads, seq_len, self.head_dim, dtype=qkv.dtype, device=dev)
-            v = torch.empty_like(k)
-            positions = _positions(bs, 0, dev)
-            q = self.rope_cache(qkv, cos, sin, k, v, positions)
-            o = flash_attn_func(q, k.transpose(1, 2), v.transpose(1, 2), causal=True)
-        return o.reshape(bs, seq_len, self.d_out)
+        start = kv_cache.cache_len if cache_pos is None else int(cache_pos)
+        kv_cache.ensure(bs, start + seq_len)
+        # (the cache may hold more sequences than this call: the kernels get
+        # this batch's rows)
+        o = _C.gqa_attend(qkv, *norms, eps, cos, sin, kv_cache.k_cache, kv_cache.v_cache, start,
+                          *shape)
+        kv_cache.cache_len = max(kv_cache.cache_len, start + seq_len)
+        return o
 
     def forward(self, x, cos, sin, kv_cache: Optional[KVCache] = None,
                 cache_pos: Optional[int] = None):

@@ -9,9 +9,12 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from torchplusplus_amd._native import ext as _ext
 from torchplusplus_amd.attention._common import norm_rope_qk
 from torchplusplus_amd.attention.flash import flash_attn_func
 from torchplusplus_amd.dlops.linear import linear
+
+_C = _ext()
 
 
 class MultiHeadAttention(nn.Module):
@@ -38,9 +41,8 @@ class MultiHeadAttention(nn.Module):
 
     def forward(self, x: torch.Tensor, cos, sin):
         bsz, seq, _ = x.shape
-        q = self._heads(linear(x, self.Wq.weight), bsz, seq)
-        k = self._heads(linear(x, self.Wk.weight), bsz, seq)
-        v = self._heads(linear(x, self.Wv.weight), bsz, seq)
+        q, k, v = (self._heads(t, bsz, seq) for t in
+                   _C.linear3(x, self.Wq.weight, self.Wk.weight, self.Wv.weight))
         q, k = norm_rope_qk(q, k, self.q_norm, self.k_norm, cos, sin)
         o = flash_attn_func(q, k, v, causal=True).reshape(bsz, seq, self.embed_dim)
         return linear(o, self.out_projection.weight, self.out_projection.bias)

@@ -7,9 +7,12 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from torchplusplus_amd._native import ext as _ext
 from torchplusplus_amd.attention._common import norm_rope_qk
 from torchplusplus_amd.attention.flash import flash_attn_func
 from torchplusplus_amd.dlops.linear import linear
+
+_C = _ext()
 
 
 class MultiQueryAttention(nn.Module):
@@ -30,9 +33,9 @@ class MultiQueryAttention(nn.Module):
 
     def forward(self, x, cos, sin):
         bsz, seq, _ = x.shape
-        q = linear(x, self.Wq.weight).view(bsz, seq, self.num_q_head, self.head_dim)
-        k = linear(x, self.Wk.weight).view(bsz, seq, 1, self.head_dim)
-        v = linear(x, self.Wv.weight).view(bsz, seq, 1, self.head_dim)
+        q, k, v = _C.linear3(x, self.Wq.weight, self.Wk.weight, self.Wv.weight)
+        q = q.view(bsz, seq, self.num_q_head, self.head_dim)
+        k, v = k.view(bsz, seq, 1, self.head_dim), v.view(bsz, seq, 1, self.head_dim)
         norms = (self.q_norm, self.k_norm) if self.qk_norm else (None, None)
         q, k = norm_rope_qk(q, k, *norms, cos, sin)
         o = flash_attn_func(q, k, v, causal=True)

@@ -2407,7 +2407,7 @@ extern "C" size_t tpp_attn_decode_workspace_size(int64_t B, int64_t Hq, int64_t 
 
 static int decode_impl(const char *name, AttnArgs &a, int64_t D, int64_t Lmax,
                        const int32_t *seqlens, const DecodeFuse &fz, int dtype, void *workspace,
-                       size_t ws_bytes, void *stream, bool may_probe = true) {
+                       size_t ws_bytes, void *stream, bool may_probe = true, int64_t len = -1) {
   if (int e = check_attn(name, a, D)) return e;
   if (a.B == 0) return TPP_OK;
   // the kernel reads cache row 0 even for empty sequences (clamped loads)
@@ -2432,7 +2432,7 @@ static int decode_impl(const char *name, AttnArgs &a, int64_t D, int64_t Lmax,
                         ? dim3((unsigned)(pl.nsplit * a.Hkv * a.B))
                         : dim3((unsigned)pl.nsplit, (unsigned)a.Hkv, (unsigned)a.B);
   return TPP_DISPATCH_HALF(dtype, [&] {
-    launch_decode<T>(a, D, a.Hq / a.Hkv, grid, seqlens, (int)Lmax, ws_o, ws_ml, counters, pl, fz,
+    launch_decode<T>(a, D, a.Hq / a.Hkv, grid, seqlens, (int)(len < 0 ? Lmax : len), ws_o, ws_ml, counters, pl, fz,
                      st);
     return check_launch(name);
   });
@@ -2532,18 +2532,16 @@ extern "C" int tpp_attn_decode_noalloc(const void *q, const void *k_cache, const
                      false);
 }
 
-extern "C" int tpp_attn_decode_fused(const void *qkv, const void *q_norm_w, const void *k_norm_w,
-                                     const void *cos, const void *sin, int64_t ctx, int cs_dtype,
-                                     float eps, void *k_cache, void *v_cache, void *o,
-                                     const int64_t *k_strides, const int64_t *v_strides,
-                                     const int64_t *o_strides, const int32_t *seqlens, int64_t B,
-                                     int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax,
-                                     float softmax_scale, int window_left, int dtype,
-                                     void *workspace, size_t ws_bytes, void *stream) {
-  const char *name = "tpp_attn_decode_fused";
+static int decode_fused(const char *name, const void *qkv, const void *q_norm_w, const void *k_norm_w,
+                        const void *cos, const void *sin, int64_t ctx, int cs_dtype, float eps,
+                        void *k_cache, void *v_cache, void *o, const int64_t *k_strides,
+                        const int64_t *v_strides, const int64_t *o_strides, const int32_t *seqlens,
+                        int64_t len, int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax,
+                        float softmax_scale, int window_left, int dtype, void *workspace,
+                        size_t ws_bytes, void *stream) {
   if (!k_strides || !v_strides || !o_strides)
     return set_error(TPP_E_INVALID, "%s: null stride array", name);
-  if (!qkv || !cos || !sin || !seqlens)
+  if (!qkv || !cos || !sin || (!seqlens && len < 0))
     return set_error(TPP_E_INVALID, "%s: qkv, cos, sin and seqlens are required", name);
   if (!aligned16(qkv) || !aligned16(cos) || !aligned16(sin) ||
       (q_norm_w && !aligned16(q_norm_w)) || (k_norm_w && !aligned16(k_norm_w)))
@@ -2560,7 +2558,36 @@ extern "C" int tpp_attn_decode_fused(const void *qkv, const void *q_norm_w, cons
   AttnArgs a = make_args(qkv, k_cache, v_cache, o, qs, k_strides, v_strides, o_strides, B, 1,
                          Lmax, Hq, Hkv, D, softmax_scale, window_left < 0 ? -1 : window_left, 0);
   DecodeFuse fz{qkv, q_norm_w, k_norm_w, cos, sin, cs_dtype, (int)ctx, eps};
-  return decode_impl(name, a, D, Lmax, seqlens, fz, dtype, workspace, ws_bytes, stream);
+  return decode_impl(name, a, D, Lmax, seqlens, fz, dtype, workspace, ws_bytes, stream, true, len);
+}
+
+extern "C" int tpp_attn_decode_fused(const void *qkv, const void *q_norm_w, const void *k_norm_w,
+                                     const void *cos, const void *sin, int64_t ctx, int cs_dtype,
+                                     float eps, void *k_cache, void *v_cache, void *o,
+                                     const int64_t *k_strides, const int64_t *v_strides,
+                                     const int64_t *o_strides, const int32_t *seqlens, int64_t B,
+                                     int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax,
+                                     float softmax_scale, int window_left, int dtype,
+                                     void *workspace, size_t ws_bytes, void *stream) {
+  return decode_fused("tpp_attn_decode_fused", qkv, q_norm_w, k_norm_w, cos, sin, ctx, cs_dtype, eps,
+                      k_cache, v_cache, o, k_strides, v_strides, o_strides, seqlens, -1, B, Hq, Hkv, D,
+                      Lmax, softmax_scale, window_left, dtype, workspace, ws_bytes, stream);
+}
+
+extern "C" int tpp_attn_decode_fused_at(const void *qkv, const void *q_norm_w, const void *k_norm_w,
+                                        const void *cos, const void *sin, int64_t ctx, int cs_dtype,
+                                        float eps, void *k_cache, void *v_cache, void *o,
+                                        const int64_t *k_strides, const int64_t *v_strides,
+                                        const int64_t *o_strides, int64_t position, int64_t B,
+                                        int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax,
+                                        float softmax_scale, int window_left, int dtype,
+                                        void *workspace, size_t ws_bytes, void *stream) {
+  const char *name = "tpp_attn_decode_fused_at";
+  if (position < 0 || position >= Lmax)
+    return set_error(TPP_E_INVALID, "%s: position %lld outside the cache", name, (long long)position);
+  return decode_fused(name, qkv, q_norm_w, k_norm_w, cos, sin, ctx, cs_dtype, eps, k_cache, v_cache, o,
+                      k_strides, v_strides, o_strides, nullptr, position + 1, B, Hq, Hkv, D, Lmax,
+                      softmax_scale, window_left, dtype, workspace, ws_bytes, stream);
 }
 
 // ---- decode attention + output projection + residual add -------------------

@@ -16,6 +16,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <limits>
+#include <string>
 #include <vector>
 
 #include "include/tpp.h"
@@ -230,9 +231,12 @@ std::vector<at::Tensor> qkrope_apply_cuda(at::Tensor q, at::Tensor k, at::Tensor
   return {qo, ko};
 }
 
-void qkv_rope_cache(at::Tensor qkv, at::Tensor q_out, at::Tensor k_cache, at::Tensor v_cache,
-                    c10::optional<at::Tensor> q_norm_w, c10::optional<at::Tensor> k_norm_w,
-                    at::Tensor cos, at::Tensor sin, at::Tensor positions, double eps) {
+// positions: int32 [B] on the device, or undefined for `start` everywhere
+void qkv_rope_cache_from(const at::Tensor &qkv, const at::Tensor &q_out, const at::Tensor &k_cache,
+                         const at::Tensor &v_cache, const c10::optional<at::Tensor> &q_norm_w,
+                         const c10::optional<at::Tensor> &k_norm_w, const at::Tensor &cos,
+                         const at::Tensor &sin, const at::Tensor &positions, int64_t start,
+                         double eps) {
   TORCH_CHECK(qkv.is_cuda() && qkv.is_contiguous() && is_half_or_bf16(qkv),
               "qkv must be a contiguous CUDA half/bfloat16 tensor [B, S, (Hq+2Hkv)*D]");
   TORCH_CHECK(q_out.dim() == 4 && q_out.is_contiguous() &&
@@ -243,8 +247,8 @@ void qkv_rope_cache(at::Tensor qkv, at::Tensor q_out, at::Tensor k_cache, at::Te
                   k_cache.scalar_type() == qkv.scalar_type() &&
                   v_cache.scalar_type() == qkv.scalar_type(),
               "caches must be contiguous [B, Hkv, Lmax, D] of the qkv dtype");
-  TORCH_CHECK(positions.is_cuda() && positions.scalar_type() == at::kInt &&
-                  positions.numel() == q_out.size(0),
+  TORCH_CHECK(!positions.defined() || (positions.is_cuda() && positions.scalar_type() == at::kInt &&
+                                       positions.numel() == q_out.size(0)),
               "positions must be a CUDA int32 tensor of length B");
   const int64_t B = q_out.size(0), S = q_out.size(1), Hq = q_out.size(2), D = q_out.size(3);
   const int64_t Hkv = k_cache.size(1), Lmax = k_cache.size(2);
@@ -270,12 +274,24 @@ void qkv_rope_cache(at::Tensor qkv, at::Tensor q_out, at::Tensor k_cache, at::Te
     kw = k_norm_w->data_ptr();
   }
   c10::DeviceGuard g(qkv.device());
-  check_rc(tpp_qkv_rope_cache(qkv.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(),
-                              v_cache.data_ptr(), qw, kw, cos.data_ptr(), sin.data_ptr(),
-                              cos.size(0), positions.data_ptr<int32_t>(), B, S, Hq, Hkv, D,
-                              Lmax, (float)eps, dtype_code(qkv), dtype_code(cos),
-                              cur_stream(qkv)),
+  const auto dt = dtype_code(qkv), cdt = dtype_code(cos);
+  check_rc(positions.defined()
+               ? tpp_qkv_rope_cache(qkv.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(),
+                                    v_cache.data_ptr(), qw, kw, cos.data_ptr(), sin.data_ptr(),
+                                    cos.size(0), positions.data_ptr<int32_t>(), B, S, Hq, Hkv, D,
+                                    Lmax, (float)eps, dt, cdt, cur_stream(qkv))
+               : tpp_qkv_rope_cache_at(qkv.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(),
+                                       v_cache.data_ptr(), qw, kw, cos.data_ptr(), sin.data_ptr(),
+                                       cos.size(0), start, B, S, Hq, Hkv, D, Lmax, (float)eps, dt, cdt,
+                                       cur_stream(qkv)),
            "qkv_rope_cache");
+}
+
+void qkv_rope_cache(at::Tensor qkv, at::Tensor q_out, at::Tensor k_cache, at::Tensor v_cache,
+                    c10::optional<at::Tensor> q_norm_w, c10::optional<at::Tensor> k_norm_w,
+                    at::Tensor cos, at::Tensor sin, at::Tensor positions, double eps) {
+  TORCH_CHECK(positions.defined(), "positions must be a CUDA int32 tensor of length B");
+  qkv_rope_cache_from(qkv, q_out, k_cache, v_cache, q_norm_w, k_norm_w, cos, sin, positions, 0, eps);
 }
 
 // per-head RMSNorm (optional) + RoPE, in place on q [B, S, Hq, D] and k
@@ -401,6 +417,37 @@ at::Tensor gemv(at::Tensor input, at::Tensor weight, c10::optional<at::Tensor> b
   return out;
 }
 
+// act(x W^T + b): the decode GEMV for up to 16 rows, the GEMM otherwise
+at::Tensor linear_any(at::Tensor input, at::Tensor weight, c10::optional<at::Tensor> bias,
+                      int64_t act) {
+  TORCH_CHECK(input.dim() >= 1 && input.size(-1) > 0, "Input must be at least 1D and not empty");
+  if (input.numel() / input.size(-1) <= 16) return gemv(input, weight, bias, act);
+  return linear_act(input, weight, bias, act);
+}
+
+// projections of one input, in one call
+std::vector<at::Tensor> linear3(at::Tensor input, at::Tensor w0, at::Tensor w1, at::Tensor w2) {
+  const c10::optional<at::Tensor> none;
+  return {linear_any(input, w0, none, TPP_ACT_NONE), linear_any(input, w1, none, TPP_ACT_NONE),
+          linear_any(input, w2, none, TPP_ACT_NONE)};
+}
+
+// What a derived weight is keyed on: each source's storage address, version
+// counter (-1 for inference tensors, which have none), dtype, device and shape
+py::bytes source_key(const std::vector<at::Tensor> &sources) {
+  std::string key;
+  auto add = [&](int64_t v) { key.append(reinterpret_cast<const char *>(&v), sizeof(v)); };
+  for (const at::Tensor &t : sources) {
+    add((int64_t)reinterpret_cast<uintptr_t>(t.data_ptr()));
+    add(t.is_inference() ? -1 : (int64_t)t._version());
+    add((int64_t)t.scalar_type());
+    add(((int64_t)t.device().type() << 32) | (uint32_t)t.device().index());
+    add(t.dim());
+    for (int64_t d : t.sizes()) add(d);
+  }
+  return py::bytes(key);
+}
+
 const void *norm_ptr(const c10::optional<at::Tensor> &nw, const at::Tensor &input, int64_t K) {
   if (!nw.has_value() || !nw->defined()) return nullptr;
   TORCH_CHECK(nw->is_cuda() && nw->scalar_type() == input.scalar_type() &&
@@ -447,6 +494,16 @@ at::Tensor gemv_swiglu(at::Tensor input, at::Tensor w_gu, c10::optional<at::Tens
                           nullptr, B, N, K, 1, dtype_code(input), cur_stream(input)),
            "gemv_swiglu");
   return out;
+}
+
+// SwiGLU from the interleaved weight, and the whole feed-forward block
+at::Tensor swiglu_any(at::Tensor input, at::Tensor w_gu) {
+  TORCH_CHECK(input.dim() >= 1 && input.size(-1) > 0, "Input must be at least 1D and not empty");
+  if (input.numel() / input.size(-1) <= 16) return gemv_swiglu(input, w_gu, c10::nullopt, 1e-6);
+  return linear_swiglu(input, w_gu);
+}
+at::Tensor ffn_forward(at::Tensor input, at::Tensor w_gu, at::Tensor w_down) {
+  return linear_any(swiglu_any(input, w_gu), w_down, c10::nullopt, TPP_ACT_NONE);
 }
 
 // greedy lm_head: returns (token ids [B] int64, logits or None)
@@ -739,10 +796,12 @@ at::Tensor argmax_rows(at::Tensor x) {
 }
 
 // decode attention with the new token's QK-norm + RoPE + cache append fused in
-at::Tensor attn_decode_fused(at::Tensor qkv, c10::optional<at::Tensor> q_norm_w,
-                             c10::optional<at::Tensor> k_norm_w, at::Tensor cos, at::Tensor sin,
-                             double eps, at::Tensor k_cache, at::Tensor v_cache,
-                             at::Tensor seqlens, double softmax_scale, int64_t window_left) {
+// (seqlens undefined: every sequence's new token at `position`)
+at::Tensor decode_fused_from(const at::Tensor &qkv, const c10::optional<at::Tensor> &q_norm_w,
+                             const c10::optional<at::Tensor> &k_norm_w, const at::Tensor &cos,
+                             const at::Tensor &sin, double eps, const at::Tensor &k_cache,
+                             const at::Tensor &v_cache, const at::Tensor &seqlens, int64_t position,
+                             double softmax_scale, int64_t window_left) {
   TORCH_CHECK(qkv.is_cuda() && qkv.is_contiguous() && is_half_or_bf16(qkv),
               "qkv must be a contiguous CUDA half/bfloat16 tensor [B, 1, (Hq+2Hkv)*D]");
   TORCH_CHECK(k_cache.is_cuda() && v_cache.is_cuda() && k_cache.dim() == 4 &&
@@ -755,8 +814,8 @@ at::Tensor attn_decode_fused(at::Tensor qkv, c10::optional<at::Tensor> q_norm_w,
   TORCH_CHECK(qkv.numel() % (B * D) == 0, "qkv size mismatch");
   const int64_t Hq = qkv.numel() / (B * D) - 2 * Hkv;
   TORCH_CHECK(Hq > 0 && Hq % Hkv == 0, "qkv size does not give a valid head count");
-  TORCH_CHECK(seqlens.is_cuda() && seqlens.scalar_type() == at::kInt && seqlens.numel() == B &&
-                  seqlens.is_contiguous(),
+  TORCH_CHECK(!seqlens.defined() || (seqlens.is_cuda() && seqlens.scalar_type() == at::kInt &&
+                                     seqlens.numel() == B && seqlens.is_contiguous()),
               "seqlens must be a contiguous CUDA int32 tensor [B]");
   TORCH_CHECK(cos.is_contiguous() && sin.is_contiguous() && cos.dim() == 2 && cos.size(1) == D &&
                   sin.sizes() == cos.sizes() && sin.scalar_type() == cos.scalar_type() &&
@@ -772,14 +831,66 @@ at::Tensor attn_decode_fused(at::Tensor qkv, c10::optional<at::Tensor> q_norm_w,
   const int64_t ks[3] = {k_cache.stride(0), k_cache.stride(2), k_cache.stride(1)};
   const int64_t vs[3] = {v_cache.stride(0), v_cache.stride(2), v_cache.stride(1)};
   const int64_t os[3] = {o.stride(0), o.stride(1), o.stride(2)};
-  check_rc(tpp_attn_decode_fused(qkv.data_ptr(), qw, kw, cos.data_ptr(), sin.data_ptr(),
-                                 cos.size(0), dtype_code(cos), (float)eps, k_cache.data_ptr(),
-                                 v_cache.data_ptr(), o.data_ptr(), ks, vs, os,
-                                 seqlens.data_ptr<int32_t>(), B, Hq, Hkv, D, Lmax,
-                                 (float)softmax_scale, (int)window_left, dtype_code(qkv),
-                                 ws.data_ptr(), (size_t)ws.numel() * 4, cur_stream(qkv)),
+  const size_t have = (size_t)ws.numel() * 4;
+  check_rc(seqlens.defined()
+               ? tpp_attn_decode_fused(qkv.data_ptr(), qw, kw, cos.data_ptr(), sin.data_ptr(),
+                                       cos.size(0), dtype_code(cos), (float)eps, k_cache.data_ptr(),
+                                       v_cache.data_ptr(), o.data_ptr(), ks, vs, os,
+                                       seqlens.data_ptr<int32_t>(), B, Hq, Hkv, D, Lmax,
+                                       (float)softmax_scale, (int)window_left, dtype_code(qkv),
+                                       ws.data_ptr(), have, cur_stream(qkv))
+               : tpp_attn_decode_fused_at(qkv.data_ptr(), qw, kw, cos.data_ptr(), sin.data_ptr(),
+                                          cos.size(0), dtype_code(cos), (float)eps, k_cache.data_ptr(),
+                                          v_cache.data_ptr(), o.data_ptr(), ks, vs, os, position, B,
+                                          Hq, Hkv, D, Lmax, (float)softmax_scale, (int)window_left,
+                                          dtype_code(qkv), ws.data_ptr(), have, cur_stream(qkv)),
            "attn_decode_fused");
   return o;
+}
+
+at::Tensor attn_decode_fused(at::Tensor qkv, c10::optional<at::Tensor> q_norm_w,
+                             c10::optional<at::Tensor> k_norm_w, at::Tensor cos, at::Tensor sin,
+                             double eps, at::Tensor k_cache, at::Tensor v_cache,
+                             at::Tensor seqlens, double softmax_scale, int64_t window_left) {
+  TORCH_CHECK(seqlens.defined(), "seqlens must be a contiguous CUDA int32 tensor [B]");
+  return decode_fused_from(qkv, q_norm_w, k_norm_w, cos, sin, eps, k_cache, v_cache, seqlens, 0,
+                           softmax_scale, window_left);
+}
+
+// The attention of a grouped-query layer on its projection qkv [B, S,
+// (Hq + 2 Hkv) * D]: per-head norm and rotation at positions start .. start +
+// S - 1, K/V into the caches [>= B, Hkv, Lmax, D] (without caches, into
+// scratch rows), causal attention over start + S keys; [B, S, Hq * D].
+at::Tensor gqa_attend(at::Tensor qkv, c10::optional<at::Tensor> q_norm_w,
+                      c10::optional<at::Tensor> k_norm_w, double eps, at::Tensor cos, at::Tensor sin,
+                      c10::optional<at::Tensor> k_cache, c10::optional<at::Tensor> v_cache,
+                      int64_t start, int64_t Hq, int64_t Hkv, int64_t D) {
+  TORCH_CHECK(qkv.is_cuda() && qkv.dim() == 3 && qkv.size(2) == (Hq + 2 * Hkv) * D,
+              "qkv must be a CUDA tensor [B, S, (Hq+2Hkv)*D]");
+  const int64_t B = qkv.size(0), S = qkv.size(1);
+  const bool cached = k_cache.has_value() && k_cache->defined();
+  c10::DeviceGuard g(qkv.device());
+  at::Tensor k, v;
+  if (cached) {
+    TORCH_CHECK(v_cache.has_value() && k_cache->dim() == 4 && v_cache->dim() == 4 &&
+                    k_cache->size(0) >= B && k_cache->sizes() == v_cache->sizes() &&
+                    k_cache->size(1) == Hkv && k_cache->size(3) == D && start >= 0 &&
+                    start + S <= k_cache->size(2),
+                "caches must be [>= B, Hkv, >= start + S, D]");
+    k = k_cache->size(0) == B ? *k_cache : k_cache->narrow(0, 0, B);
+    v = v_cache->size(0) == B ? *v_cache : v_cache->narrow(0, 0, B);
+    if (S == 1)
+      return decode_fused_from(qkv, q_norm_w, k_norm_w, cos, sin, eps, k, v, at::Tensor(), start, 0.0, -1)
+          .view({B, S, Hq * D});
+  } else {
+    k = torch::empty({B, Hkv, S, D}, qkv.options());
+    v = torch::empty_like(k);
+    start = 0;
+  }
+  auto q = torch::empty({B, S, Hq, D}, qkv.options());
+  qkv_rope_cache_from(qkv, q, k, v, q_norm_w, k_norm_w, cos, sin, at::Tensor(), start, eps);
+  if (start + S < k.size(2)) k = k.narrow(2, 0, start + S), v = v.narrow(2, 0, start + S);
+  return attn_fwd(q, k.transpose(1, 2), v.transpose(1, 2), true, -1, -1, 0.0).view({B, S, Hq * D});
 }
 
 // decode attention with the fused prologue, then the output projection and
@@ -923,6 +1034,21 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("input"), py::arg("weight"), py::arg("bias") = py::none(), py::arg("act") = 0);
   m.def("linear_swiglu", &linear_swiglu, "silu(x Wg^T) * (x Wu^T) from interleaved w_gu",
         py::arg("input"), py::arg("w_gu"));
+  m.def("linear_any", &linear_any, "act(x @ W^T + b): GEMV for <= 16 rows, GEMM otherwise",
+        py::arg("input"), py::arg("weight"), py::arg("bias") = py::none(), py::arg("act") = 0);
+  m.def("linear3", &linear3, "three bias-free projections of one input", py::arg("input"),
+        py::arg("w0"), py::arg("w1"), py::arg("w2"));
+  m.def("swiglu_any", &swiglu_any, "silu(x Wg^T) * (x Wu^T): GEMV for <= 16 rows, GEMM otherwise",
+        py::arg("input"), py::arg("w_gu"));
+  m.def("ffn_forward", &ffn_forward, "swiglu_any, then the down projection", py::arg("input"),
+        py::arg("w_gu"), py::arg("w_down"));
+  m.def("source_key", &source_key, "identity and version of a derived weight's sources",
+        py::arg("sources"));
+  m.def("gqa_attend", &gqa_attend,
+        "QK-norm + RoPE + cache append + causal attention of a projected qkv, one first position",
+        py::arg("qkv"), py::arg("q_norm_w"), py::arg("k_norm_w"), py::arg("eps"), py::arg("cos"),
+        py::arg("sin"), py::arg("k_cache"), py::arg("v_cache"), py::arg("start"), py::arg("n_heads"),
+        py::arg("n_kv_heads"), py::arg("head_dim"));
   m.def("gemv", &gemv, "decode GEMV for <= 16 rows", py::arg("input"), py::arg("weight"),
         py::arg("bias") = py::none(), py::arg("act") = 0);
   m.def("gemv_swiglu", &gemv_swiglu, "decode SwiGLU GEMV for <= 16 rows", py::arg("input"),

@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(
     const T *__restrict__ qkv, T *__restrict__ q_out, T *__restrict__ k_cache,
     T *__restrict__ v_cache, const T *__restrict__ qw, const T *__restrict__ kw,
     const CS *__restrict__ cos, const CS *__restrict__ sin,
-    const int *__restrict__ pos, int B, int S, int Hq, int Hkv, int Lmax, float eps,
+    const int *__restrict__ pos, int start, int B, int S, int Hq, int Hkv, int Lmax, float eps,
     int ctx) {
   constexpr int D = LPR * 16;
   const int H = Hq + 2 * Hkv;
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(
   for (int j = 0; j < 8; ++j) ss += x1[j] * x1[j] + x2[j] * x2[j];
   ss = group_sum<LPR>(ss);
   if (!valid) return;
-  const int p = pos[b] + s;
+  const int p = (pos ? pos[b] : start) + s;
   if (is_q || is_k) {
     const T *nw = is_q ? qw : kw;
     if (nw) {
@@ -281,7 +281,8 @@ struct QkvArgs {
   const void *qkv;
   void *q_out, *k_cache, *v_cache;
   const void *qw, *kw, *cos, *sin;
-  const int32_t *pos;
+  const int32_t *pos; // NULL: every sequence begins at `start`
+  int start;
   int B, S, Hq, Hkv, Lmax;
   float eps;
   int ctx, lpr;
@@ -293,7 +294,7 @@ template <typename T, typename CS, int LPR>
 static void launch_qkv_lpr(const QkvArgs &a) {
   qkv_rope_cache_kernel<T, CS, LPR><<<dim3(a.blocks), dim3(256), 0, a.st>>>(
       (const T *)a.qkv, (T *)a.q_out, (T *)a.k_cache, (T *)a.v_cache, (const T *)a.qw,
-      (const T *)a.kw, (const CS *)a.cos, (const CS *)a.sin, a.pos, a.B, a.S, a.Hq, a.Hkv,
+      (const T *)a.kw, (const CS *)a.cos, (const CS *)a.sin, a.pos, a.start, a.B, a.S, a.Hq, a.Hkv,
       a.Lmax, a.eps, a.ctx);
 }
 
@@ -331,15 +332,13 @@ extern "C" int tpp_rope_qk(const void *q, const void *k, void *q_out, void *k_ou
                        cs_dtype, stream, name);
 }
 
-extern "C" int tpp_qkv_rope_cache(const void *qkv, void *q_out, void *k_cache,
-                                  void *v_cache, const void *q_norm_w,
-                                  const void *k_norm_w, const void *cos, const void *sin,
-                                  int64_t ctx, const int32_t *positions, int64_t B,
-                                  int64_t S, int64_t Hq, int64_t Hkv, int64_t D,
-                                  int64_t Lmax, float eps, int dtype, int cs_dtype,
-                                  void *stream) {
-  const char *name = "tpp_qkv_rope_cache";
-  if (!qkv || !q_out || !k_cache || !v_cache || !cos || !sin || !positions)
+static int qkv_rope_cache(const char *name, const void *qkv, void *q_out, void *k_cache,
+                          void *v_cache, const void *q_norm_w, const void *k_norm_w,
+                          const void *cos, const void *sin, int64_t ctx,
+                          const int32_t *positions, int64_t start, int64_t B, int64_t S,
+                          int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax, float eps, int dtype,
+                          int cs_dtype, void *stream) {
+  if (!qkv || !q_out || !k_cache || !v_cache || !cos || !sin)
     return set_error(TPP_E_INVALID, "%s: null pointer argument", name);
   if (B <= 0 || S <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Lmax <= 0 || ctx <= 0)
     return set_error(TPP_E_INVALID, "%s: invalid shapes", name);
@@ -359,7 +358,7 @@ extern "C" int tpp_qkv_rope_cache(const void *qkv, void *q_out, void *k_cache,
   const int lpr = (int)(D / 16);
   const int64_t blocks = (rows * lpr + 255) / 256;
   if (blocks > 0x7fffffffLL) return set_error(TPP_E_UNSUPPORTED, "%s: too large", name);
-  QkvArgs a{qkv, q_out, k_cache, v_cache, q_norm_w, k_norm_w, cos, sin, positions,
+  QkvArgs a{qkv, q_out, k_cache, v_cache, q_norm_w, k_norm_w, cos, sin, positions, (int)start,
             (int)B, (int)S, (int)Hq, (int)Hkv, (int)Lmax, eps, (int)ctx, lpr,
             (unsigned)blocks, as_stream(stream)};
   return TPP_DISPATCH_HALF(dtype, [&] {
@@ -367,6 +366,31 @@ extern "C" int tpp_qkv_rope_cache(const void *qkv, void *q_out, void *k_cache,
     if (cs_dtype == TPP_F16) return launch_qkv<T, f16>(a, name);
     return launch_qkv<T, bf16>(a, name);
   });
+}
+
+extern "C" int tpp_qkv_rope_cache(const void *qkv, void *q_out, void *k_cache,
+                                  void *v_cache, const void *q_norm_w,
+                                  const void *k_norm_w, const void *cos, const void *sin,
+                                  int64_t ctx, const int32_t *positions, int64_t B,
+                                  int64_t S, int64_t Hq, int64_t Hkv, int64_t D,
+                                  int64_t Lmax, float eps, int dtype, int cs_dtype,
+                                  void *stream) {
+  const char *name = "tpp_qkv_rope_cache";
+  if (!positions) return set_error(TPP_E_INVALID, "%s: null pointer argument", name);
+  return qkv_rope_cache(name, qkv, q_out, k_cache, v_cache, q_norm_w, k_norm_w, cos, sin, ctx, positions,
+                        0, B, S, Hq, Hkv, D, Lmax, eps, dtype, cs_dtype, stream);
+}
+
+extern "C" int tpp_qkv_rope_cache_at(const void *qkv, void *q_out, void *k_cache, void *v_cache,
+                                     const void *q_norm_w, const void *k_norm_w, const void *cos,
+                                     const void *sin, int64_t ctx, int64_t start, int64_t B,
+                                     int64_t S, int64_t Hq, int64_t Hkv, int64_t D, int64_t Lmax,
+                                     float eps, int dtype, int cs_dtype, void *stream) {
+  const char *name = "tpp_qkv_rope_cache_at";
+  if (start < 0 || start > 0x7fffffff - S)
+    return set_error(TPP_E_INVALID, "%s: first position %lld", name, (long long)start);
+  return qkv_rope_cache(name, qkv, q_out, k_cache, v_cache, q_norm_w, k_norm_w, cos, sin, ctx, nullptr,
+                        start, B, S, Hq, Hkv, D, Lmax, eps, dtype, cs_dtype, stream);
 }
 
 extern "C" int tpp_qk_norm_rope(void *q, int64_t q_stride, void *k, int64_t k_stride,

@@ -22,16 +22,9 @@ from typing import Callable, Optional
 
 import torch
 
+from torchplusplus_amd._native import ext as _ext
 
-def _version(t: torch.Tensor) -> Optional[int]:
-    try:
-        return t._version
-    except RuntimeError:  # inference tensors have no version counter
-        return None
-
-
-def _key(t: torch.Tensor):
-    return (t.data_ptr(), _version(t), t.dtype, tuple(t.shape), t.device)
+_C = _ext()
 
 
 class DerivedWeight:
@@ -44,7 +37,7 @@ class DerivedWeight:
         self._key = None
 
     def get(self, *sources: torch.Tensor) -> torch.Tensor:
-        key = tuple(_key(t) for t in sources)
+        key = _C.source_key(sources)
         if key == self._key and self._buf is not None:
             return self._buf
         capturing = sources[0].is_cuda and torch.cuda.is_current_stream_capturing()

@@ -21,19 +21,13 @@ GEMV_MAX_ROWS = 16
 def linear(x: torch.Tensor, weight: torch.Tensor, bias=None, act: int = ACT_NONE) -> torch.Tensor:
     """act(x @ weight^T + bias) on the gfx950 kernels: the split-K GEMV for
     decode-sized inputs (<= 16 rows), the MFMA GEMM otherwise."""
-    rows = x.numel() // x.shape[-1]
-    if rows <= GEMV_MAX_ROWS:
-        return _C.gemv(x, weight, bias, act)
-    return _C.linear(x, weight, bias, act)
+    return _C.linear_any(x, weight, bias, act)
 
 
 def swiglu(x: torch.Tensor, w_gu: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) from a [gate|up] weight interleaved in blocks
     of 32 rows (see interleave_gate_up)."""
-    rows = x.numel() // x.shape[-1]
-    if rows <= GEMV_MAX_ROWS:
-        return _C.gemv_swiglu(x, w_gu)
-    return _C.linear_swiglu(x, w_gu)
+    return _C.swiglu_any(x, w_gu)
 
 
 def interleave_gate_up(w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:

@@ -34,7 +34,7 @@ from torchplusplus_amd._native import ext as _ext
 from torchplusplus_amd.attention.gqa import GroupedQueryAttention
 from torchplusplus_amd.dlops.derived import DerivedWeight, attach
 from torchplusplus_amd.dlops.linear import (GEMV_MAX_ROWS, LinearSILU, interleave_gate_up,
-                                             linear, swiglu)
+                                             linear)
 from torchplusplus_amd.dlops.normalization import RmsNormFused
 from torchplusplus_amd.dlops.rope import compute_rope_params
 from torchplusplus_amd.llmops.kvcache import KVCache
@@ -102,7 +102,7 @@ class FFN(nn.Module):
         return self._w_gu.get(self.fused_linear_layer1.weight, self.linear_layerP.weight)
 
     def forward(self, x):
-        return linear(swiglu(x, self.w_gu()), self.linear_layer2.weight)
+        return _C.ffn_forward(x, self.w_gu(), self.linear_layer2.weight)
 
 
 class Transformer(nn.Module):
