@@ -103,3 +103,29 @@ def test_gemm_fragment_reads_waited_for(tmp_path):
                    check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL, timeout=600)
     loads, bad = scan(open(out).read())
     assert loads > 0 and not bad, "\n".join(bad[:10])
+
+
+# (m, n, k, act, bias): 256x256 tiles over whole rounds and 128x128 tiles over
+# the remaining rows (one row block and several, ragged M and N, one K step and
+# more, one round and two)
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,act,bias", [(6227, 3072, 128, "gelu", True), (4100, 4000, 64, "relu", True),
+                                            (5633, 3072, 64, "none", True), (9990, 3076, 192, "silu", False)])
+def test_linear_mixed_tiles(dev, m, n, k, act, bias):
+    from torchplusplus_amd._native import ext
+    dtype = torch.float16 if m % 2 else torch.bfloat16
+    x, w, b = _mk(m, n, k, dtype, seed=m)
+    b = b if bias else None
+    y = ext().linear(x.to(dev), w.to(dev), None if b is None else b.to(dev), ACTS[act])
+    close(y, oracle.linear_act(x, w, b, act), what=f"mixed {act} {m}x{n}x{k}")
+
+
+@pytest.mark.gpu
+def test_swiglu_mixed_tiles(dev):
+    from torchplusplus_amd._native import ext
+    from torchplusplus_amd.dlops.linear import interleave_gate_up
+    x, wg, _ = _mk(2900, 3072, 512, torch.bfloat16, seed=3)
+    _, wu, _ = _mk(1, 3072, 512, torch.bfloat16, seed=4)
+    y = ext().linear_swiglu(x.to(dev), interleave_gate_up(wg, wu).to(dev))
+    g = oracle.linear_act(x, wg, None, "silu").float()
+    close(y, (g * oracle.linear_act(x, wu, None, "none").float()).to(x.dtype), what="mixed swiglu")

@@ -38,14 +38,9 @@ constexpr int kBM = 128, kBN = 128, kBK = 64;
 // would put rows r and r+8 on the same banks: a 2-way conflict on every read).
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 
-// K-tile depth and ring stages of the 256x256 tile (64 KB per stage at BK 64;
-// 4- and 5-stage rings of BK 32 tiles measured slower)
-#ifndef TPP_BIG_BK
-#define TPP_BIG_BK 64
-#define TPP_BIG_NST 2
-#endif
-constexpr int kBigBK = TPP_BIG_BK, kBigNST = TPP_BIG_NST;
-// the same for the 128-row tiles: BK 64, as many stages as fit 160 KB of LDS
+// The 256x256 tile takes BK 64 in 2 ring stages (64 KB each; 4- and 5-stage
+// rings of BK 32 tiles measured slower), the 128-row tiles BK 64 in as many
+// stages as fit 160 KB of LDS
 // (one block per CU): 5 for 128x128, 4 for 128x192, 3 for 128x256 (at the
 // Linear+act shape 3 stages were 6% faster than 2, and 4 another 3%)
 constexpr int kSmallBK = 64;
@@ -248,10 +243,21 @@ template <typename T> __device__ __forceinline__ void round_pairs(float (&x)[4])
   }
 }
 
+// 16-byte LDS units of a tile: the ring, or the epilogue's staging tile that
+// reuses it
+template <typename T, int EPI, int FM, int FN, int NST, int WM, int WN, int BK> constexpr int dma_tile_lds() {
+  const int ring = NST * (32 * WM * FM + 32 * WN * FN) * (BK / 8);
+  const int ows = EPI == kGSwiGLU ? FN * 16 : FN * 32;
+  const int outs = WM * WN * FM * 32 * (ows + 8) * (int)sizeof(T) / 16;
+  return ring > outs ? ring : outs;
+}
+
+// Output tile `pid` of the rows from `mb` on; `smem` holds dma_tile_lds units.
 template <typename T, int EPI, int ACT, int FM, int FN, int NST, int WM, int WN, int BK>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(
-    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
-    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
+__device__ __forceinline__ void gemm_dma_tile(
+    typename VecT<T>::v8 *smem, const T *__restrict__ A, int64_t lda, const T *__restrict__ B,
+    int64_t ldb, T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K,
+    int pid, int mb) {
   typedef typename VecT<T>::v8 V8;
   constexpr int BM = 32 * WM * FM, BN = 32 * WN * FN, NWV = WM * WN;
   constexpr int CPR = BK / 8;                // 16-byte chunks per tile row
@@ -259,15 +265,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(
   constexpr int STG = (BM + BN) * CPR;       // 16-byte slots per stage
   constexpr int NA = BM / RPI / NWV, NB = BN / RPI / NWV; // DMA instructions per wave per stage
   static_assert(NA * RPI * NWV == BM && NB * RPI * NWV == BN, "tile rows per wave");
-  // the epilogue's staging tile reuses the ring
-  constexpr int OWS = (EPI == kGSwiGLU) ? FN * 16 : FN * 32;
-  constexpr int RING = NST * STG, OUTS = NWV * FM * 32 * (OWS + 8) * (int)sizeof(T) / 16;
-  __shared__ V8 smem[RING > OUTS ? RING : OUTS];
-
-  const int ntm = (M + BM - 1) / BM, ntn = (N + BN - 1) / BN;
+  const int ntm = (M - mb + BM - 1) / BM, ntn = (N + BN - 1) / BN;
   int tm, tn;
-  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  tile_coords(pid, ntm * ntn, ntm, ntn, tm, tn);
+  const int m0 = mb + tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w / WN, wn = w % WN;
 
@@ -497,6 +498,36 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(
         if (col + e < NO) dst[e] = v[e];
     }
   }
+}
+
+template <typename T, int EPI, int ACT, int FM, int FN, int NST, int WM, int WN, int BK>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(
+    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
+    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
+  __shared__ typename VecT<T>::v8 smem[dma_tile_lds<T, EPI, FM, FN, NST, WM, WN, BK>()];
+  gemm_dma_tile<T, EPI, ACT, FM, FN, NST, WM, WN, BK>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K,
+                                                       blockIdx.x, 0);
+}
+
+// Two tile sizes in one launch: 256x256 tiles over the first Mb rows, as many
+// as fill the CUs in whole rounds, and 128x128 tiles over the rest. 256x256
+// tiles are the fastest per output, but 300 of them on 256 CUs take two rounds
+// for 1.17 rounds of work, and smaller tiles everywhere lose their operand
+// reuse: 6227 x 3072 x 1024 + bias + GeLU (bf16) 66.4 us with 256x256 tiles,
+// 74.0 with 128x128, 52.4 mixed; 3000 x 6144 x 1024 SwiGLU 54.0 -> 43.8 us;
+// 6227 x 5632 x 2048 + bias + GeLU 177 -> 146 us.
+template <typename T, int EPI, int ACT>
+__global__ __launch_bounds__(512) void gemm_mixed_kernel(
+    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
+    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K, int Mb) {
+  constexpr int LB = dma_tile_lds<T, EPI, 2, 4, 2, 4, 2, 64>(), LS = dma_tile_lds<T, EPI, 1, 2, 4, 4, 2, 64>();
+  __shared__ typename VecT<T>::v8 smem[LB > LS ? LB : LS];
+  const int nbig = Mb / 256 * ((N + 255) / 256);
+  if ((int)blockIdx.x < nbig)
+    gemm_dma_tile<T, EPI, ACT, 2, 4, 2, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, Mb, N, K, blockIdx.x, 0);
+  else
+    gemm_dma_tile<T, EPI, ACT, 1, 2, 4, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K,
+                                                   blockIdx.x - nbig, Mb);
 }
 
 // ---------------------------------------------------------------------------
@@ -959,26 +990,46 @@ __global__ __launch_bounds__(64 * NW) void gemm_ksplit_kernel(
   }
 }
 
-// Tile shape for the DMA kernel: minimise (tiles per CU, rounded up) x tile
-// area / relative efficiency (one block per CU for every candidate). SwiGLU
-// needs whole [gate|up] 64-column pairs per wave (FN even).
-static int pick_dma_tile(int64_t M, int64_t N, bool swiglu, int cus) {
-  struct Cand { int bm, bn, fn_wave; double eff; };
-  // 128x128 / 128x192 / 128x256: 8 waves (4x2) of 32x64 / 32x96 / 32x128, so
-  // two waves share each SIMD even at one block per CU (measured 7% faster
-  // than 4 waves of 64-row strips at the BASELINE Linear+act shape);
-  // 256x256: 8 waves (4x2) of 64x128
-  const Cand cands[] = {{128, 128, 2, 0.95}, {128, 192, 3, 1.0}, {128, 256, 4, 1.0},
-                        {256, 256, 4, 1.25}};
-  int best = -1;
-  double best_t = 0.0;
-  for (int c = 0; c < 4; ++c) {
-    if (swiglu && (cands[c].fn_wave & 1)) continue;
-    const int64_t bm = cands[c].bm, bn = cands[c].bn;
-    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    const int64_t per_cu = (tiles + cus - 1) / cus;
-    const double t = (double)per_cu * (double)(bm * bn) / cands[c].eff;
-    if (best < 0 || t < best_t) best = c, best_t = t;
+// Tiles of an output of kDmaMinMN elements and more: the cheapest plan by the
+// time of its rounds (tiles / CUs), in us from fits of each kernel over M 700 -
+// 16384, N 1024 - 11264, K 768 - 3072 (bf16; 6-10% rms, the rounds themselves
+// make steps of up to 2x): a round costs `full` or, not filled, `part` per 1024
+// of K plus `round`, the launch `base`. The mixed plan fills whole rounds with
+// 256x256 tiles and tiles the remaining rows by 128x128. Over 75 shapes the
+// plan chosen is within 1% of the fastest on average (at most 6%) and 9%
+// faster than the choice by tile area alone (up to 1.5x).
+enum BigTile { kTile128x128, kTile128x192, kTile128x256, kTile256x256, kTileMixed };
+struct BigPlan {
+  BigTile tile;
+  int64_t big_rows; // rows of the 256x256 part (mixed)
+};
+static BigPlan pick_dma_tile(int64_t M, int64_t N, int64_t K, bool swiglu, bool persist, int cus) {
+  struct Cand { BigTile id; int bm, bn; double base, full, part, round; };
+  const Cand cands[] = {{kTile128x128, 128, 128, 1.0, 8.7, 8.7, 3.5},
+                        {kTile128x192, 128, 192, 0.0, 11.0, 12.0, 6.0},
+                        {kTile128x256, 128, 256, 1.0, 15.0, 14.0, 5.5},
+                        {kTile256x256, 256, 256, 1.5, 25.0, 21.0, 7.5}};
+  const double k = (double)K / 1024.0;
+  BigPlan best{kTile128x128, 0};
+  double best_t = -1.0;
+  auto tiles_of = [](int64_t rows, int64_t cols, int bm, int bn) {
+    return ((rows + bm - 1) / bm) * ((cols + bn - 1) / bn);
+  };
+  for (const Cand &c : cands) {
+    if (swiglu && c.id == kTile128x192) continue; // whole [gate | up] 64-column pairs per wave
+    const int64_t tiles = tiles_of(M, N, c.bm, c.bn), full = tiles / cus, part = tiles % cus ? 1 : 0;
+    const bool loop = c.id == kTile256x256 && persist && tiles > cus; // the persistent kernel
+    const double t = (loop ? 3.0 : c.base) + (double)full * (c.full * k + (loop ? 3.5 : c.round)) +
+                     (double)part * (c.part * k + (loop ? 3.5 : c.round));
+    if (best_t < 0 || t < best_t) best = {c.id, 0}, best_t = t;
+  }
+  const int64_t ntn = (N + 255) / 256;
+  for (int64_t r = 1; r * cus <= tiles_of(M, N, 256, 256) && r <= 64; ++r) {
+    const int64_t rows = r * cus / ntn * 256; // row blocks that fit r rounds
+    if (rows < 256 || rows >= M) continue;
+    const int64_t small = (tiles_of(M - rows, N, 128, 128) + cus - 1) / cus;
+    const double t = 2.5 + (double)r * (23.5 * k + 6.5) + (double)small * (8.7 * k + 3.5);
+    if (t < best_t) best = {kTileMixed, rows}, best_t = t;
   }
   return best;
 }
@@ -1085,23 +1136,33 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
   if (vec && K % 64 == 0 && M * N >= (int64_t)kDmaMinMN && lda <= kDmaMaxLd && ldb <= kDmaMaxLd) {
     if ((M + 127) / 128 * ((N + 127) / 128) > 0x7fffffffLL)
       return set_error(TPP_E_UNSUPPORTED, "%s: too many tiles", name);
-    switch (pick_dma_tile(M, N, EPI == kGSwiGLU, device_cus())) {
-    case 0: launch_dma<T, EPI, ACT, 1, 2, 4, 2, kSmallBK, 5>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
-    case 1: launch_dma<T, EPI, ACT, 1, 3, 4, 2, kSmallBK, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
-    case 2: launch_dma<T, EPI, ACT, 1, 4, 4, 2, kSmallBK, 3>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
-    default: {
+    const int cus = device_cus();
+    const bool persist = EPI != kGBiasAct && cus % 8 == 0;
+    const BigPlan pl = pick_dma_tile(M, N, K, EPI == kGSwiGLU, persist, cus);
+    switch (pl.tile) {
+    case kTile128x128: launch_dma<T, EPI, ACT, 1, 2, 4, 2, kSmallBK, 5>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
+    case kTile128x192: launch_dma<T, EPI, ACT, 1, 3, 4, 2, kSmallBK, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
+    case kTile128x256: launch_dma<T, EPI, ACT, 1, 4, 4, 2, kSmallBK, 3>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
+    case kTileMixed: {
+      const int64_t nb = pl.big_rows / 256 * ((N + 255) / 256) +
+                         ((M - pl.big_rows + 127) / 128) * ((N + 127) / 128);
+      gemm_mixed_kernel<T, EPI, ACT><<<dim3((unsigned)nb), dim3(512), 0, st>>>(
+          (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N, (int)K,
+          (int)pl.big_rows);
+      break;
+    }
+    case kTile256x256: {
       // more tiles than CUs: the persistent kernel (plain / SwiGLU epilogue)
       bool done = false;
-      if constexpr (EPI != kGBiasAct && kBigBK == 64 && kBigNST == 2) {
-        const int cus = device_cus();
+      if constexpr (EPI != kGBiasAct) {
         const int64_t nb = ((M + 255) / 256) * ((N + 255) / 256);
-        if (cus % 8 == 0 && nb > cus) {
+        if (persist && nb > cus) {
           gemm_persist_kernel<T, EPI, ACT><<<dim3((unsigned)cus), dim3(512), 0, st>>>(
               (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N, (int)K);
           done = true;
         }
       }
-      if (!done) launch_dma<T, EPI, ACT, 2, 4, 4, 2, kBigBK, kBigNST>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
+      if (!done) launch_dma<T, EPI, ACT, 2, 4, 4, 2, 64, 2>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
       break;
     }
     }
