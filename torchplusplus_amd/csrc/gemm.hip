@@ -378,10 +378,17 @@ __device__ __forceinline__ void gemm_dma_tile(
     }
   };
   frag(smem, 0);
-  for (int kt = 0; kt < nk; ++kt) {
+  // K tile kt, with the DMA of K tile kt + NST - 1 if there is `more`. The
+  // 128-row tiles run two loops, `more` known in each: no DMA instruction under
+  // a branch and constant waits, 5-10% faster ([5367 x 1024] . [3072 x
+  // 1024]^T 47.7 -> 43.1 us, [2048 x 3072] + bias + SiLU, K 1024, 22.4 -> 21.1
+  // us); the 256x256 tile, with 32 MFMAs per sub-step, is 9% slower that way
+  // (113 -> 124 us) and keeps one loop.
+  auto ktile = [&](int kt, auto more) {
+    constexpr bool known = !std::is_same<decltype(more), bool>::value;
     const V8 *sa = smem + (kt % NST) * STG;
     const int kn = kt + NST - 1;
-    const bool more = kn < nk, next = kt + 1 < nk;
+    const bool next = more || kt + 1 < nk;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ks + 1 < KS) frag(sa, ks + 1);
@@ -400,13 +407,21 @@ __device__ __forceinline__ void gemm_dma_tile(
             // fragments of the second half of this sub-step are not consumed
             // yet, so wait for every LDS read (lgkmcnt(0); the barrier does
             // not wait for them)
-            wait_tiles<NQ, NST - 2>(nk - kt - 2);
+            if constexpr (known && std::is_same<decltype(more), std::true_type>::value) wait_vmcnt<(NST - 2) * NQ>();
+            else wait_tiles<NQ, NST - 2>(nk - kt - 2);
             wait_lgkmcnt0();
             __builtin_amdgcn_s_barrier();
             frag(smem + ((kt + 1) % NST) * STG, 0);
           }
         }
     }
+  };
+  if constexpr (FM == 1) {
+    int kt = 0;
+    for (; kt + NST - 1 < nk; ++kt) ktile(kt, std::true_type{});
+    for (; kt < nk; ++kt) ktile(kt, std::false_type{});
+  } else {
+    for (int kt = 0; kt < nk; ++kt) ktile(kt, kt + NST - 1 < nk);
   }
 
   if constexpr (EPI == kGBiasAct) {
