@@ -173,6 +173,13 @@ int tpp_linear_act(const void *x, const void *w, const void *bias, void *y,
                    int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy,
                    int act, int dtype, void *stream);
 
+/* Three bias-free projections of one input, y[i][M, N[i]] = T(x . w[i]^T)
+ * with contiguous weights [N[i], K] and outputs: an attention layer's Wq, Wk
+ * and Wv (torchpp/attention/mha.py:71-73), in one launch where that is faster
+ * than tpp_linear_act for each. */
+int tpp_linear3(const void *x, const void *const *w, void *const *y, int64_t M, const int64_t *N,
+                int64_t K, int64_t ldx, int dtype, void *stream);
+
 /* Plain GEMMs of tpp_linear_act (no bias, no activation) with at least as
  * many 256 x 256 output tiles as the device has CUs run on hipBLASLt (zero
  * workspace, plan cached per shape), as the reference runs its plain projections on

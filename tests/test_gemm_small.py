@@ -129,3 +129,22 @@ def test_swiglu_mixed_tiles(dev):
     y = ext().linear_swiglu(x.to(dev), interleave_gate_up(wg, wu).to(dev))
     g = oracle.linear_act(x, wg, None, "silu").float()
     close(y, (g * oracle.linear_act(x, wu, None, "none").float()).to(x.dtype), what="mixed swiglu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,ns,k", [(17, (64, 64, 64), 72), (36, (1024, 128, 128), 1024), (100, (1024, 1024, 1024), 1024),
+                                    (300, (1000, 33, 1), 520), (600, (512, 512, 100), 256), (1045, (1024, 1024, 1024), 192),
+                                    (2000, (1024, 1024, 1024), 128), (2000, (1024, 64, 64), 64),
+                                    (5000, (1024, 1024, 1030), 64), (3000, (1024, 1024, 1024), 1000)])
+def test_three_projections(dev, m, ns, k):
+    """Three outputs of one launch, at every tile it has: ragged rows and
+    columns, a K tail, outputs narrower than a tile; bit-equal repeats."""
+    from torchplusplus_amd._native import ext
+    dtype = torch.float16 if m % 2 else torch.bfloat16
+    x, _, _ = _mk(m, 1, k, dtype, seed=m)
+    ws = [_mk(1, n, k, dtype, seed=n + i)[1] for i, n in enumerate(ns)]
+    xd, wd = x.to(dev), [w.to(dev) for w in ws]
+    got = ext().linear3(xd, *wd)
+    for y, w, again in zip(got, ws, ext().linear3(xd, *wd)):
+        close(y, oracle.linear_act(x, w, None, "none"), what=f"three {m}x{tuple(w.shape)}")
+        assert torch.equal(y, again)

@@ -425,11 +425,31 @@ at::Tensor linear_any(at::Tensor input, at::Tensor weight, c10::optional<at::Ten
   return linear_act(input, weight, bias, act);
 }
 
-// projections of one input, in one call
+// three bias-free projections of one input: one launch, or the decode GEMV
+// for each up to 16 rows
 std::vector<at::Tensor> linear3(at::Tensor input, at::Tensor w0, at::Tensor w1, at::Tensor w2) {
   const c10::optional<at::Tensor> none;
-  return {linear_any(input, w0, none, TPP_ACT_NONE), linear_any(input, w1, none, TPP_ACT_NONE),
-          linear_any(input, w2, none, TPP_ACT_NONE)};
+  TORCH_CHECK(input.dim() >= 1 && input.size(-1) > 0, "Input must be at least 1D and not empty");
+  if (input.numel() / input.size(-1) <= 16)
+    return {gemv(input, w0, none, TPP_ACT_NONE), gemv(input, w1, none, TPP_ACT_NONE),
+            gemv(input, w2, none, TPP_ACT_NONE)};
+  const at::Tensor w[3] = {w0, w1, w2};
+  std::vector<at::Tensor> out;
+  const void *wp[3];
+  void *yp[3];
+  int64_t N[3];
+  c10::DeviceGuard g(input.device());
+  for (int i = 0; i < 3; ++i) {
+    check_linear(input, w[i]);
+    N[i] = w[i].size(0);
+    out.push_back(torch::empty(out_shape(input, N[i]), input.options()));
+    wp[i] = w[i].data_ptr(), yp[i] = out[i].data_ptr();
+  }
+  const int64_t K = input.size(-1);
+  check_rc(tpp_linear3(input.data_ptr(), wp, yp, input.numel() / K, N, K, K, dtype_code(input),
+                       cur_stream(input)),
+           "linear3");
+  return out;
 }
 
 // What a derived weight is keyed on: each source's storage address, version

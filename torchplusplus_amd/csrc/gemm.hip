@@ -252,12 +252,12 @@ template <typename T, int EPI, int FM, int FN, int NST, int WM, int WN, int BK> 
   return ring > outs ? ring : outs;
 }
 
-// Output tile `pid` of the rows from `mb` on; `smem` holds dma_tile_lds units.
+// The output tile at (m0, n0); `smem` holds dma_tile_lds units.
 template <typename T, int EPI, int ACT, int FM, int FN, int NST, int WM, int WN, int BK>
 __device__ __forceinline__ void gemm_dma_tile(
     typename VecT<T>::v8 *smem, const T *__restrict__ A, int64_t lda, const T *__restrict__ B,
     int64_t ldb, T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K,
-    int pid, int mb) {
+    int m0, int n0) {
   typedef typename VecT<T>::v8 V8;
   constexpr int BM = 32 * WM * FM, BN = 32 * WN * FN, NWV = WM * WN;
   constexpr int CPR = BK / 8;                // 16-byte chunks per tile row
@@ -265,10 +265,6 @@ __device__ __forceinline__ void gemm_dma_tile(
   constexpr int STG = (BM + BN) * CPR;       // 16-byte slots per stage
   constexpr int NA = BM / RPI / NWV, NB = BN / RPI / NWV; // DMA instructions per wave per stage
   static_assert(NA * RPI * NWV == BM && NB * RPI * NWV == BN, "tile rows per wave");
-  const int ntm = (M - mb + BM - 1) / BM, ntn = (N + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(pid, ntm * ntn, ntm, ntn, tm, tn);
-  const int m0 = mb + tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w / WN, wn = w % WN;
 
@@ -519,9 +515,13 @@ template <typename T, int EPI, int ACT, int FM, int FN, int NST, int WM, int WN,
 __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(
     const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
     T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
+  constexpr int BM = 32 * WM * FM, BN = 32 * WN * FN;
   __shared__ typename VecT<T>::v8 smem[dma_tile_lds<T, EPI, FM, FN, NST, WM, WN, BK>()];
+  const int ntm = (M + BM - 1) / BM, ntn = (N + BN - 1) / BN;
+  int tm, tn;
+  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
   gemm_dma_tile<T, EPI, ACT, FM, FN, NST, WM, WN, BK>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K,
-                                                       blockIdx.x, 0);
+                                                       tm * BM, tn * BN);
 }
 
 // Two tile sizes in one launch: 256x256 tiles over the first Mb rows, as many
@@ -537,12 +537,17 @@ __global__ __launch_bounds__(512) void gemm_mixed_kernel(
     T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K, int Mb) {
   constexpr int LB = dma_tile_lds<T, EPI, 2, 4, 2, 4, 2, 64>(), LS = dma_tile_lds<T, EPI, 1, 2, 4, 4, 2, 64>();
   __shared__ typename VecT<T>::v8 smem[LB > LS ? LB : LS];
-  const int nbig = Mb / 256 * ((N + 255) / 256);
-  if ((int)blockIdx.x < nbig)
-    gemm_dma_tile<T, EPI, ACT, 2, 4, 2, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, Mb, N, K, blockIdx.x, 0);
-  else
+  const int ntb = (N + 255) / 256, nbig = Mb / 256 * ntb;
+  int tm, tn;
+  if ((int)blockIdx.x < nbig) {
+    tile_coords(blockIdx.x, nbig, Mb / 256, ntb, tm, tn);
+    gemm_dma_tile<T, EPI, ACT, 2, 4, 2, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K, tm * 256, tn * 256);
+  } else {
+    const int ntm = (M - Mb + 127) / 128, ntn = (N + 127) / 128;
+    tile_coords(blockIdx.x - nbig, ntm * ntn, ntm, ntn, tm, tn);
     gemm_dma_tile<T, EPI, ACT, 1, 2, 4, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K,
-                                                   blockIdx.x - nbig, Mb);
+                                                   Mb + tm * 128, tn * 128);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -832,25 +837,25 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(
 // 18.7 -> 9.2. Splitting K over blocks instead would need a cross-block sum
 // (~2 us); rings of 3 and 4 slots, 8 waves per 32x32 tile and 4 waves of two
 // K halves per 64x64 tile were no faster.
+template <int FM, int FN> constexpr int ksplit_wave_lds() { // 16-byte units per wave
+  const int ring = 2 * (32 * FM + 32 * FN) * 8, part = 32 * FM * (32 * FN + 4) / 4;
+  return ring > part ? ring : part;
+}
+
 template <typename T, int EPI, int ACT, int FM, int FN, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_ksplit_kernel(
-    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
-    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
+__device__ __forceinline__ void gemm_ksplit_tile(
+    typename VecT<T>::v8 *smem, const T *__restrict__ A, int64_t lda, const T *__restrict__ B,
+    int64_t ldb, T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K,
+    int m0, int n0) {
   typedef typename VecT<T>::v8 V8;
   constexpr int NST = 2; // ring slots per wave
   constexpr int BM = 32 * FM, BN = 32 * FN, ROWS = BM + BN;
   constexpr int NQ = ROWS / 8;        // DMA instructions per chunk (8 rows of 128 bytes each)
   constexpr int STG = ROWS * 8;       // 16-byte units per ring slot
   constexpr int LDR = BN + 4;         // fp32 pitch of a partial tile (odd in 16-byte units)
-  constexpr int WREG = NST * STG > BM * LDR / 4 ? NST * STG : BM * LDR / 4; // LDS units per wave
+  constexpr int WREG = ksplit_wave_lds<FM, FN>();
   static_assert(NQ * (NST - 1) < 64, "vmcnt range");
   static_assert(EPI != kGSwiGLU || FN % 2 == 0, "whole [gate | up] pairs per tile");
-  __shared__ V8 smem[NW * WREG];
-
-  const int ntm = (M + BM - 1) / BM, ntn = (N + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   // DMA instruction q: slot rows 8q .. 8q + 7 (A rows, then B rows), lane l
@@ -1005,6 +1010,64 @@ __global__ __launch_bounds__(64 * NW) void gemm_ksplit_kernel(
   }
 }
 
+template <typename T, int EPI, int ACT, int FM, int FN, int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_ksplit_kernel(
+    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
+    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
+  constexpr int BM = 32 * FM, BN = 32 * FN;
+  __shared__ typename VecT<T>::v8 smem[NW * ksplit_wave_lds<FM, FN>()];
+  const int ntm = (M + BM - 1) / BM, ntn = (N + BN - 1) / BN;
+  int tm, tn;
+  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
+  gemm_ksplit_tile<T, EPI, ACT, FM, FN, NW>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K, tm * BM, tn * BN);
+}
+
+// Up to three plain products of one A (an attention layer's query, key and
+// value projections) in one launch: the tile columns of the three outputs
+// follow one another, each tile belonging to one of them. The projections of
+// a layer are the width of one weight each, so apart they fill the chip badly
+// (and cost a launch each). Three weights of [1024 x 1024], bf16, us, three
+// launches -> one: 100 rows 11.4 -> 5.9, 640 18.8 -> 10.5, 2000 28.9 -> 22.3,
+// 4500 51.0 -> 34.1; [1024 | 128 | 128], 2412 rows 20.5 -> 13.2.
+struct Group3 {
+  const void *B[3];
+  void *C[3];
+  int N[3];  // output columns (row pitch of C)
+  int nt[3]; // tile columns
+};
+template <typename T> struct GroupTile {
+  const T *B;
+  T *C;
+  int N, tm, tn;
+};
+template <typename T> __device__ __forceinline__ GroupTile<T> group_tile(const Group3 &g, int ntm) {
+  const int ntn = g.nt[0] + g.nt[1] + g.nt[2];
+  int tm, tn;
+  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
+  const int i = tn < g.nt[0] ? 0 : tn < g.nt[0] + g.nt[1] ? 1 : 2;
+  tn -= (i > 0 ? g.nt[0] : 0) + (i > 1 ? g.nt[1] : 0);
+  return {(const T *)(i == 0 ? g.B[0] : i == 1 ? g.B[1] : g.B[2]), (T *)(i == 0 ? g.C[0] : i == 1 ? g.C[1] : g.C[2]),
+          i == 0 ? g.N[0] : i == 1 ? g.N[1] : g.N[2], tm, tn};
+}
+template <typename T, int FM, int FN, int NST, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_group_kernel(const T *__restrict__ A, int64_t lda,
+                                                                      Group3 g, int M, int K) {
+  constexpr int BM = 32 * WM * FM, BN = 32 * WN * FN;
+  __shared__ typename VecT<T>::v8 smem[dma_tile_lds<T, kGPlain, FM, FN, NST, WM, WN, 64>()];
+  const GroupTile<T> t = group_tile<T>(g, (M + BM - 1) / BM);
+  gemm_dma_tile<T, kGPlain, TPP_ACT_NONE, FM, FN, NST, WM, WN, 64>(smem, A, lda, t.B, K, t.C, t.N, nullptr, M,
+                                                                   t.N, K, t.tm * BM, t.tn * BN);
+}
+template <typename T, int FM, int FN, int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_ksplit_group_kernel(const T *__restrict__ A, int64_t lda,
+                                                                    Group3 g, int M, int K) {
+  constexpr int BM = 32 * FM, BN = 32 * FN;
+  __shared__ typename VecT<T>::v8 smem[NW * ksplit_wave_lds<FM, FN>()];
+  const GroupTile<T> t = group_tile<T>(g, (M + BM - 1) / BM);
+  gemm_ksplit_tile<T, kGPlain, TPP_ACT_NONE, FM, FN, NW>(smem, A, lda, t.B, K, t.C, t.N, nullptr, M, t.N, K,
+                                                         t.tm * BM, t.tn * BN);
+}
+
 // Tiles of an output of kDmaMinMN elements and more: the cheapest plan by the
 // time of its rounds (tiles / CUs), in us from fits of each kernel over M 700 -
 // 16384, N 1024 - 11264, K 768 - 3072 (bf16; 6-10% rms, the rounds themselves
@@ -1017,34 +1080,44 @@ enum BigTile { kTile128x128, kTile128x192, kTile128x256, kTile256x256, kTileMixe
 struct BigPlan {
   BigTile tile;
   int64_t big_rows; // rows of the 256x256 part (mixed)
+  double us;
 };
-static BigPlan pick_dma_tile(int64_t M, int64_t N, int64_t K, bool swiglu, bool persist, int cus) {
+// Output columns of a launch: of one matrix, or of three side by side.
+struct OutCols {
+  int64_t n[3];
+  int count;
+  int64_t tiles(int bn) const {
+    int64_t t = 0;
+    for (int i = 0; i < count; ++i) t += (n[i] + bn - 1) / bn;
+    return t;
+  }
+};
+static BigPlan pick_dma_tile(int64_t M, const OutCols &cols, int64_t K, bool swiglu, bool persist, int cus,
+                             bool mixed = true) {
   struct Cand { BigTile id; int bm, bn; double base, full, part, round; };
   const Cand cands[] = {{kTile128x128, 128, 128, 1.0, 8.7, 8.7, 3.5},
                         {kTile128x192, 128, 192, 0.0, 11.0, 12.0, 6.0},
                         {kTile128x256, 128, 256, 1.0, 15.0, 14.0, 5.5},
                         {kTile256x256, 256, 256, 1.5, 25.0, 21.0, 7.5}};
   const double k = (double)K / 1024.0;
-  BigPlan best{kTile128x128, 0};
+  BigPlan best{kTile128x128, 0, 0.0};
   double best_t = -1.0;
-  auto tiles_of = [](int64_t rows, int64_t cols, int bm, int bn) {
-    return ((rows + bm - 1) / bm) * ((cols + bn - 1) / bn);
-  };
+  auto tiles_of = [&](int64_t rows, int bm, int bn) { return ((rows + bm - 1) / bm) * cols.tiles(bn); };
   for (const Cand &c : cands) {
     if (swiglu && c.id == kTile128x192) continue; // whole [gate | up] 64-column pairs per wave
-    const int64_t tiles = tiles_of(M, N, c.bm, c.bn), full = tiles / cus, part = tiles % cus ? 1 : 0;
+    const int64_t tiles = tiles_of(M, c.bm, c.bn), full = tiles / cus, part = tiles % cus ? 1 : 0;
     const bool loop = c.id == kTile256x256 && persist && tiles > cus; // the persistent kernel
     const double t = (loop ? 3.0 : c.base) + (double)full * (c.full * k + (loop ? 3.5 : c.round)) +
                      (double)part * (c.part * k + (loop ? 3.5 : c.round));
-    if (best_t < 0 || t < best_t) best = {c.id, 0}, best_t = t;
+    if (best_t < 0 || t < best_t) best = {c.id, 0, t}, best_t = t;
   }
-  const int64_t ntn = (N + 255) / 256;
-  for (int64_t r = 1; r * cus <= tiles_of(M, N, 256, 256) && r <= 64; ++r) {
+  const int64_t ntn = cols.tiles(256);
+  for (int64_t r = 1; mixed && r * cus <= tiles_of(M, 256, 256) && r <= 64; ++r) {
     const int64_t rows = r * cus / ntn * 256; // row blocks that fit r rounds
     if (rows < 256 || rows >= M) continue;
-    const int64_t small = (tiles_of(M - rows, N, 128, 128) + cus - 1) / cus;
+    const int64_t small = (tiles_of(M - rows, 128, 128) + cus - 1) / cus;
     const double t = 2.5 + (double)r * (23.5 * k + 6.5) + (double)small * (8.7 * k + 3.5);
-    if (t < best_t) best = {kTileMixed, rows}, best_t = t;
+    if (t < best_t) best = {kTileMixed, rows, t}, best_t = t;
   }
   return best;
 }
@@ -1058,7 +1131,11 @@ static BigPlan pick_dma_tile(int64_t M, int64_t N, int64_t K, bool swiglu, bool 
 // 2000x1024x1024: 16.1, 15.3, 9.7, 9.2, 128x128 11.2 us; 1000x3072x1024 +
 // bias: 28.5, 27.4, 21.1, 15.6, 13.5 us.
 enum SmallTile { kKs32x32, kKs64x32, kKs64x64w4, kKs64x64w2, kDma128x64, kDma128x128 };
-static SmallTile pick_small_tile(int64_t M, int64_t N, bool swiglu, bool dma_ok, int cus) {
+struct SmallPlan {
+  SmallTile tile;
+  double us;
+};
+static SmallPlan pick_small_tile(int64_t M, const OutCols &cols, int64_t K, bool swiglu, bool dma_ok, int cus) {
   struct Cand { SmallTile id; int bm, bn, per_cu; double one, full; };
   const Cand cands[] = {{kKs32x32, 32, 32, 2, 1.25, 2.6},   {kKs64x32, 64, 32, 1, 1.95, 2.6},
                         {kKs64x64w4, 64, 64, 1, 3.6, 4.2},  {kKs64x64w2, 64, 64, 2, 4.5, 6.2},
@@ -1069,12 +1146,12 @@ static SmallTile pick_small_tile(int64_t M, int64_t N, bool swiglu, bool dma_ok,
     // SwiGLU needs whole [gate | up] 64-column pairs per wave
     if (swiglu && (c.bn < 64 || c.id == kDma128x64)) continue;
     if (!dma_ok && (c.id == kDma128x64 || c.id == kDma128x128)) continue;
-    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * cols.tiles(c.bn);
     const int64_t round = (int64_t)cus * c.per_cu;
     const double t = tiles <= cus ? c.one : (double)((tiles + round - 1) / round) * c.full;
     if (best_t < 0 || t < best_t) best = c.id, best_t = t;
   }
-  return best;
+  return {best, 3.0 + best_t * (double)K / 1024.0};
 }
 
 static int device_cus() {
@@ -1153,7 +1230,7 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
       return set_error(TPP_E_UNSUPPORTED, "%s: too many tiles", name);
     const int cus = device_cus();
     const bool persist = EPI != kGBiasAct && cus % 8 == 0;
-    const BigPlan pl = pick_dma_tile(M, N, K, EPI == kGSwiGLU, persist, cus);
+    const BigPlan pl = pick_dma_tile(M, {{N}, 1}, K, EPI == kGSwiGLU, persist, cus);
     switch (pl.tile) {
     case kTile128x128: launch_dma<T, EPI, ACT, 1, 2, 4, 2, kSmallBK, 5>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
     case kTile128x192: launch_dma<T, EPI, ACT, 1, 3, 4, 2, kSmallBK, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
@@ -1183,7 +1260,7 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
     }
   } else if (vec && M * N < (int64_t)kDmaMinMN) {
     const bool dma_ok = K % 64 == 0 && lda <= kDmaMaxLd && ldb <= kDmaMaxLd;
-    switch (pick_small_tile(M, N, EPI == kGSwiGLU, dma_ok, device_cus())) {
+    switch (pick_small_tile(M, {{N}, 1}, K, EPI == kGSwiGLU, dma_ok, device_cus()).tile) {
     case kKs32x32:
       if constexpr (EPI != kGSwiGLU) launch_ksplit<T, EPI, ACT, 1, 1, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
       break;
@@ -1209,6 +1286,80 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
     gemm_scalar_kernel<T, EPI, ACT><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
         (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)NO,
         (int)K);
+  }
+  return check_launch(name);
+}
+
+// y[i][M, N_i] = x . w[i]^T for three weights: one launch where the tile
+// rules above expect it to take no longer than three (a weight whose 256x256
+// tiles fill the chip is faster by itself; near that line the two meet: three
+// weights of [1024 x 1024], us apart and in one, 3320 rows 38.4 and 29.9, 8192
+// rows 70.5 and 72.5), three where the operands are not 16-byte aligned.
+template <typename T>
+static int launch_gemm3(const void *x, int64_t ldx, const void *const *w, void *const *y, int64_t M,
+                        const int64_t *N, int64_t K, hipStream_t st, const char *name) {
+  const int cus = device_cus();
+  const OutCols cols{{N[0], N[1], N[2]}, 3};
+  const int64_t total = N[0] + N[1] + N[2];
+  const bool dma_ok = K % 64 == 0 && ldx <= kDmaMaxLd;
+  const bool big = M * total >= (int64_t)kDmaMinMN;
+  bool one = K % 8 == 0 && ldx % 8 == 0 && aligned16(x) && M > 0 && (dma_ok || !big);
+  for (int i = 0; i < 3; ++i) one = one && aligned16(w[i]) && ((M + 255) / 256) * ((N[i] + 255) / 256) < cus;
+  BigPlan bp{kTile128x128, 0, 0.0};
+  SmallPlan sp{kKs64x64w4, 0.0};
+  if (one) {
+    if (big) bp = pick_dma_tile(M, cols, K, false, false, cus, false);
+    else sp = pick_small_tile(M, cols, K, false, dma_ok, cus);
+    double apart = 0.0;
+    for (int i = 0; i < 3; ++i)
+      apart += M * N[i] >= (int64_t)kDmaMinMN ? pick_dma_tile(M, {{N[i]}, 1}, K, false, false, cus).us
+                                              : pick_small_tile(M, {{N[i]}, 1}, K, false, dma_ok, cus).us;
+    one = (big ? bp.us : sp.us) <= apart;
+  }
+  if (!one) {
+    for (int i = 0; i < 3; ++i)
+      if (int e = launch_gemm<T, kGPlain, TPP_ACT_NONE>(x, ldx, w[i], K, y[i], N[i], nullptr, M, N[i], K, st, name))
+        return e;
+    return TPP_OK;
+  }
+  Group3 g;
+  auto tiles = [&](int bm, int bn) {
+    int64_t n = 0;
+    for (int i = 0; i < 3; ++i) {
+      g.B[i] = w[i], g.C[i] = y[i], g.N[i] = (int)N[i], g.nt[i] = (int)((N[i] + bn - 1) / bn);
+      n += g.nt[i];
+    }
+    return dim3((unsigned)(n * ((M + bm - 1) / bm)));
+  };
+  const T *a = (const T *)x;
+  if (big) {
+    switch (bp.tile) {
+    case kTile128x192:
+      gemm_dma_group_kernel<T, 1, 3, 4, 4, 2><<<tiles(128, 192), dim3(512), 0, st>>>(a, ldx, g, (int)M, (int)K);
+      break;
+    case kTile128x256:
+      gemm_dma_group_kernel<T, 1, 4, 3, 4, 2><<<tiles(128, 256), dim3(512), 0, st>>>(a, ldx, g, (int)M, (int)K);
+      break;
+    case kTile256x256:
+      gemm_dma_group_kernel<T, 2, 4, 2, 4, 2><<<tiles(256, 256), dim3(512), 0, st>>>(a, ldx, g, (int)M, (int)K);
+      break;
+    default:
+      gemm_dma_group_kernel<T, 1, 2, 5, 4, 2><<<tiles(128, 128), dim3(512), 0, st>>>(a, ldx, g, (int)M, (int)K);
+      break;
+    }
+  } else {
+    switch (sp.tile) {
+    case kKs32x32: gemm_ksplit_group_kernel<T, 1, 1, 4><<<tiles(32, 32), dim3(256), 0, st>>>(a, ldx, g, (int)M, (int)K); break;
+    case kKs64x32: gemm_ksplit_group_kernel<T, 2, 1, 4><<<tiles(64, 32), dim3(256), 0, st>>>(a, ldx, g, (int)M, (int)K); break;
+    case kKs64x64w4: gemm_ksplit_group_kernel<T, 2, 2, 4><<<tiles(64, 64), dim3(256), 0, st>>>(a, ldx, g, (int)M, (int)K); break;
+    case kKs64x64w2: gemm_ksplit_group_kernel<T, 2, 2, 2><<<tiles(64, 64), dim3(128), 0, st>>>(a, ldx, g, (int)M, (int)K); break;
+    case kDma128x64:
+      gemm_dma_group_kernel<T, 1, 1, 3, 4, 2><<<tiles(128, 64), dim3(512), 0, st>>>(a, ldx, g, (int)M, (int)K);
+      break;
+    case kDma128x128:
+      gemm_dma_group_kernel<T, 1, 2, 5, 4, 2><<<tiles(128, 128), dim3(512), 0, st>>>(a, ldx, g, (int)M, (int)K);
+      break;
+    }
   }
   return check_launch(name);
 }
@@ -1257,6 +1408,16 @@ extern "C" int tpp_linear_act(const void *x, const void *w, const void *bias, vo
                                                      name);
     }
   });
+}
+
+extern "C" int tpp_linear3(const void *x, const void *const *w, void *const *y, int64_t M,
+                           const int64_t *N, int64_t K, int64_t ldx, int dtype, void *stream) {
+  const char *name = "tpp_linear3";
+  if (!w || !y || !N) return set_error(TPP_E_INVALID, "%s: null pointer", name);
+  for (int i = 0; i < 3; ++i)
+    if (int e = gemm_args(name, x, w[i], y[i], M, N[i], K, ldx)) return e;
+  hipStream_t st = as_stream(stream);
+  return TPP_DISPATCH_HALF(dtype, [&] { return launch_gemm3<T>(x, ldx, w, y, M, N, K, st, name); });
 }
 
 extern "C" int tpp_linear_swiglu(const void *x, const void *w_gu, void *y, int64_t M,
