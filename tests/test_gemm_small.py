@@ -148,3 +148,23 @@ def test_three_projections(dev, m, ns, k):
     for y, w, again in zip(got, ws, ext().linear3(xd, *wd)):
         close(y, oracle.linear_act(x, w, None, "none"), what=f"three {m}x{tuple(w.shape)}")
         assert torch.equal(y, again)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(2049, 2100, 8), (2049, 2100, 136), (4096, 4096, 72), (4090, 4099, 200),
+                                   (4300, 4096, 72), (4300, 4099, 120), (6000, 1500, 1000)])
+def test_k_tail_large(dev, m, n, k):
+    """Large outputs whose K is a multiple of 8 but not of 64: 128x128 tiles,
+    256x256 tiles and both, one and several K tiles, with every epilogue."""
+    from torchplusplus_amd._native import ext
+    from torchplusplus_amd.dlops.linear import interleave_gate_up
+    dtype = torch.float16 if m % 2 else torch.bfloat16
+    x, w, b = _mk(m, n, k, dtype, seed=k)
+    xd, wd, bd = x.to(dev), w.to(dev), b.to(dev)
+    close(ext().linear(xd, wd), oracle.linear_act(x, w, None, "none"), what=f"plain {m}x{n}x{k}")
+    close(ext().linear(xd, wd, bd, ACTS["silu"]), oracle.linear_act(x, w, b, "silu"), what=f"silu {m}x{n}x{k}")
+    i = n // 64 * 32
+    wg, wu = w[:i], w[i:2 * i]
+    y = ext().linear_swiglu(xd, interleave_gate_up(wg, wu).to(dev))
+    g = oracle.linear_act(x, wg, None, "silu").float()
+    close(y, (g * oracle.linear_act(x, wu, None, "none").float()).to(dtype), what=f"swiglu {m}x{i}x{k}")

@@ -14,11 +14,9 @@
 //   SwiGLU     weight rows interleaved in blocks of 32 ([gate 32 | up 32]...):
 //              C[:, 32j+c] = T(T(silu(T(g))) * T(u)), the eager FFN chain.
 //
-// Tiling: 128x128 block tile, BK = 64, 256 threads = 4 waves in a 2x2 grid,
-// each wave a 64x64 tile of 2x2 v_mfma_f32_32x32x16 accumulators (64 fp32
-// VGPRs). Global -> VGPR -> LDS with 128-bit accesses, LDS rows XOR-swizzled
-// in 16-byte chunks (conflict-free ds_read_b128 for the MFMA operand
-// pattern), double-buffered with one barrier per K step. Blocks are mapped
+// Tiles: 32x32 to 256x256 outputs per block of v_mfma_f32_32x32x16
+// accumulators, operands by LDS-DMA in 16-byte chunks, LDS rows XOR-swizzled
+// (conflict-free ds_read_b128 for the MFMA operand pattern). Blocks are mapped
 // XCD-aware: the hardware deals blocks round-robin to the 8 XCDs, so block
 // ids are remapped so that each XCD works on a compact group of tiles that
 // share A rows and B columns in its own L2.
@@ -27,8 +25,6 @@
 namespace tpp {
 
 enum GemmEpi { kGPlain = 0, kGBiasAct = 1, kGSwiGLU = 2 };
-
-constexpr int kBM = 128, kBN = 128, kBK = 64;
 
 // LDS tiles hold 128-byte rows of eight 16-byte chunks; chunk c of row r is
 // stored at position c ^ swz(r). A ds_read_b128 serves 16 lanes (16 rows of
@@ -76,119 +72,8 @@ __device__ __forceinline__ void tile_coords(int pid, int nb, int ntm, int ntn, i
   tn = within / gsz;
 }
 
-template <typename T, int EPI, int ACT>
-__global__ __launch_bounds__(256) void gemm_kernel(
-    const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
-    T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K) {
-  typedef typename VecT<T>::v8 V8;
-  __shared__ V8 sA[2][kBM * kBK / 8];
-  __shared__ V8 sB[2][kBN * kBK / 8];
-
-  const int ntm = (M + kBM - 1) / kBM, ntn = (N + kBN - 1) / kBN;
-  int tm, tn;
-  tile_coords(blockIdx.x, ntm * ntn, ntm, ntn, tm, tn);
-  const int m0 = tm * kBM, n0 = tn * kBN;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 1, wn = w & 1;
-
-  V8 ra[4], rb[4];
-  V8 zero;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) zero[i] = (T)0.0f;
-
-  auto gload = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i, row = c >> 3, kc = c & 7;
-      const int gk = kt * kBK + kc * 8;
-      const int gm = m0 + row, gn = n0 + row;
-      ra[i] = (gm < M && gk < K) ? *reinterpret_cast<const V8 *>(A + (int64_t)gm * lda + gk)
-                                 : zero;
-      rb[i] = (gn < N && gk < K) ? *reinterpret_cast<const V8 *>(B + (int64_t)gn * ldb + gk)
-                                 : zero;
-    }
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i, row = c >> 3, kc = c & 7;
-      sA[buf][row * 8 + (kc ^ swz(row))] = ra[i];
-      sB[buf][row * 8 + (kc ^ swz(row))] = rb[i];
-    }
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const int nk = (K + kBK - 1) / kBK;
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) gload(kt + 1);
-#pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
-      V8 af[2], bfr[2];
-      const int kc = ks * 2 + (lane >> 5);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int row = wm * 64 + i * 32 + (lane & 31);
-        af[i] = sA[buf][row * 8 + (kc ^ swz(row))];
-        const int col = wn * 64 + i * 32 + (lane & 31);
-        bfr[i] = sB[buf][col * 8 + (kc ^ swz(col))];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32<T>(af[i], bfr[j], acc[i][j]);
-    }
-    if (kt + 1 < nk) sstore(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue. 32x32 accumulator layout: lane -> column (lane & 31),
-  // register r -> row (r/4)*8 + (lane/32)*4 + (r%4).
-  const int half = lane >> 5, cl = lane & 31;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = m0 + wm * 64 + i * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
-      if (row >= M) continue;
-      if constexpr (EPI == kGSwiGLU) {
-        const int gcol = n0 + wn * 64 + cl; // gate row of W (tile j = 0)
-        if (gcol + 32 < N) {
-          const float gt = to_f32(from_f32<T>(acc[i][0][r]));
-          const float s = to_f32(from_f32<T>(act_silu(gt)));
-          const float ut = to_f32(from_f32<T>(acc[i][1][r]));
-          const int ocol = (n0 + wn * 64) / 2 + cl;
-          C[(int64_t)row * ldc + ocol] = from_f32<T>(s * ut);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int col = n0 + wn * 64 + j * 32 + cl;
-          if (col >= N) continue;
-          float v = acc[i][j][r];
-          if constexpr (EPI == kGBiasAct) {
-            if (bias) v += to_f32(bias[col]);
-            v = apply_act<ACT>(to_f32(from_f32<T>(v)));
-          }
-          C[(int64_t)row * ldc + col] = from_f32<T>(v);
-        }
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// Pipelined variant for K % 64 == 0: operands go HBM/L2 -> LDS directly with
+// Outputs of a round of 128x128 tiles and more: operands go HBM/L2 -> LDS directly with
 // global_load_lds_dwordx4 (no VGPR staging, no ds_write), through an
 // NST-stage ring (NST-1 K tiles in flight while one is multiplied). Block
 // tile (32*WM*FM) x (32*WN*FN), WM x WN waves, wave tile (32*FM) x (32*FN).
@@ -252,8 +137,10 @@ template <typename T, int EPI, int FM, int FN, int NST, int WM, int WN, int BK> 
   return ring > outs ? ring : outs;
 }
 
-// The output tile at (m0, n0); `smem` holds dma_tile_lds units.
-template <typename T, int EPI, int ACT, int FM, int FN, int NST, int WM, int WN, int BK>
+// The output tile at (m0, n0); `smem` holds dma_tile_lds units. TAIL: K is a
+// multiple of 8 only; the last K tile's chunks past K fetch the row's last
+// chunk and both fragments are zeroed there.
+template <typename T, int EPI, int ACT, int FM, int FN, int NST, int WM, int WN, int BK, bool TAIL = false>
 __device__ __forceinline__ void gemm_dma_tile(
     typename VecT<T>::v8 *smem, const T *__restrict__ A, int64_t lda, const T *__restrict__ B,
     int64_t ldb, T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K,
@@ -289,10 +176,12 @@ __device__ __forceinline__ void gemm_dma_tile(
   for (int q = 0; q < NB; ++q)
     off[NA + q] = (uint32_t)((int64_t)(min(n0 + w * RPI + lrow + RPI * NWV * q, N - 1) - n0) * ldb + lkc * 8) *
                   (uint32_t)sizeof(T);
+  const int nk = (K + BK - 1) / BK;
   // DMA instruction q (0 .. NQ - 1) of K tile kt into a stage
   auto issue_one = [&](int stage, int kt, int q) {
     V8 *sa = smem + stage * STG, *sb = sa + BM * CPR;
-    const int64_t kb = (int64_t)kt * BK * sizeof(T);
+    int64_t kb = (int64_t)kt * BK * (int64_t)sizeof(T);
+    if (TAIL && kt == nk - 1) kb += min(0, K - 8 - (kt * BK + lkc * 8)) * (int)sizeof(T);
     if (q < NA)
       __builtin_amdgcn_global_load_lds((const void *)(ta + kb + off[q]),
                                        (__attribute__((address_space(3))) void *)(sa + (q * NWV + w) * 64),
@@ -349,7 +238,6 @@ __device__ __forceinline__ void gemm_dma_tile(
   constexpr int MID = NMF - (FM * FN) / 2; // MFMAs of a K tile issued before its barrier
   constexpr int SP = (NMF / 2) / NQ > 0 ? (NMF / 2) / NQ : 1; // MFMAs per DMA instruction
   static_assert(NQ * SP <= MID, "all DMA of a K tile issued before its barrier");
-  const int nk = K / BK;
 #pragma unroll
   for (int p = 0; p < NST - 1; ++p)
     if (p < nk)
@@ -388,6 +276,16 @@ __device__ __forceinline__ void gemm_dma_tile(
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ks + 1 < KS) frag(sa, ks + 1);
+      if (TAIL && kt == nk - 1) {
+        const bool past = kt * BK + ks * 16 + (lane >> 5) * 8 >= K;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+#pragma unroll
+          for (int i = 0; i < FM; ++i) af[ks & 1][i][e] = past ? (T)0.0f : af[ks & 1][i][e];
+#pragma unroll
+          for (int j = 0; j < FN; ++j) bfr[ks & 1][j][e] = past ? (T)0.0f : bfr[ks & 1][j][e];
+        }
+      }
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -530,8 +428,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(
 // for 1.17 rounds of work, and smaller tiles everywhere lose their operand
 // reuse: 6227 x 3072 x 1024 + bias + GeLU (bf16) 66.4 us with 256x256 tiles,
 // 74.0 with 128x128, 52.4 mixed; 3000 x 6144 x 1024 SwiGLU 54.0 -> 43.8 us;
-// 6227 x 5632 x 2048 + bias + GeLU 177 -> 146 us.
-template <typename T, int EPI, int ACT>
+// 6227 x 5632 x 2048 + bias + GeLU 177 -> 146 us. The TAIL form takes any K % 8
+// == 0, with all rows (or none) in 256x256 tiles where those (or 128x128) are
+// the better plan. It took the place of a register-staged 128x128 kernel:
+// 6227 x 3072 x 1000 + bias + GeLU 101 -> 55 us, 16384 x 3072 x 1000 + bias +
+// SiLU 220 -> 120, 2649 x 3072 x 1000 40 -> 32, 1600 x 5632 x 2008 80 -> 53.
+template <typename T, int EPI, int ACT, bool TAIL>
 __global__ __launch_bounds__(512) void gemm_mixed_kernel(
     const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb,
     T *__restrict__ C, int64_t ldc, const T *__restrict__ bias, int M, int N, int K, int Mb) {
@@ -541,11 +443,11 @@ __global__ __launch_bounds__(512) void gemm_mixed_kernel(
   int tm, tn;
   if ((int)blockIdx.x < nbig) {
     tile_coords(blockIdx.x, nbig, Mb / 256, ntb, tm, tn);
-    gemm_dma_tile<T, EPI, ACT, 2, 4, 2, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K, tm * 256, tn * 256);
+    gemm_dma_tile<T, EPI, ACT, 2, 4, 2, 4, 2, 64, TAIL>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K, tm * 256, tn * 256);
   } else {
     const int ntm = (M - Mb + 127) / 128, ntn = (N + 127) / 128;
     tile_coords(blockIdx.x - nbig, ntm * ntn, ntm, ntn, tm, tn);
-    gemm_dma_tile<T, EPI, ACT, 1, 2, 4, 4, 2, 64>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K,
+    gemm_dma_tile<T, EPI, ACT, 1, 2, 4, 4, 2, 64, TAIL>(smem, A, lda, B, ldb, C, ldc, bias, M, N, K,
                                                    Mb + tm * 128, tn * 128);
   }
 }
@@ -875,12 +777,12 @@ __device__ __forceinline__ void gemm_ksplit_tile(
   // units past K (the last chunk of a K that is no multiple of 64) read the
   // row's last one; the fragments zero them
   auto issue = [&](int c, int slot) {
-    const int ke = min(c * 64 + k_even, K - 8) * (int)sizeof(T);
-    const int ko = min(c * 64 + k_odd, K - 8) * (int)sizeof(T);
+    const uint32_t ke = (uint32_t)min(c * 64 + k_even, K - 8) * (uint32_t)sizeof(T);
+    const uint32_t ko = (uint32_t)min(c * 64 + k_odd, K - 8) * (uint32_t)sizeof(T);
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
       __builtin_amdgcn_global_load_lds(
-          (const void *)(src[q] + (uint32_t)((q & 1) ? ko : ke)),
+          (const void *)(src[q] + ((q & 1) ? ko : ke)),
           (__attribute__((address_space(3))) void *)(ring + slot * STG + q * 64), 16, 0, 0);
   };
 
@@ -1093,7 +995,7 @@ struct OutCols {
   }
 };
 static BigPlan pick_dma_tile(int64_t M, const OutCols &cols, int64_t K, bool swiglu, bool persist, int cus,
-                             bool mixed = true) {
+                             bool mixed = true, bool tail = false) {
   struct Cand { BigTile id; int bm, bn; double base, full, part, round; };
   const Cand cands[] = {{kTile128x128, 128, 128, 1.0, 8.7, 8.7, 3.5},
                         {kTile128x192, 128, 192, 0.0, 11.0, 12.0, 6.0},
@@ -1105,6 +1007,7 @@ static BigPlan pick_dma_tile(int64_t M, const OutCols &cols, int64_t K, bool swi
   auto tiles_of = [&](int64_t rows, int bm, int bn) { return ((rows + bm - 1) / bm) * cols.tiles(bn); };
   for (const Cand &c : cands) {
     if (swiglu && c.id == kTile128x192) continue; // whole [gate | up] 64-column pairs per wave
+    if (tail && (c.id == kTile128x192 || c.id == kTile128x256)) continue; // tiles of the mixed kernel
     const int64_t tiles = tiles_of(M, c.bm, c.bn), full = tiles / cus, part = tiles % cus ? 1 : 0;
     const bool loop = c.id == kTile256x256 && persist && tiles > cus; // the persistent kernel
     const double t = (loop ? 3.0 : c.base) + (double)full * (c.full * k + (loop ? 3.5 : c.round)) +
@@ -1225,24 +1128,31 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
         lt_gemm(A, lda, B, ldb, C, ldc, M, N, K, __is_same(T, bf16), st))
       return check_launch(name);
   }
-  if (vec && K % 64 == 0 && M * N >= (int64_t)kDmaMinMN && lda <= kDmaMaxLd && ldb <= kDmaMaxLd) {
+  const bool dma_ld = lda <= kDmaMaxLd && ldb <= kDmaMaxLd;
+  if (vec && M * N >= (int64_t)kDmaMinMN && dma_ld) {
     if ((M + 127) / 128 * ((N + 127) / 128) > 0x7fffffffLL)
       return set_error(TPP_E_UNSUPPORTED, "%s: too many tiles", name);
     const int cus = device_cus();
     const bool persist = EPI != kGBiasAct && cus % 8 == 0;
-    const BigPlan pl = pick_dma_tile(M, {{N}, 1}, K, EPI == kGSwiGLU, persist, cus);
+    const bool tail = K % 64 != 0;
+    const BigPlan pl = pick_dma_tile(M, {{N}, 1}, K, EPI == kGSwiGLU, persist && !tail, cus, true, tail);
+    auto mixed = [&](int64_t big_rows, auto tl) {
+      const int64_t small_rows = M > big_rows ? M - big_rows : 0;
+      const int64_t nb = big_rows / 256 * ((N + 255) / 256) + (small_rows + 127) / 128 * ((N + 127) / 128);
+      gemm_mixed_kernel<T, EPI, ACT, decltype(tl)::value><<<dim3((unsigned)nb), dim3(512), 0, st>>>(
+          (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N, (int)K,
+          (int)big_rows);
+    };
+    if (tail) {
+      mixed(pl.tile == kTileMixed ? pl.big_rows : pl.tile == kTile256x256 ? (M + 255) / 256 * 256 : 0,
+            std::true_type{});
+      return check_launch(name);
+    }
     switch (pl.tile) {
     case kTile128x128: launch_dma<T, EPI, ACT, 1, 2, 4, 2, kSmallBK, 5>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
     case kTile128x192: launch_dma<T, EPI, ACT, 1, 3, 4, 2, kSmallBK, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
     case kTile128x256: launch_dma<T, EPI, ACT, 1, 4, 4, 2, kSmallBK, 3>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
-    case kTileMixed: {
-      const int64_t nb = pl.big_rows / 256 * ((N + 255) / 256) +
-                         ((M - pl.big_rows + 127) / 128) * ((N + 127) / 128);
-      gemm_mixed_kernel<T, EPI, ACT><<<dim3((unsigned)nb), dim3(512), 0, st>>>(
-          (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N, (int)K,
-          (int)pl.big_rows);
-      break;
-    }
+    case kTileMixed: mixed(pl.big_rows, std::false_type{}); break;
     case kTile256x256: {
       // more tiles than CUs: the persistent kernel (plain / SwiGLU epilogue)
       bool done = false;
@@ -1259,7 +1169,7 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
     }
     }
   } else if (vec && M * N < (int64_t)kDmaMinMN) {
-    const bool dma_ok = K % 64 == 0 && lda <= kDmaMaxLd && ldb <= kDmaMaxLd;
+    const bool dma_ok = K % 64 == 0 && dma_ld;
     switch (pick_small_tile(M, {{N}, 1}, K, EPI == kGSwiGLU, dma_ok, device_cus()).tile) {
     case kKs32x32:
       if constexpr (EPI != kGSwiGLU) launch_ksplit<T, EPI, ACT, 1, 1, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
@@ -1275,11 +1185,10 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
     case kDma128x128: launch_dma<T, EPI, ACT, 1, 2, 4, 2, kSmallBK, 5>(A, lda, B, ldb, C, ldc, bias, M, N, K, st); break;
     }
   } else if (vec) {
-    const int64_t nb = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
-    if (nb > 0x7fffffffLL) return set_error(TPP_E_UNSUPPORTED, "%s: too many tiles", name);
-    gemm_kernel<T, EPI, ACT><<<dim3((unsigned)nb), dim3(256), 0, st>>>(
-        (const T *)A, lda, (const T *)B, ldb, (T *)C, ldc, (const T *)bias, (int)M, (int)N,
-        (int)K);
+    // row pitches past the DMA tiles' 32-bit offsets: the tile with 64-bit row addresses
+    if ((M + 63) / 64 * ((N + 63) / 64) > 0x7fffffffLL)
+      return set_error(TPP_E_UNSUPPORTED, "%s: too many tiles", name);
+    launch_ksplit<T, EPI, ACT, 2, 2, 4>(A, lda, B, ldb, C, ldc, bias, M, N, K, st);
   } else {
     const int64_t NO = (EPI == kGSwiGLU) ? N / 2 : N;
     const int64_t blocks = (M * NO + 255) / 256;
