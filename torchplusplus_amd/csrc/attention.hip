@@ -1427,7 +1427,8 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
   // leave at once, except that the folded projection needs every workgroup.
   // The length is one scalar load ahead of the first K/V loads (0.4 us;
   // loading two batches of the capacity's split before the length was known
-  // cost more wherever the sequence is short: 64 KB per batch and block).
+  // cost more wherever the sequence is short: 64 KB per batch and block). A
+  // full cache pays for it: 1 x 3933 keys of 4096, 8 heads, 11.0 -> 11.1 us.
   const int Lraw = seqlens ? seqlens[b] : fixed_len;
   const int L = Lraw < p.Sk ? (Lraw > 0 ? Lraw : 0) : p.Sk; // never read past the cache
   const SplitRun run = split_run(L, p.left, STRIDE, nsplit, nsplit_inv);
