@@ -320,6 +320,16 @@ int tpp_attn_prefill_ws(const void *q, const void *k, const void *v, void *o,
                         int causal, int window_left, int window_right, int dtype,
                         void *workspace, size_t ws_bytes, void *stream);
 
+/* How tpp_attn_prefill_ws deals the keys of a call to its workgroups (host
+ * only, for checks and tuning). dims[4]: queries per query tile, keys per key
+ * tile, query tiles, chunks per query tile; zeros where the keys are not
+ * split. ranges (NULL: none), where `capacity` ints hold it, gets per query
+ * tile the number of chunks that the merge reads, then the first key tile of
+ * every chunk and the one past its last (empty: nothing computed). */
+int tpp_attn_prefill_chunks(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
+                            int causal, int window_left, int window_right, int32_t *dims,
+                            int32_t *ranges, int64_t capacity);
+
 /* Bytes of workspace tpp_attn_decode needs. The workspace must be 128-byte
  * aligned and its first 64 KiB zero-filled before the first use: they hold
  * per-(batch, KV head) arrival counters that every call leaves at zero

@@ -126,6 +126,18 @@ __host__ __device__ inline KeyBand key_band(int q0, int q_last, int Sq, int Sk, 
   return {tb, hi > lo ? (hi + kt - 1) / kt : tb};
 }
 
+// Key-split prefill: the tiles of a query tile's band that chunk `split`
+// takes, and the chunks of the band that have a tile. The kernel and the merge
+// both go by these two.
+__host__ __device__ inline KeyBand key_chunk(const KeyBand &kb, int split, int ct) {
+  const int t0 = kb.t_begin + split * ct;
+  return {t0, kb.t_end < t0 + ct ? kb.t_end : t0 + ct};
+}
+__host__ __device__ inline int key_chunks(const KeyBand &kb, int ct, int nsmax) {
+  const int n = (kb.t_end - kb.t_begin + ct - 1) / ct;
+  return n < nsmax ? n : nsmax; // the workspace has nsmax slots per row
+}
+
 // K / V ring slots of the prefill kernel: tile t in slot (t - t_begin) % 3
 constexpr int kPrefillSlots = 3;
 template <typename T, int D> struct PrefillSmem {
@@ -669,7 +681,8 @@ __global__ __launch_bounds__(512) void attn_prefill_split_kernel(AttnArgs p, int
   const int qw = q0 + (hpb == 2 ? 0 : wu * 32);
   const int off = p.Sk - p.Sq;
   const KeyBand kb = key_band(q0, q_last, p.Sq, p.Sk, p.left, p.right, KT);
-  const int t0 = kb.t_begin + split * ct, t1 = min(kb.t_end, t0 + ct);
+  const KeyBand chunk = key_chunk(kb, split, ct);
+  const int t0 = chunk.t_begin, t1 = chunk.t_end;
   if (t0 >= t1 && (split > 0 || nsmax > 1)) return; // (no key at all and one chunk: rows of zeros)
   const int niter = t0 < t1 ? (t1 - t0 + NG - 1) / NG : 0;
 
@@ -918,7 +931,7 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnArgs p, int
   const int qi = (int)(row % p.Sq), hq = (int)(row / p.Sq % p.Hq), b = (int)(row / p.Sq / p.Hq);
   const int q0 = qi / QL * QL, q_last = (q0 + QL < p.Sq ? q0 + QL : p.Sq) - 1;
   const KeyBand kb = key_band(q0, q_last, p.Sq, p.Sk, p.left, p.right, kSplitTile<D>);
-  const int ns = (kb.t_end - kb.t_begin + ct - 1) / ct; // chunks written for this query tile
+  const int ns = key_chunks(kb, ct, nsmax); // chunks written for this query tile
   float mu = -INFINITY, ls = 0.f, os[4] = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < ns; s0 += MG) {
     float2 ml[MG];
@@ -2372,6 +2385,35 @@ extern "C" size_t tpp_attn_prefill_workspace_size(int64_t B, int64_t Sq, int64_t
     return 0;
   const int right = causal ? 0 : (window_right < 0 ? -1 : window_right);
   return plan_prefill(B, Sq, Sk, Hq, Hkv, D, window_left < 0 ? -1 : window_left, right, true).ws_bytes;
+}
+
+extern "C" int tpp_attn_prefill_chunks(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
+                                       int causal, int window_left, int window_right, int32_t *dims,
+                                       int32_t *ranges, int64_t capacity) {
+  const char *name = "tpp_attn_prefill_chunks";
+  if (!dims) return set_error(TPP_E_INVALID, "%s: null pointer argument", name);
+  if (B < 1 || Sq < 1 || Sk < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || B > 0x7fffffff || Sq > 0x7fffffff ||
+      Sk > 0x7fffffff)
+    return set_error(TPP_E_INVALID, "%s: invalid shapes", name);
+  const int right = causal ? 0 : (window_right < 0 ? -1 : window_right), left = window_left < 0 ? -1 : window_left;
+  dims[0] = dims[1] = dims[2] = dims[3] = 0;
+  if (D != 64 && D != 128) return TPP_OK;
+  const PrefillPlan pl = plan_prefill(B, Sq, Sk, Hq, Hkv, D, left, right, true);
+  if (!pl.split) return TPP_OK;
+  const int ql = 64 / pl.hpb, kt = D == 128 ? kSplitTile<128> : kSplitTile<64>;
+  const int64_t nqt = (Sq + ql - 1) / ql, each = 1 + 2 * (int64_t)pl.nsmax;
+  dims[0] = ql, dims[1] = kt, dims[2] = (int32_t)nqt, dims[3] = pl.nsmax;
+  if (!ranges || capacity < nqt * each) return TPP_OK;
+  for (int64_t t = 0; t < nqt; ++t, ranges += each) {
+    const int64_t q0 = t * ql, last = (q0 + ql < Sq ? q0 + ql : Sq) - 1;
+    const KeyBand kb = key_band((int)q0, (int)last, (int)Sq, (int)Sk, left, right, kt);
+    ranges[0] = key_chunks(kb, pl.ct, pl.nsmax);
+    for (int c = 0; c < pl.nsmax; ++c) {
+      const KeyBand r = key_chunk(kb, c, pl.ct);
+      ranges[1 + 2 * c] = r.t_begin, ranges[2 + 2 * c] = r.t_end;
+    }
+  }
+  return TPP_OK;
 }
 
 extern "C" int tpp_attn_prefill_ws(const void *q, const void *k, const void *v, void *o,
