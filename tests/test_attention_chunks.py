@@ -48,6 +48,45 @@ NAMED = [(1, 300, 300, 16, 8, 64, True, (200, 0)), (1, 700, 700, 16, 8, 64, True
          (1, 521, 821, 4, 4, 128, True, (700, 0)), (1, 260, 260, 16, 8, 128, False, (199, 50))]
 
 
+def _visible_tiles(sq, sk, ql, kt, window):
+    """First and end tile of the keys that each query tile sees (empty: both
+    equal), one query row at a time: key j is visible from query i iff
+    -left <= j - (i + sk - sq) <= right."""
+    left, right = window
+    pos = np.arange(sq) + sk - sq
+    lo = np.maximum(pos - left, 0) if left >= 0 else np.zeros(sq, dtype=np.int64)
+    hi = np.minimum(pos + right + 1, sk) if right >= 0 else np.full(sq, sk)
+    some = hi > lo
+    tile = np.arange(sq) // ql
+    first = np.full(tile[-1] + 1, 1 << 30)
+    end = np.zeros(tile[-1] + 1, dtype=np.int64)
+    np.minimum.at(first, tile[some], lo[some] // kt)
+    np.maximum.at(end, tile[some], (hi[some] + kt - 1) // kt)
+    return np.where(end > 0, first, 0), end
+
+
+def test_every_visible_key_is_in_one_chunk():
+    """The chunks of a query tile follow one another without a gap, from no
+    later than its first visible key to no earlier than its last."""
+    several = 0
+    for call in NAMED + list(_calls()):
+        plan = _chunks(*call)
+        if plan is None:
+            continue
+        (_, sq, sk, _, _, _, causal, window), (ql, kt, merged, first, end) = call, plan
+        want_first, want_end = _visible_tiles(sq, sk, ql, kt, (window[0], 0 if causal else window[1]))
+        seen = want_end > 0
+        several += first.shape[1] > 1
+        ran = np.arange(first.shape[1])[None, :] < merged[:, None]
+        assert (merged[seen] > 0).all(), call
+        last = np.take_along_axis(end, np.maximum(merged - 1, 0)[:, None], 1)[:, 0]
+        assert (first[:, 0] <= want_first)[seen].all() and (last >= want_end)[seen].all(), call
+        assert (first[:, 1:] == end[:, :-1])[ran[:, 1:]].all(), call
+        # no chunk longer than a full one (its time is what the plan counted)
+        assert ((end - first).max(axis=1) <= (end - first)[:, 0])[merged > 1].all(), call
+    assert several > 500
+
+
 def test_merge_reads_only_chunks_that_were_written():
     split = 0
     for call in NAMED + list(_calls()):

@@ -55,6 +55,39 @@ def test_split_prefill(dev, dtype, b, sq, sk, hq, hkv, d, causal, window):
     assert torch.equal(o, again)
 
 
+# windows whose widest query tile is not the first, middle or last one: key
+# tiles of 64 against 32 queries (odd and even tiles differ), a middle tile cut
+# at key 0 beside a short last one, bounds on both sides; one chunk and several
+WINDOWS = [(1, 300, 300, 16, 8, 64, True, (200, 0)), (1, 700, 700, 16, 8, 64, True, (200, 0)),
+           (1, 400, 400, 8, 8, 128, True, (199, 0)), (1, 340, 340, 16, 16, 128, True, (199, 0)),
+           (1, 900, 1100, 8, 4, 128, True, (1000, 0)), (1, 784, 784, 24, 8, 64, False, (601, 77)),
+           (1, 260, 260, 16, 8, 128, False, (199, 50)), (1, 177, 2495, 24, 6, 64, False, (1392, 78)),
+           (1, 521, 821, 4, 4, 128, True, (700, 0))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,sq,sk,hq,hkv,d,causal,window", WINDOWS)
+def test_split_prefill_windows(dev, dtype, b, sq, sk, hq, hkv, d, causal, window):
+    from torchplusplus_amd.attention import flash_attn_func
+    q, k, v = _qkv(b, sq, sk, hq, hkv, d, dtype, seed=sq)
+    o = flash_attn_func(q.to(dev), k.to(dev), v.to(dev), causal=causal, window_size=window)
+    close(o, oracle.attention(q, k, v, causal=causal, window=window), what=f"window {window} of {sq} x {sk}")
+
+
+@pytest.mark.parametrize("embed,heads,seq", [(1024, 8, 400), (1024, 16, 340), (512, 8, 700)])
+def test_sliding_window_layer_of_200(dev, embed, heads, seq):
+    """A window that is no power of two, through the layer (oracle/modules.py)."""
+    from oracle import modules as om
+    from tests.test_modules import _randomize, _tables, _x
+    from torchplusplus_amd.attention import SlidingWindowAttention
+    mod = SlidingWindowAttention(200, embed, heads, dtype=torch.bfloat16, device=dev)
+    p, x = _randomize(mod, 3), _x((1, seq, embed), torch.bfloat16, 4)
+    c, s, cd, sd = _tables(embed // heads, seq, dev)
+    with torch.no_grad():
+        got = mod(x.to(dev), cd, sd)
+    close(got, om.mha(x, p, c, s, heads, window_size=200), what=f"SWA 200 over {seq}")
+
+
 def test_split_prefill_captured(dev):
     """Several chunks inside a graph: every replay equals the eager result."""
     from torchplusplus_amd.attention import flash_attn_func

@@ -127,11 +127,12 @@ __host__ __device__ inline KeyBand key_band(int q0, int q_last, int Sq, int Sk, 
 }
 
 // Key-split prefill: the tiles of a query tile's band that chunk `split`
-// takes, and the chunks of the band that have a tile. The kernel and the merge
-// both go by these two.
-__host__ __device__ inline KeyBand key_chunk(const KeyBand &kb, int split, int ct) {
+// takes (the last one to the band's end, whatever the plan expected), and the
+// chunks of the band that have a tile. The kernel and the merge both go by
+// these two.
+__host__ __device__ inline KeyBand key_chunk(const KeyBand &kb, int split, int ct, int nsmax) {
   const int t0 = kb.t_begin + split * ct;
-  return {t0, kb.t_end < t0 + ct ? kb.t_end : t0 + ct};
+  return {t0, split == nsmax - 1 || kb.t_end < t0 + ct ? kb.t_end : t0 + ct};
 }
 __host__ __device__ inline int key_chunks(const KeyBand &kb, int ct, int nsmax) {
   const int n = (kb.t_end - kb.t_begin + ct - 1) / ct;
@@ -681,7 +682,7 @@ __global__ __launch_bounds__(512) void attn_prefill_split_kernel(AttnArgs p, int
   const int qw = q0 + (hpb == 2 ? 0 : wu * 32);
   const int off = p.Sk - p.Sq;
   const KeyBand kb = key_band(q0, q_last, p.Sq, p.Sk, p.left, p.right, KT);
-  const KeyBand chunk = key_chunk(kb, split, ct);
+  const KeyBand chunk = key_chunk(kb, split, ct, nsmax);
   const int t0 = chunk.t_begin, t1 = chunk.t_end;
   if (t0 >= t1 && (split > 0 || nsmax > 1)) return; // (no key at all and one chunk: rows of zeros)
   const int niter = t0 < t1 ? (t1 - t0 + NG - 1) / NG : 0;
@@ -2147,18 +2148,30 @@ static PrefillPlan plan_prefill(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, i
   pl.hpb = G % 2 == 0 ? 2 : 1;
   const int64_t ql = 64 / pl.hpb, nqt = (Sq + ql - 1) / ql, npair = B * (Hq / pl.hpb);
   if (npair * nqt > 8 * (int64_t)cus || Sk > (1 << 30)) return pl;
-  // tiles of `kt` keys per query tile of `len` queries: largest and average
-  // (first, middle and last tile)
+  // tiles of `kt` keys per query tile of `len` queries: an upper bound (the
+  // chunks are cut by it) and the average of the first, middle and last tile
   auto tiles = [&](int64_t len, int kt, double &most, double &mean) {
     const int64_t n = (Sq + len - 1) / len;
     auto at = [&](int64_t t) {
       const int64_t q0 = t * len, last = (q0 + len < Sq ? q0 + len : Sq) - 1;
-      const KeyBand kb = key_band((int)q0, (int)last, (int)Sq, (int)Sk, left, right, kt);
-      return (double)(kb.t_end - kb.t_begin);
+      return key_band((int)q0, (int)last, (int)Sq, (int)Sk, left, right, kt);
     };
-    const double f = at(0), m = at(n / 2), l = at(n - 1);
-    most = f > m ? (f > l ? f : l) : (m > l ? m : l);
-    mean = (f + 2 * m + l) / 4;
+    const KeyBand f = at(0), m = at(n / 2), l = at(n - 1);
+    mean = (double)((f.t_end - f.t_begin) + 2 * (m.t_end - m.t_begin) + (l.t_end - l.t_begin)) / 4;
+    // bands move right with the query; bounded on both sides, a whole one also
+    // has at most the tiles that its keys touch from where one can begin in a
+    // tile (kt and len are powers of two: kt / len places, or one)
+    int64_t top = l.t_end - f.t_begin;
+    if (left >= 0 && right >= 0) {
+      const int64_t keys = (len < Sq ? len : Sq) + left + right;
+      int64_t touched = 0;
+      for (int64_t q0 = 0; q0 < (kt > len ? kt : len); q0 += len) {
+        const int64_t begin = (q0 + Sk - Sq - left) & (kt - 1), t = (begin + keys - 1) / kt + 1;
+        touched = t > touched ? t : touched;
+      }
+      top = touched < top ? touched : top;
+    }
+    most = (double)top;
   };
   double most, mean;
   const int hpb8 = (G % 4 == 0) ? 4 : (G % 2 == 0) ? 2 : 1;
@@ -2409,7 +2422,7 @@ extern "C" int tpp_attn_prefill_chunks(int64_t B, int64_t Sq, int64_t Sk, int64_
     const KeyBand kb = key_band((int)q0, (int)last, (int)Sq, (int)Sk, left, right, kt);
     ranges[0] = key_chunks(kb, pl.ct, pl.nsmax);
     for (int c = 0; c < pl.nsmax; ++c) {
-      const KeyBand r = key_chunk(kb, c, pl.ct);
+      const KeyBand r = key_chunk(kb, c, pl.ct, pl.nsmax);
       ranges[1 + 2 * c] = r.t_begin, ranges[2 + 2 * c] = r.t_end;
     }
   }
