@@ -196,3 +196,57 @@ def test_decode_group_keeps_infinities(dev):
     assert torch.equal(torch.isinf(o), torch.isinf(want)) and not torch.isnan(o).any()
     fin = torch.isfinite(want)
     close(o[fin], want[fin], what="finite columns")
+
+
+def _decode_64(q, k, v, n):
+    """64-bit decode attention of one sequence, one KV head: q [1, 1, H, D]."""
+    s = q[0, 0].double() @ k[0, 0, :n].double().t() / q.shape[-1] ** 0.5
+    return torch.softmax(s, dim=-1) @ v[0, 0, :n].double()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("bits,value", [(20, 3.0), (26, 500.0), (40, 30000.0)])
+def test_decode_group_keeps_small_probabilities(dev, dtype, d, bits, value):
+    """One key of weight 1 whose V is zero, and 3000 of about 2^-bits: their
+    sum is all there is. The result is rounded to T once; fp32 sums of 3000
+    equal terms add less than that (2^-24 * 3000 / 2 < 2^-13). V stays below the
+    largest half (65504), the results above the smallest normal one (2^-14)."""
+    from torchplusplus_amd.attention import decode_attention
+    q, k, v = (torch.zeros(1, s, h, d).to(dtype) for s, h in ((1, 4), (1, 3001), (1, 3001)))
+    q[..., 0] = 16
+    k[0, 0, 777, 0] = bits * 0.6931 * d ** 0.5 / 16
+    v[0, 0] = value * (1 + torch.arange(d) / d).to(dtype)
+    v[0, 0, 777] = 0
+    o = decode_attention(q.to(dev), k.to(dev), v.to(dev), torch.tensor([3001], dtype=torch.int32, device=dev))
+    want = _decode_64(q, k, v, 3001)
+    rel = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + 2.0 ** -13
+    err = (o[0, 0].double().cpu() - want).abs() / want
+    assert err.max() <= rel, f"weights 2^-{bits}: relative error {err.max():.2e}"
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_decode_group_keeps_24_bits_of_a_probability(dev, d):
+    """A weight w in (0.5, 1) against its two leading bfloat16 parts, taken off
+    by two keys of weight 1: what is left, w - hi - mid, is near 2^-18 and has
+    the error of fp32 alone (2^-24 each for the weight and three sums: 2^-22,
+    a sixteenth of it)."""
+    from torchplusplus_amd.attention import decode_attention
+    steps = torch.arange(1, 200, dtype=torch.float64) / 512
+    kb = (-steps).bfloat16()
+    w = torch.exp(16 * kb.double() / d ** 0.5)
+    hi = w.bfloat16()
+    mid = (w - hi.double()).bfloat16()
+    left = (w - hi.double() - mid.double()).abs()
+    best = int(torch.where(w > 0.5, left, torch.zeros_like(left)).argmax())
+    assert left[best] > 2.0 ** -19
+    q, k, v = (torch.zeros(1, s, h, d).bfloat16() for s, h in ((1, 4), (1, 300), (1, 300)))
+    q[..., 0] = 16
+    k[0, 0, :, 0] = -8
+    k[0, 0, 17:20, 0] = torch.stack([torch.zeros_like(kb[best]), torch.zeros_like(kb[best]), kb[best]])
+    for row, value in ((17, -hi[best]), (18, -mid[best]), (19, torch.ones(()))):
+        v[0, 0, row] = value
+    o = decode_attention(q.to(dev), k.to(dev), v.to(dev), torch.tensor([300], dtype=torch.int32, device=dev))
+    want = _decode_64(q, k, v, 300)
+    err = ((o[0, 0].double().cpu() - want) / want).abs().max()
+    assert err <= 2.0 ** -22 / left[best] + 2.0 ** -8, f"relative error {err:.2e}"

@@ -1750,13 +1750,17 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
 // of O^T = V^T P^T. A block is 4 waves; each wave streams its own tiles of the
 // split's run (K and V by LDS-DMA into a private slot, no barrier in the
 // loop): the next K tile is requested as soon as this one's fragments are
-// read, the next V tile after this one's. The probabilities stay fp32-exact to
-// 2^-17: P = hi + lo in T, two products. Waves, then splits, are merged as in
-// the kernel above. Measured (bf16): 16 sequences of 2000 keys, 32 / 8 heads,
-// D 128, 41.1 -> 26.6 us; 64 sequences of 64-4000 keys, 8 / 1 heads, 57.6 ->
-// 22.2 us; 8 of 300-3000, 32 / 8 heads, D 64, 22.1 -> 12.1 us; two heads: 1
-// sequence of 900 keys, 16 / 8 heads, D 128, 9.1 -> 8.3 us, 32 of 100-4096
-// 55.3 -> 51.8 us, 8 of 2058 16.9 -> 17.0 us.
+// read, the next V tile after this one's. The probabilities keep their fp32
+// bits: P is the sum of three parts in T, each what the ones ahead leave (8
+// bits each in bf16, 11 in fp16), and the parts are columns 0-7, 8-15 and
+// 16-23 of one product, summed in fp32 at the end. Two parts in two products
+// lost a P below 2^-25 in fp16 and the last bits in bf16, in the same time
+// (bf16 within 0.3 us either way, fp16 0.1-0.5 us faster). Waves, then splits,
+// are merged as in the kernel above. Measured (bf16, the VALU kernel first): 16
+// sequences of 2000 keys, 32 / 8 heads, D 128, 41.1 -> 26.1 us; 64 sequences of
+// 64-4000 keys, 8 / 1 heads, 57.6 -> 22.3 us; 8 of 300-3000, 32 / 8 heads, D
+// 64, 22.1 -> 12.0 us; two heads: 1 sequence of 900 keys, 16 / 8 heads, D 128,
+// 9.1 -> 7.9 us, 32 of 100-4096 55.3 -> 52.1 us, 8 of 2058 16.9 -> 16.7 us.
 // ---------------------------------------------------------------------------
 template <typename T, int D>
 __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const int *__restrict__ seqlens,
@@ -1771,7 +1775,13 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
   constexpr int LDO = D + 4; // fp32 pitch of a wave's partial rows
   __shared__ V8 smem[NW * 2 * TU];
   __shared__ float s_m[NW][kDecMaxG], s_l[NW][kDecMaxG];
-  static_assert(kDecMaxG * LDO * 4 <= 2 * TU * 16, "a wave's partial rows fit its tile slot");
+  constexpr int NP = 3; // parts of a probability
+  static_assert(NP * kDecMaxG * LDO * 4 <= 2 * TU * 16 && kDecMaxG == 8 && NP * kDecMaxG <= 32,
+                "a wave's partial rows fit its tile slot, its parts the columns");
+  // fp16 parts are scaled by 2^15 (P is 1 at most) and by 2^11 more each: what
+  // falls below the least half of the last one is under 2^-61 of P's largest
+  constexpr bool H = !__is_same(T, bf16);
+  constexpr float kScale0 = H ? 32768.f : 1.f, kScale1 = H ? 2048.f : 1.f;
 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, ql = lane & 31, G = p.Hq / p.Hkv;
@@ -1815,8 +1825,36 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
     issue(true, first);
     issue(false, first);
   }
-  // query heads of the group as columns (columns past G repeat the last head)
-  const T *qp = (const T *)p.q + (int64_t)b * p.q_sb + (int64_t)(hk * G + min(ql, G - 1)) * p.q_sh;
+  // Query heads of the group as columns ql % 8 (past G the last head again),
+  // once for each part of the probabilities (columns past the parts repeat the
+  // last part): every lane of a head computes the same scores.
+  const int head = ql % kDecMaxG, prt = ql / kDecMaxG;
+  // this lane's part of eight probabilities x[8 half ..]: what the parts ahead
+  // of it leave, cut (not rounded) to T, two values at a time
+  const float off1 = prt > 0 ? -1.f : 0.f, off2 = prt > 1 ? -1.f : 0.f;
+  const float sc1 = prt > 0 ? kScale1 : 1.f, sc2 = prt > 1 ? kScale1 : 1.f;
+  const unsigned m1 = prt > 0 ? 0xffff0000u : 0u, m2 = prt > 1 ? 0xffff0000u : 0u;
+  auto part_of = [&](const f32x16 &x, int half) {
+    u32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float a = x[half * 8 + 2 * j], b = x[half * 8 + 2 * j + 1];
+      if constexpr (H) {
+        a *= kScale0, b *= kScale0;
+        const auto h0 = __builtin_amdgcn_cvt_pkrtz(a, b);
+        a = fmaf(off1, (float)h0[0], a) * sc1, b = fmaf(off1, (float)h0[1], b) * sc1;
+        const auto h1 = __builtin_amdgcn_cvt_pkrtz(a, b);
+        a = fmaf(off2, (float)h1[0], a) * sc2, b = fmaf(off2, (float)h1[1], b) * sc2;
+        r[j] = __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(a, b));
+      } else { // a bfloat16 is the upper half of a float
+        a -= __uint_as_float(__float_as_uint(a) & m1), b -= __uint_as_float(__float_as_uint(b) & m1);
+        a -= __uint_as_float(__float_as_uint(a) & m2), b -= __uint_as_float(__float_as_uint(b) & m2);
+        r[j] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+      }
+    }
+    return __builtin_bit_cast(V8, r);
+  };
+  const T *qp = (const T *)p.q + (int64_t)b * p.q_sb + (int64_t)(hk * G + min(head, G - 1)) * p.q_sh;
   V8 qf[D / 16];
 #pragma unroll
   for (int i = 0; i < D / 16; ++i) qf[i] = *reinterpret_cast<const V8 *>(qp + i * 16 + h * 8);
@@ -1919,15 +1957,10 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[tt][r] *= alpha;
     }
-    V8 ph[2 * NB], pl[2 * NB];
+    // this lane's part of each probability: what the parts ahead leave
+    V8 pb[2 * NB];
 #pragma unroll
-    for (int c = 0; c < 2 * NB; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float e = s[c >> 1][(c & 1) * 8 + j];
-        ph[c][j] = from_f32<T>(e);
-        pl[c][j] = from_f32<T>(e - to_f32(ph[c][j]));
-      }
+    for (int c = 0; c < 2 * NB; ++c) pb[c] = part_of(s[c >> 1], c & 1);
     // this tile's V landed (the next K may be in flight)
     if (more) vm_wait<NDMA>();
     else vm_wait<0>();
@@ -1955,9 +1988,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
 #pragma unroll
       for (int tt = 0; tt < NT; ++tt) {
         const s16x8 r12 = __builtin_shufflevector(vr[c % 2][2 * tt], vr[c % 2][2 * tt + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-        const V8 va = __builtin_bit_cast(V8, r12);
-        o[tt] = mfma32x32<T>(va, ph[c], o[tt]);
-        o[tt] = mfma32x32<T>(va, pl[c], o[tt]);
+        o[tt] = mfma32x32<T>(__builtin_bit_cast(V8, r12), pb[c], o[tt]);
       }
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -1966,7 +1997,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
   // this wave's rows (its tile slot is drained), then the block's
   const float l = l_run + __shfl_xor(l_run, 32, kWave);
   float *const part = reinterpret_cast<float *>(ring);
-  if (ql < G) {
+  if (head < G && prt < NP) {
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
@@ -1976,10 +2007,10 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
         for (int e = 0; e < 4; ++e) v[e] = o[tt][rg * 4 + e];
         *reinterpret_cast<f32x4 *>(part + ql * LDO + tt * 32 + rg * 8 + h * 4) = v;
       }
-    if (h == 0) s_m[w][ql] = m_run == -INFINITY ? m_run : m_run * c2, s_l[w][ql] = l;
+    if (h == 0 && prt == 0) s_m[w][head] = m_run == -INFINITY ? m_run : m_run * c2, s_l[w][head] = l;
   }
-  // An infinity in V: its products with the two halves of P (which may be zero
-  // or of opposite sign) sum to NaN where P times V is infinite. A wave with a
+  // An infinity in V: its products with the parts of P (which may be zero or
+  // of opposite sign) sum to NaN where P times V is infinite. A wave with a
   // non-finite sum therefore redoes its sums with one product per key.
   bool odd = false;
 #pragma unroll
@@ -2004,7 +2035,11 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
           for (int c = 0; c < D / 64; ++c) acc[c] += e * to_f32(vr[c * 64 + lane]);
         }
 #pragma unroll
-      for (int c = 0; c < D / 64; ++c) part[gi * LDO + c * 64 + lane] = acc[c];
+      for (int c = 0; c < D / 64; ++c) {
+        part[gi * LDO + c * 64 + lane] = acc[c] * kScale0;
+#pragma unroll
+        for (int x = 1; x < NP; ++x) part[(x * kDecMaxG + gi) * LDO + c * 64 + lane] = 0.f;
+      }
     }
   }
   __syncthreads();
@@ -2020,7 +2055,11 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnArgs p, const
     for (int ww = 0; ww < NW; ++ww) {
       const float c = exp2f(s_m[ww][gi] - mu);
       ls += s_l[ww][gi] * c;
-      os += reinterpret_cast<const float *>(smem + ww * (2 * TU))[gi * LDO + d] * c;
+      const float *pr = reinterpret_cast<const float *>(smem + ww * (2 * TU)) + gi * LDO + d;
+      float sum = 0.f; // the least part first
+#pragma unroll
+      for (int x = NP - 1; x >= 0; --x) sum = sum * (1.f / kScale1) + pr[x * kDecMaxG * LDO];
+      os += sum * (1.f / kScale0) * c;
     }
     const int hq = hk * G + gi;
     if (live == 1) {
