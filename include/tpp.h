@@ -180,6 +180,15 @@ int tpp_linear_act(const void *x, const void *w, const void *bias, void *y,
 int tpp_linear3(const void *x, const void *const *w, void *const *y, int64_t M, const int64_t *N,
                 int64_t K, int64_t ldx, int dtype, void *stream);
 
+/* The output tile that tpp_linear_act (outputs 1; `fused`: with a bias or an
+ * activation), tpp_linear_swiglu (`swiglu`, N[0] = 2 I) or tpp_linear3 (outputs
+ * 3) take for aligned operands (host only, for checks and tuning). tile[4]:
+ * rows, columns, waves that share the K dimension (0: not split), and the rows
+ * that 256 x 256 tiles cover ahead of these (two sizes in one launch). All zero:
+ * hipBLASLt, or three launches. */
+int tpp_linear_tiles(int64_t M, const int64_t *N, int outputs, int64_t K, int fused, int swiglu,
+                     int32_t *tile);
+
 /* Plain GEMMs of tpp_linear_act (no bias, no activation) with at least as
  * many 256 x 256 output tiles as the device has CUs run on hipBLASLt (zero
  * workspace, plan cached per shape), as the reference runs its plain projections on

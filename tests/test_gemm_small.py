@@ -30,7 +30,8 @@ def _mk(m, n, k, dtype, seed=0, wstd=0.05):
 SHAPES = [(17, 1, 8), (17, 33, 64), (31, 64, 72), (32, 96, 200), (33, 100, 248), (77, 1024, 3072),
           (65, 1003, 1000), (230, 1024, 2048), (300, 2048, 1000), (510, 1024, 1024),
           (230, 4096, 1024), (600, 1028, 520), (2000, 1024, 1024), (1990, 1030, 320),
-          (1000, 3072, 1024), (1000, 4100, 64), (1024, 4095, 128), (513, 4000, 192)]
+          (1000, 3072, 1024), (1000, 4100, 64), (1024, 4095, 128), (513, 4000, 192),
+          (6700, 570, 128), (2451, 1590, 64)]
 
 
 @pytest.mark.gpu
@@ -131,11 +132,16 @@ def test_swiglu_mixed_tiles(dev):
     close(y, (g * oracle.linear_act(x, wu, None, "none").float()).to(x.dtype), what="mixed swiglu")
 
 
+THREE = [(17, (64, 64, 64), 72), (36, (1024, 128, 128), 1024), (100, (1024, 1024, 1024), 1024),
+         (300, (1000, 33, 1), 520), (600, (512, 512, 100), 256), (1045, (1024, 1024, 1024), 192),
+         (2000, (1024, 1024, 1024), 128), (2000, (1024, 64, 64), 64),
+         (5000, (1024, 1024, 1030), 64), (3000, (1024, 1024, 1024), 1000), (321, (1024, 1024, 1024), 1024),
+         (330, (1024, 1000, 1030), 200), (1366, (1024, 1024, 1024), 64), (2689, (1024, 1024, 1024), 128),
+         (3300, (1024, 64, 64), 64), (3301, (1024, 70, 60), 192)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,ns,k", [(17, (64, 64, 64), 72), (36, (1024, 128, 128), 1024), (100, (1024, 1024, 1024), 1024),
-                                    (300, (1000, 33, 1), 520), (600, (512, 512, 100), 256), (1045, (1024, 1024, 1024), 192),
-                                    (2000, (1024, 1024, 1024), 128), (2000, (1024, 64, 64), 64),
-                                    (5000, (1024, 1024, 1030), 64), (3000, (1024, 1024, 1024), 1000)])
+@pytest.mark.parametrize("m,ns,k", THREE)
 def test_three_projections(dev, m, ns, k):
     """Three outputs of one launch, at every tile it has: ragged rows and
     columns, a K tail, outputs narrower than a tile; bit-equal repeats."""
@@ -168,3 +174,29 @@ def test_k_tail_large(dev, m, n, k):
     y = ext().linear_swiglu(xd, interleave_gate_up(wg, wu).to(dev))
     g = oracle.linear_act(x, wg, None, "silu").float()
     close(y, (g * oracle.linear_act(x, wu, None, "none").float()).to(dtype), what=f"swiglu {m}x{i}x{k}")
+
+
+def _tile(m, ns, k, fused=False, swiglu=False):
+    """(rows, columns, waves that share K, rows of 256x256 tiles ahead)."""
+    from torchplusplus_amd._native import lib
+    out = (ctypes.c_int32 * 4)()
+    rc = lib().tpp_linear_tiles(ctypes.c_int64(m), (ctypes.c_int64 * len(ns))(*ns), len(ns), ctypes.c_int64(k),
+                                int(fused), int(swiglu), out)
+    assert rc == 0
+    return tuple(out)
+
+
+SMALL = {(32, 32, 4, 0), (64, 32, 4, 0), (64, 64, 4, 0), (64, 64, 2, 0), (128, 64, 0, 0), (128, 128, 0, 0)}
+
+
+def test_shapes_reach_every_tile():
+    """The shapes above take every tile of the launches they are for (host
+    arithmetic, 256 CUs): a retuned rule must not empty a case unseen."""
+    for fused in (False, True):
+        assert {_tile(m, [n], k, fused) for m, n, k in SHAPES} == SMALL
+    separate = (0, 0, 0, 0)
+    assert {_tile(m, ns, k) for m, ns, k in THREE} == SMALL | {
+        (128, 192, 0, 0), (128, 256, 0, 0), (256, 256, 0, 0), separate}
+    for m, n, k in ((6227, 3072, 128), (4100, 4000, 64), (5633, 3072, 64), (9990, 3076, 192)):
+        assert _tile(m, [n], k, fused=True)[3] > 0
+    assert _tile(2900, [6144], 512, swiglu=True)[3] > 0

@@ -81,9 +81,9 @@ __device__ __forceinline__ void tile_coords(int pid, int nb, int ntm, int ntn, i
 // consume 4096 bf16 flop/clk, so a BM x BN tile needs (BM+BN)/(BM*BN) <=
 // 1/64 byte per flop; 128x128 sits exactly at that limit, 256x256 at half.
 // Measured on MI355X: 256x256 with 8 waves (4x2 of 64x128, two per SIMD)
-// runs ~37-43% of MFMA peak on the prefill shapes vs ~31% for 128x128; with
-// fewer tiles than CUs the 128-row tiles (two blocks per CU with a 2-stage
-// ring) win.
+// runs ~37-43% of MFMA peak on the prefill shapes vs ~31% for 128x128; where
+// the rounds of 256x256 tiles leave CUs idle the 128-row tiles win (one block
+// per CU, rings of 3 to 5 stages; pick_dma_tile has the cost of each round).
 // An LDS-DMA instruction writes lane i's 16 bytes at base + 16*i; lane i of
 // a row group therefore fetches the 16-byte chunk kc = (i%8) ^ swz(row), which
 // lands the tile in the same XOR-swizzled layout the fragment reads expect.
@@ -1199,33 +1199,45 @@ static int launch_gemm(const void *A, int64_t lda, const void *B, int64_t ldb, v
   return check_launch(name);
 }
 
-// y[i][M, N_i] = x . w[i]^T for three weights: one launch where the tile
-// rules above expect it to take no longer than three (a weight whose 256x256
-// tiles fill the chip is faster by itself; near that line the two meet: three
-// weights of [1024 x 1024], us apart and in one, 3320 rows 38.4 and 29.9, 8192
-// rows 70.5 and 72.5), three where the operands are not 16-byte aligned.
+// Three projections of one input: one launch where the tile rules above
+// expect it to take no longer than three (a weight whose 256x256 tiles fill the
+// chip is faster by itself; near that line the two meet: three weights of [1024
+// x 1024], us apart and in one, 3320 rows 38.4 and 29.9, 8192 rows 70.5 and
+// 72.5).
+struct Plan3 {
+  bool one, big; // one launch; its tile is bp's, or sp's
+  BigPlan bp;
+  SmallPlan sp;
+};
+static Plan3 plan_gemm3(int64_t M, const int64_t *N, int64_t K, bool dma_ok, int cus) {
+  const OutCols cols{{N[0], N[1], N[2]}, 3};
+  Plan3 pl{true, M * (N[0] + N[1] + N[2]) >= (int64_t)kDmaMinMN, {kTile128x128, 0, 0.0}, {kKs64x64w4, 0.0}};
+  if (pl.big && !dma_ok) pl.one = false;
+  for (int i = 0; i < 3; ++i) pl.one = pl.one && ((M + 255) / 256) * ((N[i] + 255) / 256) < cus;
+  if (!pl.one) return pl;
+  if (pl.big) pl.bp = pick_dma_tile(M, cols, K, false, false, cus, false);
+  else pl.sp = pick_small_tile(M, cols, K, false, dma_ok, cus);
+  double apart = 0.0;
+  for (int i = 0; i < 3; ++i)
+    apart += M * N[i] >= (int64_t)kDmaMinMN ? pick_dma_tile(M, {{N[i]}, 1}, K, false, false, cus).us
+                                            : pick_small_tile(M, {{N[i]}, 1}, K, false, dma_ok, cus).us;
+  pl.one = (pl.big ? pl.bp.us : pl.sp.us) <= apart;
+  return pl;
+}
+
+// y[i][M, N_i] = x . w[i]^T for three weights, as planned; three launches
+// where the operands are not 16-byte aligned.
 template <typename T>
 static int launch_gemm3(const void *x, int64_t ldx, const void *const *w, void *const *y, int64_t M,
                         const int64_t *N, int64_t K, hipStream_t st, const char *name) {
-  const int cus = device_cus();
-  const OutCols cols{{N[0], N[1], N[2]}, 3};
-  const int64_t total = N[0] + N[1] + N[2];
-  const bool dma_ok = K % 64 == 0 && ldx <= kDmaMaxLd;
-  const bool big = M * total >= (int64_t)kDmaMinMN;
-  bool one = K % 8 == 0 && ldx % 8 == 0 && aligned16(x) && M > 0 && (dma_ok || !big);
-  for (int i = 0; i < 3; ++i) one = one && aligned16(w[i]) && ((M + 255) / 256) * ((N[i] + 255) / 256) < cus;
-  BigPlan bp{kTile128x128, 0, 0.0};
-  SmallPlan sp{kKs64x64w4, 0.0};
-  if (one) {
-    if (big) bp = pick_dma_tile(M, cols, K, false, false, cus, false);
-    else sp = pick_small_tile(M, cols, K, false, dma_ok, cus);
-    double apart = 0.0;
-    for (int i = 0; i < 3; ++i)
-      apart += M * N[i] >= (int64_t)kDmaMinMN ? pick_dma_tile(M, {{N[i]}, 1}, K, false, false, cus).us
-                                              : pick_small_tile(M, {{N[i]}, 1}, K, false, dma_ok, cus).us;
-    one = (big ? bp.us : sp.us) <= apart;
-  }
-  if (!one) {
+  bool one = K % 8 == 0 && ldx % 8 == 0 && aligned16(x) && M > 0;
+  for (int i = 0; i < 3; ++i) one = one && aligned16(w[i]);
+  Plan3 pl{};
+  if (one) pl = plan_gemm3(M, N, K, K % 64 == 0 && ldx <= kDmaMaxLd, device_cus());
+  const bool big = pl.big;
+  const BigPlan &bp = pl.bp;
+  const SmallPlan &sp = pl.sp;
+  if (!one || !pl.one) {
     for (int i = 0; i < 3; ++i)
       if (int e = launch_gemm<T, kGPlain, TPP_ACT_NONE>(x, ldx, w[i], K, y[i], N[i], nullptr, M, N[i], K, st, name))
         return e;
@@ -1327,6 +1339,39 @@ extern "C" int tpp_linear3(const void *x, const void *const *w, void *const *y, 
     if (int e = gemm_args(name, x, w[i], y[i], M, N[i], K, ldx)) return e;
   hipStream_t st = as_stream(stream);
   return TPP_DISPATCH_HALF(dtype, [&] { return launch_gemm3<T>(x, ldx, w, y, M, N, K, st, name); });
+}
+
+extern "C" int tpp_linear_tiles(int64_t M, const int64_t *N, int outputs, int64_t K, int fused,
+                                int swiglu, int32_t *tile) {
+  const char *name = "tpp_linear_tiles";
+  if (!N || !tile) return set_error(TPP_E_INVALID, "%s: null pointer argument", name);
+  if (M < 1 || K < 8 || K % 8 != 0 || (outputs != 1 && outputs != 3) || (outputs == 3 && (fused || swiglu)))
+    return set_error(TPP_E_INVALID, "%s: invalid shapes", name);
+  for (int i = 0; i < outputs; ++i)
+    if (N[i] < 1) return set_error(TPP_E_INVALID, "%s: invalid shapes", name);
+  const int cus = device_cus();
+  const bool tail = K % 64 != 0;
+  bool big = M * N[0] >= (int64_t)kDmaMinMN;
+  BigPlan bp{};
+  SmallPlan sp{};
+  tile[0] = tile[1] = tile[2] = tile[3] = 0;
+  if (outputs == 3) {
+    const Plan3 pl = plan_gemm3(M, N, K, !tail, cus);
+    if (!pl.one) return TPP_OK;
+    big = pl.big, bp = pl.bp, sp = pl.sp;
+  } else {
+    if (!fused && !swiglu && lt_gemm_wanted(M, N[0], cus)) return TPP_OK;
+    if (big) bp = pick_dma_tile(M, {{N[0]}, 1}, K, swiglu, !fused && cus % 8 == 0 && !tail, cus, true, tail);
+    else sp = pick_small_tile(M, {{N[0]}, 1}, K, swiglu, !tail, cus);
+  }
+  if (big) {
+    const int bn[] = {128, 192, 256, 256, 128};
+    tile[0] = bp.tile == kTile256x256 ? 256 : 128, tile[1] = bn[bp.tile], tile[3] = (int32_t)bp.big_rows;
+  } else {
+    const int bm[] = {32, 64, 64, 64, 128, 128}, bn[] = {32, 32, 64, 64, 64, 128}, nw[] = {4, 4, 4, 2, 0, 0};
+    tile[0] = bm[sp.tile], tile[1] = bn[sp.tile], tile[2] = nw[sp.tile];
+  }
+  return TPP_OK;
 }
 
 extern "C" int tpp_linear_swiglu(const void *x, const void *w_gu, void *y, int64_t M,
