@@ -43,6 +43,37 @@ def test_gqa_attend_equals_separate_calls(dev, dtype, b, s, start, rows):
         C.gqa_attend(qkv, qw, kw, 1e-6, cos, sin, *got_c, cap, hq, hkv, d)  # past the cache
 
 
+@pytest.mark.parametrize("qk_norm", [True, False])
+def test_gqa_sequences_at_their_own_positions(dev, qk_norm):
+    """rope_cache and decode_fused with a position per sequence: each sequence
+    gets the cache rows (bit-exact) and the output that a call of its own at
+    that position gives."""
+    from tests.conftest import close
+    from torchplusplus_amd.attention import GroupedQueryAttention
+    from torchplusplus_amd.llmops.kvcache import KVCache
+    hq, hkv, d, cap, dtype = 4, 2, 64, 256, torch.bfloat16
+    mod = GroupedQueryAttention(256, hq, hkv, d, qk_norm=qk_norm, dtype=dtype, device=dev).eval()
+    cos, sin = (_rand((cap, d), torch.float16, i).to(dev) for i in (4, 5))
+    base = [_rand((2, hkv, cap, d), dtype, i).to(dev) for i in (6, 7)]
+    starts = [5, 131]
+    pos = torch.tensor(starts, dtype=torch.int32, device=dev)
+    for s in (1, 20):
+        qkv = _rand((2, s, (hq + 2 * hkv) * d), dtype, s).to(dev)
+        got = [t.clone() for t in base]
+        with torch.no_grad():
+            if s == 1:
+                out = mod.decode_fused(qkv, cos, sin, *got, pos + 1).reshape(2, 1, hq * d)
+            else:
+                mod.rope_cache(qkv, cos, sin, *got, pos)
+            for b, start in enumerate(starts):
+                cache = KVCache(cap, hkv, d, dtype, dev, 1)
+                cache.update(base[0][b:b + 1], base[1][b:b + 1])
+                alone = mod.attend(qkv[b:b + 1].contiguous(), cos, sin, cache, start)
+                assert torch.equal(got[0][b], cache.k_cache[0]) and torch.equal(got[1][b], cache.v_cache[0])
+                if s == 1:
+                    close(out[b:b + 1], alone, what=f"sequence {b} at {start}")
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 40])
 def test_ffn_and_projections_equal_separate_calls(dev, rows):
     from torchplusplus_amd._native import ext

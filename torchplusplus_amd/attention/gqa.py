@@ -81,36 +81,36 @@ class GroupedQueryAttention(nn.Module):
         """[(Hq+2Hkv)*D, d_in]: Wq, Wk, Wv stacked, current with the parameters."""
         return self._wqkv.get(self.Wq.weight, self.Wk.weight, self.Wv.weight)
 
+    def _norms(self):
+        """Per-head norm weights of Q and K (None: no norm) and their eps."""
+        qn, kn = self.q_norm, self.k_norm
+        eps = qn.eps if qn is not None and qn.eps is not None else 1e-6
+        return None if qn is None else qn.weight, None if kn is None else kn.weight, eps
+
     def rope_cache(self, qkv, cos, sin, k_dst, v_dst, positions):
-        """Step 2 on a projected qkv [B, S, (Hq+2Hkv)*D]: returns q [B, S, Hq, D];
-        K/V rows land in k_dst/v_dst ([B, Hkv, L, D]) at positions[b] + s."""
+        """Step 2 on a projected qkv [B, S, (Hq+2Hkv)*D], each sequence from a
+        position of its own: returns q [B, S, Hq, D]; K/V rows land in
+        k_dst/v_dst ([B, Hkv, L, D]) at positions[b] + s."""
         bs, seq_len = qkv.shape[0], qkv.shape[1]
         q = torch.empty(bs, seq_len, self.num_heads, self.head_dim, dtype=qkv.dtype, device=qkv.device)
-        eps = self.q_norm.eps if self.q_norm is not None and self.q_norm.eps is not None else 1e-6
-        _C.qkv_rope_cache(qkv, q, k_dst, v_dst,
-                          self.q_norm.weight if self.q_norm is not None else None,
-                          self.k_norm.weight if self.k_norm is not None else None,
-                          cos, sin, positions, eps)
+        q_norm, k_norm, eps = self._norms()
+        _C.qkv_rope_cache(qkv, q, k_dst, v_dst, q_norm, k_norm, cos, sin, positions, eps)
         return q
 
     def decode_fused(self, qkv, cos, sin, k_cache, v_cache, seqlens):
-        """One new token per sequence: QK-norm + RoPE at position seqlens-1,
-        K/V appended to the caches, split-KV attention over seqlens keys;
-        returns [B, 1, Hq, D]."""
-        eps = self.q_norm.eps if self.q_norm is not None and self.q_norm.eps is not None else 1e-6
-        return _C.attn_decode_fused(qkv, self.q_norm.weight if self.q_norm is not None else None,
-                                    self.k_norm.weight if self.k_norm is not None else None,
-                                    cos, sin, eps, k_cache, v_cache, seqlens)
+        """One new token per sequence, each sequence of a length of its own:
+        QK-norm + RoPE at position seqlens-1, K/V appended to the caches,
+        split-KV attention over seqlens keys; returns [B, 1, Hq, D]."""
+        q_norm, k_norm, eps = self._norms()
+        return _C.attn_decode_fused(qkv, q_norm, k_norm, cos, sin, eps, k_cache, v_cache, seqlens)
 
     def decode_oproj(self, qkv, cos, sin, k_cache, v_cache, seqlens, residual):
         """decode_fused, then the output projection with the residual add:
         residual [B, 1, d_in] <- residual + out_projection(attention output),
         in place (one launch at the Qwen3-0.6B decode shape); returns the
         attention output [B, 1, Hq, D]."""
-        eps = self.q_norm.eps if self.q_norm is not None and self.q_norm.eps is not None else 1e-6
-        return _C.attn_decode_oproj(qkv, self.q_norm.weight if self.q_norm is not None else None,
-                                    self.k_norm.weight if self.k_norm is not None else None,
-                                    cos, sin, eps, k_cache, v_cache, seqlens,
+        q_norm, k_norm, eps = self._norms()
+        return _C.attn_decode_oproj(qkv, q_norm, k_norm, cos, sin, eps, k_cache, v_cache, seqlens,
                                     self.out_projection.weight, residual)
 
     def attend_oproj(self, qkv, cos, sin, kv_cache: KVCache, cache_pos: Optional[int],
@@ -129,19 +129,16 @@ class GroupedQueryAttention(nn.Module):
                cache_pos: Optional[int] = None) -> torch.Tensor:
         """Steps 2-3: rope/cache the projected qkv and attend; returns the
         attention output [B, S, Hq*D] (before the output projection)."""
-        qn, kn = self.q_norm, self.k_norm
-        eps = qn.eps if qn is not None and qn.eps is not None else 1e-6
+        norms = self._norms()
         shape = (self.num_heads, self.n_kv_heads, self.head_dim)
-        norms = (None if qn is None else qn.weight, None if kn is None else kn.weight)
         if kv_cache is None:
-            return _C.gqa_attend(qkv, *norms, eps, cos, sin, None, None, 0, *shape)
+            return _C.gqa_attend(qkv, *norms, cos, sin, None, None, 0, *shape)
         bs, seq_len = qkv.shape[0], qkv.shape[1]
         start = kv_cache.cache_len if cache_pos is None else int(cache_pos)
         kv_cache.ensure(bs, start + seq_len)
         # (the cache may hold more sequences than this call: the kernels get
         # this batch's rows)
-        o = _C.gqa_attend(qkv, *norms, eps, cos, sin, kv_cache.k_cache, kv_cache.v_cache, start,
-                          *shape)
+        o = _C.gqa_attend(qkv, *norms, cos, sin, kv_cache.k_cache, kv_cache.v_cache, start, *shape)
         kv_cache.cache_len = max(kv_cache.cache_len, start + seq_len)
         return o
 
