@@ -1449,7 +1449,8 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(AttnArgs p, const 
   // The length is one scalar load ahead of the first K/V loads (0.4 us;
   // loading two batches of the capacity's split before the length was known
   // cost more wherever the sequence is short: 64 KB per batch and block). A
-  // full cache pays for it: 1 x 3933 keys of 4096, 8 heads, 11.0 -> 11.1 us.
+  // full cache pays for it: 1 x 4096 keys of 4096, 8 heads, 11.7 -> 12.0 us, 32
+  // x 1000 of 1024, 16 heads, D 64, 23.8 -> 24.5 us.
   const int Lraw = seqlens ? seqlens[b] : fixed_len;
   const int L = Lraw < p.Sk ? (Lraw > 0 ? Lraw : 0) : p.Sk; // never read past the cache
   const SplitRun run = split_run(L, p.left, STRIDE, nsplit, nsplit_inv);
@@ -2174,10 +2175,11 @@ struct PrefillPlan {
 // round of four tiles, and several chunks a merge launch of 2.5 us + 0.55 us
 // per MB of partials. The split kernel is taken where it is expected to be
 // 10% faster at least (the margin covers the estimate's error), e.g. 230
-// causal tokens of 16 heads 12.6 -> 9.0 us, 1000 tokens 32.6 -> 17.0 us, 200
-// tokens against 3001 cached keys 80.4 -> 20.1 us (4 chunks), 33 against 8000
-// 203 -> 17.2 us (16 chunks); left alone: 4 x 512 tokens (20.5 against 21.5
-// us), 4096 tokens in a window of 512 (32 against 50 us).
+// causal tokens of 16 heads 12.3 -> 8.6 us, 1000 tokens 32.4 -> 16.5 us, 200
+// tokens against 3001 cached keys 80.4 -> 21.5 us (3 chunks), 33 against 8000
+// 202 -> 19.7 us (11 chunks), 2 x 1000 tokens of 16 / 16 heads, D 64, in a
+// window of 512 22.0 -> 17.1 us; left alone: 4 x 512 tokens (20.8 against 21.5
+// us), 4096 tokens in a window of 512 (29 against 50 us).
 static PrefillPlan plan_prefill(int64_t B, int64_t Sq, int64_t Sk, int64_t Hq, int64_t Hkv, int64_t D,
                                 int left, int right, bool workspace) {
   PrefillPlan pl{};
